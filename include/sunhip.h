@@ -211,14 +211,11 @@ int sh_synchronize(sh_ctx *ctx);
  * counterpart (its passes are host loops, src/dqmc_ft_core/dqmc_ft_sweep_b0.f90:36-207). */
 int sh_set_graphs(sh_ctx *ctx, int enable);
 
-/* Autotuner of the delay depth / submatrix block and of the DFT kernels' vectors per workgroup,
- * in place of the heuristic tables of src/model_para.f90:382-415: after sh_sweep_start_0b, the
- * update of one slice is timed on the chains' own G at every candidate depth (delay 4, 8, 16, 32,
- * and 64 where the delayed vectors do not fit in registers; submatrix 8 .. 64) and the fastest is
- * kept for every chain; with the FFT kinetic form the DFT kernels are timed at 2 .. 16 vectors
- * per workgroup.  The chains' state is left bit for bit as it was (the next updating pass draws
- * its own uniforms).  tuned[0] = chosen nublock, tuned[1] = vectors per workgroup (0: not FFT).
- * The delay depth changes rounding only, not the algorithm (dqmc_update_delay.f90:39-128). */
+/* Autotuner, after sh_sweep_start_0b: with the FFT kinetic form the DFT kernels are timed at 2 .. 16
+ * vectors per workgroup on scratch matrices and the fastest is kept for every chain.  The on-site
+ * update needs no depth (it flushes once per block of sites), so the batch's nublock, which the
+ * bond field's delay and submatrix forms use, is returned as it is.  tuned[0] = nublock, tuned[1] =
+ * vectors per workgroup (0: not FFT).  The chains' state is left bit for bit as it was. */
 int sh_autotune(sh_ctx *ctx, int *tuned);
 
 #ifdef __cplusplus

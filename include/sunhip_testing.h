@@ -28,11 +28,11 @@ int sh_dbg_get(sh_ctx *ctx, int chain, int sel, int pt, double *dst);
  *  7: right product on G: k_cb_rows program a0, kinetic table a1, V table a2, slice a3
  *  8: green_equaltime: right point (saved a0, pt a1), left point (saved a2, pt a3) -> Gs, slot 4,5
  *  9: green_equaltimebb from point a0 -> Gs
- * 10: delay (or submatrix) update of slice a0 using the pass uniforms of slice index a1
+ * 10: on-site update of slice a0 using the pass uniforms of slice index a1
  * 11: draw the pass uniforms (2 N ltrot) from each chain's generator
  * 12: measurement of G into the observable sums
  * 13: wrap check/replace (compare = a0)
- * 14: a0 != 0 selects the delay update that keeps its vectors in L2 instead of registers */
+ * 14: a0 != 0 selects the fast form of the bond-field update whatever the batch's update is */
 int sh_dbg_op(sh_ctx *ctx, int op, const int *a);
 
 #ifdef __cplusplus

@@ -500,7 +500,7 @@ template __global__ void k_zgemm<0, 1>(const DChain *, int, int, int, int, int, 
 
 // ------------------------------------------------------------------------------------------
 // Workgroup-level rank-k update on MFMA: G(n x n) = (G + A B^T) diag(cs) with A, B n x k
-// column-major (leading dimension n).  Used by the delay flush (cs = 1) and the submatrix flush.
+// column-major (leading dimension n).  Used by the bond field's delay flush (cs = 1) and submatrix flush.
 // Computed as G^T tiles so that every global access is a 16-element column run.
 // ------------------------------------------------------------------------------------------
 __device__ static void wg_rank_k(cplx *G, int n, const cplx *A, const cplx *B, int k, const double *csr,
@@ -539,568 +539,6 @@ __device__ static void wg_rank_k(cplx *G, int n, const cplx *A, const cplx *B, i
                 G[(size_t)row + (size_t)col * n] = v;
             }
         }
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// The same rank-k update G += A B^T for k <= K known at compile time, organised for latency:
-// a wave owns 16-row strips of G; the strip's A fragment (K/4 complex per lane) stays in
-// registers while the wave walks the 16-column tiles.  Every load has a clamped, in-bounds
-// address and no branch around it (rows and columns past n compute values that are never
-// stored; entries past k are zero in the A fragment), so nothing waits on a load before its
-// use: G tiles are loaded two tiles ahead into one of two alternating register sets (the flush
-// alone takes 210 VGPRs so; three sets take 251, four spill), the B fragment one tile ahead (a
-// second B set would spill in the delay kernel).  At k = 32 the
-// update reads and writes G for 8 flops per byte, so it is bound by HBM, not by the MFMAs; G
-// streams through with nontemporal accesses so that the A and B fragments, re-read for every
-// tile, stay in L2.
-// ------------------------------------------------------------------------------------------
-template <int KS>
-__device__ __forceinline__ void rank_k_tile(GAS cplx *G, GAS cplx *B, int n, int k, int row, bool rok, int kq, int l16,
-                                            int tj, const cplx (&y)[KS], cplx (&x)[KS], cplx (&g)[4])
-{
-    const int j0 = tj * 16;
-    double4_t accr, acci;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        accr[r] = g[r].x;
-        acci[r] = g[r].y;
-    }
-    // this register set now takes tile tj + 2 (clamped: past the last tile it reloads the last
-    // columns, which are never used); the B fragment takes tile tj + 1
-    const size_t rowc = (size_t)min(row, n - 1);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int col = min(j0 + 32 + kq + 4 * r, n - 1);
-        g[r] = gld_nt(G + (rowc + (size_t)col * n));
-    }
-    const size_t xcol = (size_t)min(j0 + 16 + l16, n - 1);
-#pragma unroll
-    for (int s = 0; s < KS; s++) {
-        accr = mfma(x[s].x, y[s].x, accr);
-        accr = mfma(-x[s].y, y[s].y, accr);
-        acci = mfma(x[s].x, y[s].y, acci);
-        acci = mfma(x[s].y, y[s].x, acci);
-        const int mc = min(4 * s + kq, k - 1);
-        x[s] = gld(B + (xcol + (size_t)mc * n));
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int col = j0 + kq + 4 * r;
-        if (rok && col < n) gst_nt(G + ((size_t)row + (size_t)col * n), make_double2(accr[r], acci[r]));
-    }
-}
-
-template <int K>
-__device__ static void wg_rank_k_strips(cplx *G_, int n, const cplx *A_, const cplx *B_, int k)
-{
-    constexpr int KS = K / 4;
-    GAS cplx *G = gp(G_), *A = gp(A_), *B = gp(B_);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    const int nt = (n + 15) >> 4;
-    const int l16 = lane & 15, kq = lane >> 4;
-    for (int si = w; si < nt; si += nw) {
-        const int row = si * 16 + l16;
-        const bool rok = row < n;
-        const size_t rowc = (size_t)min(row, n - 1);
-        const size_t xcol = (size_t)min(l16, n - 1);
-        cplx y[KS], x[KS], ga[4], gb[4];
-#pragma unroll
-        for (int s = 0; s < KS; s++) {
-            const int m = 4 * s + kq, mc = min(m, k - 1);
-            const cplx a = gld(A + (rowc + (size_t)mc * n));
-            y[s] = m < k ? a : make_double2(0.0, 0.0);
-            x[s] = gld(B + (xcol + (size_t)mc * n));
-        }
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            ga[r] = gld_nt(G + (rowc + (size_t)min(kq + 4 * r, n - 1) * n));
-            gb[r] = gld_nt(G + (rowc + (size_t)min(16 + kq + 4 * r, n - 1) * n));
-        }
-        for (int tj = 0; tj < nt; tj += 2) {
-            rank_k_tile<KS>(G, B, n, k, row, rok, kq, l16, tj, y, x, ga);
-            if (tj + 1 < nt) rank_k_tile<KS>(G, B, n, k, row, rok, kq, l16, tj + 1, y, x, gb);
-        }
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// Metropolis decision of one site (dqmc_update_delay.f90:45-76), evaluated identically by
-// every thread of the chain's workgroup.
-// ------------------------------------------------------------------------------------------
-struct SiteDraw {
-    int is, isp, fl;
-    cplx db;
-};
-
-// the HS tables a site decision reads, copied to LDS once per launch (the same field names as
-// DChain so that the decision helpers take either)
-struct HsTab {
-    int lcomp, nflr;
-    double gaml[4];
-    cplx delta_bmat[12], phase_ratio[12];
-    cplx qf[12];   // gaml(isp)/gaml(is) phase_ratio(iflip, is): the field-only factor of ratiotot
-};
-
-__device__ static void hs_tab_load(HsTab &t, const DChain &c)
-{
-    if (threadIdx.x == 0) {
-        t.lcomp = c.lcomp;
-        t.nflr = c.nflr;
-        for (int k = 0; k < 4; k++) t.gaml[k] = c.gaml[k];
-        for (int k = 0; k < 12; k++) { t.delta_bmat[k] = c.delta_bmat[k]; t.phase_ratio[k] = c.phase_ratio[k]; }
-        for (int is = 1; is <= c.lcomp; is++)
-            for (int fl = 1; fl < c.lcomp; fl++) {
-                const int k = (fl - 1) + (c.lcomp - 1) * (is - 1), isp = (is + fl - 1) % c.lcomp + 1;
-                t.qf[k] = cscale(c.phase_ratio[k], c.gaml[isp - 1] / c.gaml[is - 1]);
-            }
-    }
-}
-
-// The decision of dqmc_update_delay.f90:55-76 without divisions: ratiotot = ratio1^nflr qf and
-// accept when |Re(ratiotot phase)| > u2 |Re(phase)|, which is |ratio_re| > u2 for the reference's
-// ratio_re = Re(ratiotot phase) / Re(phase).  Only the direction of phase matters here, so the
-// caller may carry it unnormalised.
-__device__ __forceinline__ bool site_accept_fast(const HsTab &t, cplx ratio1, const SiteDraw &d, double u2,
-                                                 cplx phase, cplx *ratiotot)
-{
-    cplx rt = ratio1;
-    for (int f = 1; f < t.nflr; f++) rt = cmul(rt, ratio1);
-    rt = cmul(rt, t.qf[(d.fl - 1) + (t.lcomp - 1) * (d.is - 1)]);
-    *ratiotot = rt;
-    return fabs(cmul(rt, phase).x) > u2 * fabs(phase.x);
-}
-
-template <class Tab>
-__device__ __forceinline__ bool site_accept(const Tab &c, cplx ratio1, const SiteDraw &d, double u2,
-                                            cplx phase, cplx *ratiotot)
-{
-    cplx rt = make_double2(1.0, 0.0);
-    for (int f = 0; f < c.nflr; f++) rt = cmul(rt, ratio1);
-    rt = cscale(rt, c.gaml[d.isp - 1] / c.gaml[d.is - 1]);
-    rt = cmul(rt, c.phase_ratio[(d.fl - 1) + (c.lcomp - 1) * (d.is - 1)]);
-    double ratio_re = cmul(rt, phase).x / phase.x;
-    double ratio_abs = ratio_re < 0.0 ? -ratio_re : ratio_re;
-    *ratiotot = rt;
-    return ratio_abs > u2;
-}
-
-template <class Tab>
-__device__ __forceinline__ SiteDraw site_draw(const Tab &c, int is, double u1)
-{
-    SiteDraw d;
-    d.is = is;
-    d.fl = (int)ceil(u1 * (c.lcomp - 1));
-    d.isp = (is + d.fl - 1) % c.lcomp + 1;
-    d.db = c.delta_bmat[(d.fl - 1) + (c.lcomp - 1) * (is - 1)];
-    return d;
-}
-
-__device__ __forceinline__ cplx phase_after(cplx phase, cplx rt)
-{
-    double wgt = sqrt(cmul(rt, cconj(rt)).x);
-    return cscale(cmul(phase, rt), 1.0 / wgt);
-}
-
-// delay update of one slice (src/dqmc_config_u/dqmc_update_delay.f90:39-128); one workgroup per
-// chain, the delayed vectors avec / bvec in global memory (any N and depth; the register kernel
-// below covers N <= 256).  The slice's HS field and uniforms and the HS tables are staged in LDS
-// (the field goes back at the end), so that the site loop reads global memory only for G's row
-// and column and the delayed vectors of an accepted site, four steps of the products in flight.
-// LDS: diag(G) (n), the accepted site's rows of avec / bvec (2 x 64), uniforms (2n), field (n).
-extern "C" __global__ void __launch_bounds__(256)
-k_update_delay(const DChain *chains, int nt, int slice_in_pass)
-{
-    extern __shared__ cplx sh[];
-    const DChain &c = chains[blockIdx.x];
-    const int n = c.n, K = c.nublock;
-    cplx *diagg = sh;                 // n
-    cplx *rowa = sh + n;              // 64: avec(s, 0:ik)
-    cplx *rowb = rowa + 64;           // 64: bvec(s, 0:ik)
-    double *us = (double *)(rowb + 64);   // 2n
-    int *cfs = (int *)(us + 2 * n);   // n
-    __shared__ HsTab tab;
-    cplx *G = c.G, *avec = c.avec, *bvec = c.bvec;
-    GAS cplx *Gg = gp(c.G), *ag = gp(c.avec), *bg = gp(c.bvec);
-    int32_t *cf = c.conf + (size_t)(nt - 1) * n;
-    const double *u = c.unif + (size_t)2 * n * slice_in_pass;
-    cplx phase = make_double2(c.sc[SC_PHASE], c.sc[SC_PHASE + 1]);
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-        diagg[r] = G[(size_t)r + (size_t)r * n];
-        cfs[r] = cf[r];
-    }
-    for (int q = threadIdx.x; q < 2 * n; q += blockDim.x) us[q] = u[q];
-    hs_tab_load(tab, c);
-    __syncthreads();
-    // every load issued so far has landed (the phase above would otherwise keep the compiler
-    // waiting on all outstanding memory operations inside the site loop)
-    __builtin_amdgcn_s_waitcnt(0);
-    int ik = 0;
-    double accm = 0.0;
-    for (int s = 0; s < n; s++) {
-        const SiteDraw d = site_draw(tab, cfs[s], us[2 * s]);
-        cplx dg = diagg[s];
-        cplx ratio1 = cadd(cmul(make_double2(1.0 - dg.x, -dg.y), d.db), make_double2(1.0, 0.0));
-        cplx rt;
-        const bool acc = __builtin_amdgcn_readfirstlane((int)site_accept(tab, ratio1, d, us[2 * s + 1], phase, &rt)) != 0;
-        if (acc) {
-            accm += 1.0;
-            phase = phase_after(phase, rt);
-            cplx sscl = cdiv(d.db, ratio1);
-            for (int m = threadIdx.x; m < ik; m += blockDim.x) {
-                rowa[m] = gld(ag + ((size_t)s + (size_t)m * n));
-                rowb[m] = gld(bg + ((size_t)s + (size_t)m * n));
-            }
-            __syncthreads();
-            // every thread has read this site's field above: thread 0 records the flip
-            if (threadIdx.x == 0) cfs[s] = d.isp;
-            for (int r = threadIdx.x; r < n; r += blockDim.x) {
-                cplx a = gld(Gg + ((size_t)r + (size_t)s * n));
-                cplx b = gld(Gg + ((size_t)s + (size_t)r * n));
-                // the sums in the order m = 0, 1, ..., four steps' loads issued together
-                int m = 0;
-                for (; m + 4 <= ik; m += 4) {
-                    cplx av[4], bv[4];
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        av[j] = gld(ag + ((size_t)r + (size_t)(m + j) * n));
-                        bv[j] = gld(bg + ((size_t)r + (size_t)(m + j) * n));
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        a = cadd(a, cmul(rowb[m + j], av[j]));
-                        b = cadd(b, cmul(rowa[m + j], bv[j]));
-                    }
-                }
-                for (; m < ik; m++) {
-                    a = cadd(a, cmul(rowb[m], gld(ag + ((size_t)r + (size_t)m * n))));
-                    b = cadd(b, cmul(rowa[m], gld(bg + ((size_t)r + (size_t)m * n))));
-                }
-                a = cmul(a, sscl);
-                if (r == s) b.x -= 1.0;
-                diagg[r] = cadd(diagg[r], cmul(a, b));
-                avec[(size_t)r + (size_t)ik * n] = a;
-                bvec[(size_t)r + (size_t)ik * n] = b;
-            }
-            ik++;
-            __syncthreads();
-        }
-        if (ik == K || s == n - 1) {
-            // G += avec bvec^T on the prefetching MFMA strips at the depth of the accepted count
-            if (ik > 0) {
-                if (ik <= 16) {
-                    wg_rank_k_strips<16>(G, n, avec, bvec, ik);
-                } else if (ik <= 32) {
-                    wg_rank_k_strips<32>(G, n, avec, bvec, ik);
-                } else if (ik <= 48) {
-                    wg_rank_k_strips<48>(G, n, avec, bvec, ik);
-                } else {
-                    wg_rank_k_strips<32>(G, n, avec, bvec, 32);
-                    __syncthreads();
-                    wg_rank_k_strips<32>(G, n, avec + (size_t)32 * n, bvec + (size_t)32 * n, ik - 32);
-                }
-            }
-            __syncthreads();
-            ik = 0;
-            if (s < n - 1)
-                for (int r = threadIdx.x; r < n; r += blockDim.x) diagg[r] = gld(Gg + ((size_t)r + (size_t)r * n));
-            __syncthreads();
-            __builtin_amdgcn_s_waitcnt(0);
-        }
-    }
-    for (int r = threadIdx.x; r < n; r += blockDim.x) cf[r] = cfs[r];
-    if (threadIdx.x == 0) {
-        c.sc[SC_PHASE] = phase.x;
-        c.sc[SC_PHASE + 1] = phase.y;
-        c.sc[SC_ACC] += accm;
-        c.sc[SC_TRIED] += n;
-    }
-}
-
-// the factors of one site's draw that do not depend on G (the submatrix kernel evaluates them
-// for a staged block of sites at once, off the per-site critical path)
-struct SubSite {
-    cplx db, idb, f, pr;   // delta, 1 / delta, 1 / (1 + delta), phase_ratio(fl, is)
-    double gr, u2;         // gaml(isp) / gaml(is), the acceptance uniform
-    int isp;
-};
-
-// lane l's complex value as a wave-uniform (scalar) operand; l must be wave-uniform
-__device__ __forceinline__ cplx readlane_c(cplx v, int l)
-{
-    auto rd = [l](double x) {
-        const long long b = __double_as_longlong(x);
-        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, l);
-        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
-        return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-    };
-    return make_double2(rd(v.x), rd(v.y));
-}
-
-// submatrix update of one slice (src/dqmc_config_u/dqmc_update_submatrix.f90:55-162).
-// Gcuta is kept implicitly as G diag(cs); the flush writes (G + (G(:,p) Gamma^-1) G(p,:)) diag(cs),
-// where cs differs from 1 only at the accepted sites p.
-// G does not change between flushes, so the columns and rows of G at the next dss sites are
-// staged in LDS (as in the delay kernel): G(s, p), G(p, s), G(s, s) and the column and row of G
-// an accepted site records come from LDS.  Per site, v1 = G(s, p) Gamma^-1 and
-// v4 = Gamma^-1 G(p, s) are formed before the decision, each by two waves over halves of p
-// (partial sums in LDS, double-buffered by site parity so that no barrier separates one site's
-// reads from the next site's writes); the decision needs v = v1 . G(p, s) only.
-// The site loop itself reads and writes no global memory (its draws are staged with the block
-// and the accepted sites' fields, columns and rows are taken at the flush).
-// Scratch: avec = G(:,p) columns, W1 = G(p,:)^T, bvec = Gmat1, W2 = Gamma^-1 (ld ik).
-// LDS: Gamma^-1 (K (K+1)), the K column scales, dss columns and dss rows of G.
-extern "C" __global__ void __launch_bounds__(256)
-k_update_submatrix(const DChain *chains, int nt, int slice_in_pass, int dss)
-{
-    extern __shared__ cplx sh[];
-    const DChain &c = chains[blockIdx.x];
-    const int n = c.n, K = c.nublock, KL = K + 1;
-    dss = max(1, min(dss, 8));        // the staged draws hold 8 sites
-    cplx *gi = sh;                    // Gamma^-1, column-major, leading dimension K + 1 (lanes reading
-                                      // one entry of K columns each fall on different banks)
-    cplx *csk = gi + KL * K;          // K: cs of the accepted sites
-    cplx *gcol = csk + K;             // dss x n: G(:, s0 + j)
-    cplx *grow = gcol + (size_t)dss * n;  // dss x n: G(s0 + j, :)
-    __shared__ int pvec[256];
-    __shared__ cplx part[2][256];     // [parity][wave * 64 + i]: v1 halves (waves 0, 1), v4 halves (2, 3)
-    __shared__ cplx vsum[2][2];       // [parity][wave]: v halves
-    __shared__ HsTab tab;
-    __shared__ SubSite sfac[8];       // the draws of the staged sites
-    __shared__ int ispk[64];          // the new HS field of the accepted sites, written at the flush
-    cplx *G = c.G, *gm1 = c.avec, *gmat1 = c.bvec, *gm2t = c.W1;
-    GAS cplx *Gg = gp(c.G);
-    int32_t *cf = c.conf + (size_t)(nt - 1) * n;
-    GAS const int32_t *cfg = gp(cf);
-    GAS const double *ug = gp(c.unif + (size_t)2 * n * slice_in_pass);
-    cplx phase = make_double2(c.sc[SC_PHASE], c.sc[SC_PHASE + 1]);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    hs_tab_load(tab, c);
-    __syncthreads();
-    // every load issued so far has landed: without this the compiler cannot tell, inside the
-    // site loop, that the phase loaded above is no longer in flight, and waits for all
-    // outstanding memory operations (the accepted sites' stores) at each use
-    __builtin_amdgcn_s_waitcnt(0);
-    int ik = 0, s0 = -1;
-    double accm = 0.0;
-    for (int s = 0; s < n; s++) {
-        if (s0 < 0 || s >= s0 + dss) {
-            // stage G(:, s..s+nb) (one contiguous run) and G(s..s+nb, :) (nb-element runs);
-            // valid until the next flush changes G.  A lane may still read the previous block.
-            if (s0 >= 0) __syncthreads();
-            s0 = s;
-            const int nb = min(dss, n - s), tot = nb * n;
-            GAS cplx *Gc = Gg + (size_t)s * n;
-            // the sites' draws come with the block (thread t: site s + t), so that the site loop
-            // itself waits on no global load (a wait there would also wait for stores in flight)
-            int cfv = 1;
-            double u1v = 0.5, u2v = 0.0;
-            if (threadIdx.x < nb) {
-                cfv = cfg[s + threadIdx.x];
-                u1v = ug[2 * (s + threadIdx.x)];
-                u2v = ug[2 * (s + threadIdx.x) + 1];
-            }
-            // 8 column and 8 row elements per thread in flight (clamped addresses)
-            for (int base = threadIdx.x; base < tot; base += 8 * (int)blockDim.x) {
-                cplx a[8], b[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const int e = min(base + u * (int)blockDim.x, tot - 1);
-                    a[u] = gld(Gc + e);
-                    b[u] = gld(Gg + ((size_t)(s + e % nb) + (size_t)(e / nb) * n));
-                }
-                if (base == (int)threadIdx.x && threadIdx.x < nb) {
-                    const SiteDraw dd = site_draw(tab, cfv, u1v);
-                    SubSite q;
-                    q.db = dd.db;
-                    q.idb = cinv(dd.db);
-                    q.f = cdiv(make_double2(1.0, 0.0), cadd(make_double2(1.0, 0.0), dd.db));
-                    q.pr = tab.phase_ratio[(dd.fl - 1) + (tab.lcomp - 1) * (dd.is - 1)];
-                    q.gr = tab.gaml[dd.isp - 1] / tab.gaml[dd.is - 1];
-                    q.u2 = u2v;
-                    q.isp = dd.isp;
-                    sfac[threadIdx.x] = q;
-                }
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const int e = base + u * (int)blockDim.x;
-                    if (e < tot) {
-                        gcol[e] = a[u];
-                        grow[(e % nb) * n + e / nb] = b[u];
-                    }
-                }
-            }
-            __syncthreads();
-        }
-        const cplx *gcs = gcol + (size_t)(s - s0) * n, *grs = grow + (size_t)(s - s0) * n;
-        const int par = s & 1;
-        const SubSite q = sfac[s - s0];
-        {
-            // waves 0, 1: v1(i) = sum_m G(s, p_m) Gamma^-1(m, i); waves 2, 3: v4(i) =
-            // sum_m Gamma^-1(i, m) G(p_m, s); m over [0, h) (even waves) or [h, ik) (odd)
-            // lane j holds G(s, p_j) (v1 waves) or G(p_j, s), broadcast to the wave by readlane;
-            // lanes past ik compute on clamped indices and store nothing
-            const int i = lane, h = (ik + 1) >> 1;
-            const int mb = (w & 1) ? h : 0, me = (w & 1) ? ik : h;
-            const int pj = i < ik ? pvec[i] : s, ic = min(i, K - 1);
-            const cplx bvi = gcs[pj], own = w < 2 ? grs[pj] : bvi;
-            cplx a = make_double2(0.0, 0.0), pv = make_double2(0.0, 0.0);
-            // four LDS reads in flight per step; the sum keeps the order m = mb, mb + 1, ...
-            const int gs = w < 2 ? 1 : KL, go = w < 2 ? ic * KL : ic;   // Gamma^-1 entry (m, ic) or (ic, m)
-            int m = mb;
-            for (; m + 4 <= me; m += 4) {
-                const cplx g0 = gi[go + m * gs], g1 = gi[go + (m + 1) * gs], g2 = gi[go + (m + 2) * gs],
-                           g3 = gi[go + (m + 3) * gs];
-                if (w < 2) {
-                    a = cadd(a, cmul(readlane_c(own, m), g0));
-                    a = cadd(a, cmul(readlane_c(own, m + 1), g1));
-                    a = cadd(a, cmul(readlane_c(own, m + 2), g2));
-                    a = cadd(a, cmul(readlane_c(own, m + 3), g3));
-                } else {
-                    a = cadd(a, cmul(g0, readlane_c(own, m)));
-                    a = cadd(a, cmul(g1, readlane_c(own, m + 1)));
-                    a = cadd(a, cmul(g2, readlane_c(own, m + 2)));
-                    a = cadd(a, cmul(g3, readlane_c(own, m + 3)));
-                }
-            }
-            for (; m < me; m++) {
-                const cplx g = gi[go + m * gs];
-                a = w < 2 ? cadd(a, cmul(readlane_c(own, m), g)) : cadd(a, cmul(g, readlane_c(own, m)));
-            }
-            if (w < 2 && i < ik) pv = cmul(a, bvi);
-            if (i < ik) part[par][w * 64 + i] = a;
-            if (w < 2) {
-                pv.x = wave_sum_dpp(pv.x);
-                pv.y = wave_sum_dpp(pv.y);
-                if (i == 0) vsum[par][w] = pv;
-            }
-        }
-        // G(s, s) is in the staged column; read before the barrier, after which the next
-        // block may be staged
-        const cplx gss = gcs[s];
-        __syncthreads();
-        const cplx v = cadd(vsum[par][0], vsum[par][1]);
-        cplx v2 = make_double2(v.x + gss.x - 1.0, v.y + gss.y);
-        cplx ratio1 = csub(make_double2(1.0, 0.0), cmul(v2, q.db));
-        // the decision of site_accept with its draw-only factors precomputed (the same
-        // operations in the same order); every thread evaluates it, and reading it from lane 0
-        // makes the branch scalar
-        cplx rt = make_double2(1.0, 0.0);
-        for (int q = 0; q < tab.nflr; q++) rt = cmul(rt, ratio1);
-        rt = cmul(cscale(rt, q.gr), q.pr);
-        const double ratio_re = cmul(rt, phase).x / phase.x;
-        const bool acc = __builtin_amdgcn_readfirstlane((int)(fabs(ratio_re) > q.u2)) != 0;
-        if (acc) {
-            accm += 1.0;
-            phase = phase_after(phase, rt);
-            cplx den = make_double2(-v.x + 1.0 - gss.x, -v.y - gss.y);
-            den = cadd(den, q.idb);
-            cplx v3 = cinv(den);
-            // Gamma^-1 += (v4 v3) v1 and its new border: lane i of every wave holds v4(i) v3 and
-            // v1(i); wave w updates the columns m = w, w + 4, ... with v1(m) broadcast by readlane
-            const cplx *pp = part[par];
-            const int i = lane, ic = min(i, K - 1);
-            const cplx v1own = cadd(pp[ic], pp[64 + ic]);
-            const cplx v4v3 = cmul(cadd(pp[128 + ic], pp[192 + ic]), v3);
-#pragma unroll 4
-            for (int m = w; m < ik; m += 4) {
-                const cplx v1m = readlane_c(v1own, m);
-                if (i < ik) gi[i + m * KL] = cadd(gi[i + m * KL], cmul(v4v3, v1m));
-            }
-            if (w == 0 && i < ik) {
-                gi[ik + i * KL] = cmul(v3, v1own);
-                gi[i + ik * KL] = v4v3;
-            }
-            if (threadIdx.x == 0) {
-                gi[ik + ik * KL] = v3;
-                pvec[ik] = s;
-                ispk[ik] = q.isp;
-                // cs(s) is 1 until its site is accepted (reset at every flush)
-                csk[ik] = cmul(make_double2(1.0, 0.0), q.f);
-            }
-            ik++;
-            __syncthreads();
-        }
-        if (ik == K || s == n - 1) {
-            if (ik > 0) {
-                // Gmat1 = G(:,p) Gamma^-1 as an MFMA product (Gamma^-1 staged through W2, which
-                // the update does not use)
-                cplx *gig = c.W2;
-                for (int e = threadIdx.x; e < ik * ik; e += blockDim.x) {
-                    const int i = e % ik, j = e / ik;
-                    gig[i + (size_t)j * ik] = gi[i + j * KL];  // ld ik: ik^2 entries
-                }
-                if (threadIdx.x < ik) cf[pvec[threadIdx.x]] = ispk[threadIdx.x];
-                // the accepted sites' columns G(:, p) and rows G(p, :) (the site loop itself
-                // touches no global memory), 8 + 8 elements per thread in flight
-                {
-                    const int tot = ik * n;
-                    for (int base = threadIdx.x; base < tot; base += 8 * (int)blockDim.x) {
-                        cplx a[8], b[8];
-#pragma unroll
-                        for (int u = 0; u < 8; u++) {
-                            const int e = min(base + u * (int)blockDim.x, tot - 1), i = e / n, r = e - i * n;
-                            a[u] = gld(Gg + ((size_t)r + (size_t)pvec[i] * n));
-                            b[u] = gld(Gg + ((size_t)pvec[i] + (size_t)r * n));
-                        }
-#pragma unroll
-                        for (int u = 0; u < 8; u++) {
-                            const int e = base + u * (int)blockDim.x;
-                            if (e < tot) {
-                                gm1[e] = a[u];      // gm1(r, i) = G(r, p_i), ld n
-                                gm2t[e] = b[u];     // gm2t(r, i) = G(p_i, r), ld n
-                            }
-                        }
-                    }
-                }
-                __syncthreads();
-                for (int tm = 0; tm < n; tm += GT)
-                    zgemm_tile<0, 0>(gm1, n, gig, ik, gmat1, n, n, ik, ik, tm, 0, 1.0, 0.0, 0.0, 0.0);
-                __syncthreads();
-                // G += Gmat1 G(p,:): one pass over G up to 48 sites (fragment depth the next
-                // multiple of 16), two passes of up to 32 beyond (a depth-64 fragment would not
-                // fit in registers)
-                if (ik <= 16) {
-                    wg_rank_k_strips<16>(G, n, gmat1, gm2t, ik);
-                } else if (ik <= 32) {
-                    wg_rank_k_strips<32>(G, n, gmat1, gm2t, ik);
-                } else if (ik <= 48) {
-                    wg_rank_k_strips<48>(G, n, gmat1, gm2t, ik);
-                } else {
-                    wg_rank_k_strips<32>(G, n, gmat1, gm2t, 32);
-                    __syncthreads();
-                    wg_rank_k_strips<32>(G, n, gmat1 + (size_t)32 * n, gm2t + (size_t)32 * n, ik - 32);
-                }
-                __syncthreads();
-                // the columns of the accepted sites times their cs, 8 elements per thread in flight
-                const int tot = ik * n;
-                for (int base = threadIdx.x; base < tot; base += 8 * (int)blockDim.x) {
-                    cplx v[8];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const int e = min(base + u * (int)blockDim.x, tot - 1), i = e / n;
-                        v[u] = gld(Gg + ((size_t)(e - i * n) + (size_t)pvec[i] * n));
-                    }
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const int e = base + u * (int)blockDim.x, i = e / n;
-                        if (e < tot) gst(Gg + ((size_t)(e - i * n) + (size_t)pvec[i] * n), cmul(v[u], csk[i]));
-                    }
-                }
-            }
-            __syncthreads();
-            // the flush's last prefetches are never consumed; retiring them here keeps the
-            // compiler from waiting on them (and on every store in flight) inside the site loop
-            __builtin_amdgcn_s_waitcnt(0);
-            ik = 0;
-            s0 = -1;                  // G changed: stage again
-        }
-    }
-    if (threadIdx.x == 0) {
-        c.sc[SC_PHASE] = phase.x;
-        c.sc[SC_PHASE + 1] = phase.y;
-        c.sc[SC_ACC] += accm;
-        c.sc[SC_TRIED] += n;
     }
 }
 
@@ -2126,199 +1564,3 @@ k_save_point(const DChain *chains, int pt)
     if (e < (size_t)n) c.Ds[e] = c.D[(size_t)n * pt + e];
     if (e == 0) { c.sc[SC_LDQ_SAVE] = c.ldq[pt].x; c.sc[SC_LDQ_SAVE + 1] = c.ldq[pt].y; }
 }
-
-// ------------------------------------------------------------------------------------------
-// Delay update with the delayed vectors held in registers (src/dqmc_config_u/dqmc_update_delay.f90:39-128).
-// Wave w covers rows 32w .. 32w+31: lane l < 32 keeps avec(32w + l, 0:K), lane l + 32 keeps
-// bvec of the same row, so a row's two new entries meet through a lane shuffle.  Each site
-// costs one workgroup barrier: the rows avec(s, :) and bvec(s, :) that site s needs are
-// published by row s's lanes at the end of site s - 1 into one of two LDS buffers (by the
-// parity of s), and diagg(s) is only read at site s, so no lane rewrites a value another lane
-// may still be reading.  avec/bvec reach memory only for the MFMA flush.
-// ------------------------------------------------------------------------------------------
-#define DSB 8   // sites per staged block of G columns and rows
-
-// sum_{m < ik} other[m] reg[m] in chunks of four entries: ik is uniform over the workgroup,
-// so each chunk is a scalar branch and only the filled chunks are read (entries of a partly
-// filled chunk beyond ik are zero in reg).  Two accumulators alternate over m.
-template <int K>
-__device__ __forceinline__ cplx delay_dot(int ik, const cplx (&reg)[K], const cplx *other)
-{
-    double vr = 0.0, vi = 0.0, wr = 0.0, wi = 0.0;
-#pragma unroll
-    for (int c = 0; c < K / 4; c++) {
-        if (4 * c < ik) {
-            const cplx o0 = other[4 * c], o1 = other[4 * c + 1], o2 = other[4 * c + 2], o3 = other[4 * c + 3];
-            vr += o0.x * reg[4 * c].x - o0.y * reg[4 * c].y;
-            vi += o0.x * reg[4 * c].y + o0.y * reg[4 * c].x;
-            wr += o1.x * reg[4 * c + 1].x - o1.y * reg[4 * c + 1].y;
-            wi += o1.x * reg[4 * c + 1].y + o1.y * reg[4 * c + 1].x;
-            vr += o2.x * reg[4 * c + 2].x - o2.y * reg[4 * c + 2].y;
-            vi += o2.x * reg[4 * c + 2].y + o2.y * reg[4 * c + 2].x;
-            wr += o3.x * reg[4 * c + 3].x - o3.y * reg[4 * c + 3].y;
-            wi += o3.x * reg[4 * c + 3].y + o3.y * reg[4 * c + 3].x;
-        }
-    }
-    return make_double2(vr + wr, vi + wi);
-}
-
-// the value of lane l ^ 32 (v_permlane32_swap exchanges the two 32-lane halves)
-__device__ __forceinline__ double partner32(double v)
-{
-    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
-    const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-    const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-    const bool upper = (threadIdx.x & 32) != 0;
-    return __hiloint2double((int)(upper ? b[0] : b[1]), (int)(upper ? a[0] : a[1]));
-}
-
-// reg[ik] = v by a binary tree of uniform branches; the empty volatile asm keeps each leaf a
-// real branch target instead of a select over all K registers
-template <int K, int LO, int HI>
-__device__ __forceinline__ void delay_put(int ik, cplx (&reg)[K], cplx v)
-{
-    if constexpr (HI - LO == 1) {
-        reg[LO] = v;
-        asm volatile("" ::: "memory");
-    } else {
-        constexpr int MID = (LO + HI) / 2;
-        if (ik < MID)
-            delay_put<K, LO, MID>(ik, reg, v);
-        else
-            delay_put<K, MID, HI>(ik, reg, v);
-    }
-}
-
-template <int K>
-__global__ void __launch_bounds__(K >= 8 ? 512 : 1024)
-k_update_delay_reg(const DChain *chains, int nt, int slice_in_pass)
-{
-    extern __shared__ cplx sh[];
-    const DChain &c = chains[blockIdx.x];
-    const int n = c.n, kb = c.nublock;
-    const int lane = threadIdx.x & 63;
-    const bool isA = lane < 32;
-    const int r = 32 * (threadIdx.x >> 6) + (lane & 31);
-    cplx *diagg = sh;                   // n
-    cplx *gcol = diagg + n;             // DSB x n: G(:, s0+j)
-    cplx *grow = gcol + DSB * n;        // DSB x n: G(s0+j, :)
-    cplx *rows = grow + DSB * n;        // 2 buffers x (avec row K, bvec row K)
-    double *us = (double *)(rows + 4 * K);  // 2n uniforms of this slice
-    int *cfs = (int *)(us + 2 * n);     // n: HS field of this slice (read-only here)
-    __shared__ HsTab tab;
-    GAS cplx *G = gp(c.G);
-    int32_t *cf = c.conf + (size_t)(nt - 1) * n;
-    const double *u = c.unif + (size_t)2 * n * slice_in_pass;
-    cplx phase = make_double2(c.sc[SC_PHASE], c.sc[SC_PHASE + 1]);
-    cplx reg[K];
-#pragma unroll
-    for (int m = 0; m < K; m++) reg[m] = make_double2(0.0, 0.0);
-    for (int q = threadIdx.x; q < n; q += blockDim.x) {
-        diagg[q] = gld(G + ((size_t)q + (size_t)q * n));
-        cfs[q] = cf[q];
-    }
-    for (int q = threadIdx.x; q < 2 * n; q += blockDim.x) us[q] = u[q];
-    for (int q = threadIdx.x; q < 4 * K; q += blockDim.x) rows[q] = make_double2(0.0, 0.0);
-    hs_tab_load(tab, c);
-    int ik = 0, s0 = -1;
-    double accm = 0.0;
-    for (int s = 0; s < n; s++) {
-        if (s0 < 0 || s >= s0 + DSB) {
-            // stage G(:, s..s+DSB) and G(s..s+DSB, :); valid until the next flush changes G.
-            // The previous site's lanes may still read the old block.
-            if (s0 >= 0) __syncthreads();
-            s0 = s;
-            const int nb = min(DSB, n - s);
-            // columns s..s+nb are one contiguous run; a row block is read as nb-element runs
-            GAS cplx *Gc = G + (size_t)s * n;
-            stage_in_map<4>(gcol, nb * n, [=](int e) { return gld_nt(Gc + (e)); }, [](int e) { return e; });
-            stage_in_map<4>(grow, nb * n, [=](int e) { return gld_nt(G + ((size_t)(s + e % nb) + (size_t)(e / nb) * n)); },
-                            [=](int e) { return (e % nb) * n + e / nb; });
-        }
-        __syncthreads();
-        const SiteDraw d = site_draw(tab, cfs[s], us[2 * s]);
-        const cplx dg = diagg[s];
-        const cplx ratio1 = cadd(cmul(make_double2(1.0 - dg.x, -dg.y), d.db), make_double2(1.0, 0.0));
-        // delta / ratio1, evaluated next to the decision (independent of it) so that the two
-        // dependency chains overlap
-        const cplx sscl = cdiv(d.db, ratio1);
-        cplx rt;
-        // every thread evaluates the same decision; reading it from lane 0 makes the branch
-        // and the delay count scalar
-        const bool acc = __builtin_amdgcn_readfirstlane((int)site_accept_fast(tab, ratio1, d, us[2 * s + 1], phase, &rt)) != 0;
-        if (acc) {
-            accm += 1.0;
-            phase = cmul(phase, rt);   // normalised at the next flush
-            const cplx *rw = rows + (s & 1) * 2 * K;      // avec(s, :), then bvec(s, :)
-            // A lanes: sum_m bvec(s,m) avec(r,m); B lanes: sum_m avec(s,m) bvec(r,m)
-            const cplx *other = isA ? rw + K : rw;
-            const int iku = __builtin_amdgcn_readfirstlane(ik);
-            const cplx dot = delay_dot<K>(iku, reg, other);
-            cplx v = make_double2(0.0, 0.0);
-            if (r < n) {
-                if (isA) {
-                    const cplx gc = gcol[(s - s0) * n + r];
-                    v = cmul(make_double2(gc.x + dot.x, gc.y + dot.y), sscl);
-                } else {
-                    const cplx gr = grow[(s - s0) * n + r];
-                    v = make_double2(gr.x + dot.x, gr.y + dot.y);
-                    if (r == s) v.x -= 1.0;
-                }
-            }
-            delay_put<K, 0, K>(iku, reg, v);
-            // the row's other entry from the partner lane (A <-> B)
-            const cplx w = make_double2(partner32(v.x), partner32(v.y));
-            if (isA && r > s && r < n) diagg[r] = cadd(diagg[r], cmul(v, w));
-            if (threadIdx.x == 0) cf[s] = d.isp;
-            ik++;
-        }
-        // row s+1 publishes its filled vector entries for the next site (the reader's products
-        // cover the same chunks, and its entries past ik are zero)
-        if (r == s + 1 && r < n) {
-            cplx *pw = rows + ((s + 1) & 1) * 2 * K + (isA ? 0 : K);
-            const int iku = __builtin_amdgcn_readfirstlane(ik);
-#pragma unroll
-            for (int c4 = 0; c4 < K / 4; c4++)
-                if (4 * c4 < iku) {
-                    pw[4 * c4] = reg[4 * c4];
-                    pw[4 * c4 + 1] = reg[4 * c4 + 1];
-                    pw[4 * c4 + 2] = reg[4 * c4 + 2];
-                    pw[4 * c4 + 3] = reg[4 * c4 + 3];
-                }
-        }
-        if (ik == kb || s == n - 1) {
-            __syncthreads();
-            if (ik > 0) {
-                if (r < n) {
-                    GAS cplx *dst = gp(isA ? c.avec : c.bvec);
-#pragma unroll
-                    for (int m = 0; m < K; m++)
-                        if (m < ik) gst(dst + ((size_t)r + (size_t)m * n), reg[m]);
-                }
-                // the vectors restart from zero after the flush; clearing them here frees
-                // their registers for the flush
-#pragma unroll
-                for (int m = 0; m < K; m++) reg[m] = make_double2(0.0, 0.0);
-                __syncthreads();
-                wg_rank_k_strips<K>(c.G, n, c.avec, c.bvec, ik);
-            }
-            __syncthreads();
-            phase = cscale(phase, 1.0 / sqrt(cabs2(phase)));
-            ik = 0;
-            s0 = -1;
-            if (s < n - 1)
-                for (int q = threadIdx.x; q < n; q += blockDim.x) diagg[q] = gld(G + ((size_t)q + (size_t)q * n));
-        }
-    }
-    if (threadIdx.x == 0) {
-        c.sc[SC_PHASE] = phase.x;
-        c.sc[SC_PHASE + 1] = phase.y;
-        c.sc[SC_ACC] += accm;
-        c.sc[SC_TRIED] += n;
-    }
-}
-
-template __global__ void k_update_delay_reg<4>(const DChain *, int, int);
-template __global__ void k_update_delay_reg<8>(const DChain *, int, int);
-template __global__ void k_update_delay_reg<16>(const DChain *, int, int);
-template __global__ void k_update_delay_reg<32>(const DChain *, int, int);

@@ -180,10 +180,9 @@ void update_family(shp_ctx *ctx, int nt, int nf, size_t uoff0)
 }
 
 // the G-based forms (dqmc_proj_update_delay.f90, dqmc_proj_update_submatrix_G.f90): G from the
-// current UR, (UL UR)^-1, UL; the finite-temperature delay or submatrix kernel on it through the
+// current UR, (UL UR)^-1, UL; the finite-temperature site update on it through the
 // chain's view (its uniforms are the pass buffer at 2 N per slice: the on-site field alone);
 // UR's flipped rows; a fresh (UL UR)^-1
-
 void update_u_g(shp_ctx *ctx, int nt, size_t uoff0)
 {
     const int n = ctx->n;
@@ -191,14 +190,7 @@ void update_u_g(shp_ctx *ctx, int nt, size_t uoff0)
     Tic t(ctx, T_UPDATE);
     hipLaunchKernelGGL(kp_u_save, dim3((n + 255) / 256, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nt);
     const int slice = (int)(uoff0 / (2 * (size_t)n));
-    if (ctx->update == SHP_U_DELAY) {
-        const size_t lds = (size_t)(n + 2 * 64) * sizeof(cplx) + (size_t)n * 20;
-        hipLaunchKernelGGL(k_update_delay, dim3(ctx->nch), dim3(256), lds, ctx->st, ctx->dview, nt, slice);
-    } else {
-        const int K = ctx->gblock, dss = sub_stage(n, K);
-        hipLaunchKernelGGL(k_update_submatrix, dim3(ctx->nch), dim3(256), lds_sub(n, K, dss), ctx->st, ctx->dview, nt,
-                           slice, dss);
-    }
+    site_update(ctx->st, ctx->dview, ctx->nch, n, nt, slice);
     hipLaunchKernelGGL(kp_u_rescale, dim3((unsigned)(((size_t)n * ctx->ne + 255) / 256), 1, ctx->nch), dim3(256), 0,
                        ctx->st, ctx->dc, nt);
     inverse(ctx, P_UL, P_UR, P_ULRINV, -1);
@@ -572,11 +564,13 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
             }
             // (the bond field's submatrix form borders by 2 x 2 blocks: at least two columns)
             const int Ka = std::max(K, 2);
-            v.avec = dalloc<cplx>(ctx, (size_t)n * Ka);
-            v.bvec = dalloc<cplx>(ctx, (size_t)n * Ka);
+            v.avec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX);
+            v.bvec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX);
+            v.updt = dalloc<cplx>(ctx, (size_t)UB * UB);
+            v.updp = dalloc<int32_t>(ctx, UB + 1);
             v.W1 = dalloc<cplx>(ctx, (size_t)n * Ka);
             v.W2 = dalloc<cplx>(ctx, (size_t)Ka * Ka);
-            if (!c.uold || !v.avec || !v.bvec || !v.W1 || !v.W2) {
+            if (!c.uold || !v.avec || !v.bvec || !v.updt || !v.updp || !v.W1 || !v.W2) {
                 int rc = fail(ctx, SH_E_HIP, "device allocation failed");
                 shp_destroy(ctx);
                 return rc;
@@ -585,14 +579,10 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
     }
     if (ctx->update == SHP_U_SUBMATRIX_G) {
         const int Kb = std::max(2, ctx->gblock & ~1);
-        const size_t lds = SUB_LDS_CAP;   // sub_stage's cap; the attribute is shared per function
         const size_t ldsv = (size_t)(Kb * (Kb + 1) + 8 * Kb) * sizeof(cplx);
-        if ((lds > 64 * 1024 &&
-             hipFuncSetAttribute((const void *)k_update_submatrix, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-                 hipSuccess) ||
-            (ldsv > 64 * 1024 &&
-             hipFuncSetAttribute((const void *)k_vupdate_submatrix, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsv) !=
-                 hipSuccess)) {
+        if (ldsv > 64 * 1024 &&
+            hipFuncSetAttribute((const void *)k_vupdate_submatrix, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsv) !=
+                hipSuccess) {
             (void)hipGetLastError();
             int rc = fail(ctx, SH_E_HIP, "dynamic LDS request above the device limit");
             shp_destroy(ctx);

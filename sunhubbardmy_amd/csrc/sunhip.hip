@@ -8,6 +8,7 @@
 #include "dyn_kernels.hip"
 #include "eqt_kernels.hip"
 #include "tv_kernels.hip"
+#include "update_kernels.hip"
 #include "plq_kernels.hip"
 #include "fft_kernels.hip"
 #include "../../include/sunhip.h"
@@ -18,6 +19,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -25,7 +27,7 @@ namespace {
 // timer classes: one per kernel group, in the order reported by sh_timers
 enum {
     T_WRAP = 0,   // k_cb_cols / k_cb_rows / dense-K GEMMs on G, per slice
-    T_UPDATE,     // k_update_delay / k_update_submatrix
+    T_UPDATE,     // k_upd_sites, k_upd_panel, k_upd_flush; the bond and plaquette updates
     T_BPROD,      // B products of the stabilization (k_cb_cols over nwrap slices)
     T_QR,         // k_prepivot + k_qr
     T_FORMQ,      // k_formq
@@ -68,7 +70,7 @@ struct sh_ctx : ctx_base {
     DChain *dc = nullptr;
     int32_t *d_seeds = nullptr;
     bool started = false;
-    bool legacy_update = false;   // test hook: the L2-resident delay update kernel
+    bool legacy_update = false;   // test hook: the fast form of the bond update whatever the build's
     int ntdm = -1;                // time-displaced measurement: bins 0 .. ntdm, -1 = off
     size_t eqt_lds = 0;           // LDS of k_eqt, 0 while no chain has correlation bins
     int lwrapv = 0;               // the batch carries the t-V bond field
@@ -92,8 +94,6 @@ struct sh_ctx : ctx_base {
     int graph_epoch = 1;
     hipGraphExec_t gexec[8] = {};
     int gepoch[8] = {};
-    // autotuner (sh_autotune): saved chain state per chain (G, HS field, scalars)
-    std::vector<void *> tune_save;
 };
 
 #define HIPCHK(x)                                                                  \
@@ -576,59 +576,32 @@ static void set_identity(sh_ctx *ctx, int pt)
     hipLaunchKernelGGL(k_set_identity, grid_elem(ctx), dim3(256), 0, ctx->st, ctx->dc, pt);
 }
 
-// register-resident delay update: the template depth covering every chain's nublock, and the
-// thread count 2 * rows; 0 when the register budget does not allow it
-// the submatrix kernel's LDS: Gamma^-1, the K column scales and dss staged columns and rows of G;
-// dss = the largest staging depth <= 8 within SUB_LDS_CAP (>= 1 up to N = 1024 at K = 64)
-// the kernel also holds 44 KiB of static LDS (the MFMA tiles of the flush, the per-site partial
-// sums); static plus dynamic stays within the 160 KiB of a CU
-#define SUB_LDS_CAP ((size_t)112 * 1024)
-static size_t lds_sub(int n, int K, int dss) { return (size_t)(K * (K + 1) + K + 2 * (size_t)dss * n) * sizeof(cplx); }
-static int sub_stage(int n, int K)
+// the on-site update of one slice (update_kernels.hip), for the chains of either sweep: one kernel
+// while every chain's G fits in the registers of a workgroup, else three launches per block of
+// UB sites (the last block's kernel is sized for the largest chain's remainder)
+static void site_update(hipStream_t st, const DChain *dc, int nch, int nmax, int nt, int slice)
 {
-    int dss = 8;
-    while (dss > 1 && lds_sub(n, K, dss) > SUB_LDS_CAP) dss--;
-    return dss;
-}
-static int delay_reg_depth(sh_ctx *ctx, int *threads)
-{
-    int kmax = 0;
-    for (auto &c : ctx->hc) kmax = std::max(kmax, c.nublock);
-    int kt = kmax <= 4 ? 4 : kmax <= 8 ? 8 : kmax <= 16 ? 16 : kmax <= 32 ? 32 : 0;
-    int rows = (ctx->nmax + 31) / 32 * 32;
-    int nt = 2 * rows;
-    if (kt == 0 || nt > (kt >= 8 ? 512 : 1024)) return 0;
-    // LDS: diag, DSB staged columns and rows, two row buffers, uniforms and HS field
-    if ((size_t)(1 + 2 * DSB) * ctx->nmax * sizeof(cplx) + 4 * kt * sizeof(cplx) + (size_t)ctx->nmax * 20 > 150 * 1024)
-        return 0;
-    *threads = nt;
-    return kt;
+    auto sites = [&](auto whole, int rem, int s0) {
+        constexpr bool W = decltype(whole)::value;
+        auto k = rem <= 16 ? k_upd_sites<1, W> : rem <= 32 ? k_upd_sites<2, W> : rem <= 48 ? k_upd_sites<3, W> : k_upd_sites<4, W>;
+        hipLaunchKernelGGL(k, dim3(nch), dim3(256), 0, st, dc, nt, slice, s0);
+    };
+    if (nmax <= UB) {
+        sites(std::true_type(), nmax, 0);
+        return;
+    }
+    const int ntl = (nmax + GT - 1) / GT, nch8 = (nch + 7) / 8 * 8;
+    for (int s0 = 0; s0 < nmax; s0 += UB) {
+        sites(std::false_type(), std::min(UB, nmax - s0), s0);
+        hipLaunchKernelGGL(k_upd_panel, dim3(ntl, 1, nch), dim3(256), 0, st, dc, s0);
+        hipLaunchKernelGGL(k_upd_flush, dim3(nch8 * ntl * ntl), dim3(256), 0, st, dc, nch, ntl, s0);
+    }
 }
 
 static void update_slice(sh_ctx *ctx, int nt, int slice_in_pass)
 {
     Tic t(ctx, T_UPDATE);
-    int nthr = 0;
-    int kt = (ctx->update == SH_U_DELAY && !ctx->legacy_update) ? delay_reg_depth(ctx, &nthr) : 0;
-    if (kt) {
-        size_t lds = (size_t)(ctx->nmax + 2 * DSB * ctx->nmax + 4 * kt) * sizeof(cplx) + (size_t)ctx->nmax * 20;
-        switch (kt) {
-        case 4: hipLaunchKernelGGL(k_update_delay_reg<4>, dim3(ctx->nch), dim3(nthr), lds, ctx->st, ctx->dc, nt, slice_in_pass); break;
-        case 8: hipLaunchKernelGGL(k_update_delay_reg<8>, dim3(ctx->nch), dim3(nthr), lds, ctx->st, ctx->dc, nt, slice_in_pass); break;
-        case 16: hipLaunchKernelGGL(k_update_delay_reg<16>, dim3(ctx->nch), dim3(nthr), lds, ctx->st, ctx->dc, nt, slice_in_pass); break;
-        default: hipLaunchKernelGGL(k_update_delay_reg<32>, dim3(ctx->nch), dim3(nthr), lds, ctx->st, ctx->dc, nt, slice_in_pass); break;
-        }
-    } else if (ctx->update == SH_U_DELAY) {
-        // diag(G), two rows of the delayed vectors, the slice's uniforms and HS field
-        size_t lds = (size_t)(ctx->nmax + 2 * 64) * sizeof(cplx) + (size_t)ctx->nmax * 20;
-        hipLaunchKernelGGL(k_update_delay, dim3(ctx->nch), dim3(256), lds, ctx->st, ctx->dc, nt, slice_in_pass);
-    } else {
-        int K = 0;
-        for (auto &c : ctx->hc) K = std::max(K, c.nublock);
-        const int dss = sub_stage(ctx->nmax, K);
-        hipLaunchKernelGGL(k_update_submatrix, dim3(ctx->nch), dim3(256), lds_sub(ctx->nmax, K, dss), ctx->st, ctx->dc, nt,
-                           slice_in_pass, dss);
-    }
+    site_update(ctx->st, ctx->dc, ctx->nch, ctx->nmax, nt, slice_in_pass);
 }
 
 static void measure(sh_ctx *ctx)
@@ -791,14 +764,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         struct { const void *f; size_t bytes; } big[] = {
             {(const void *)k_cb_rows, lds_rows(ctx)}, {(const void *)k_cb_cols, lds_cols(ctx)},
             {(const void *)k_fft_rows, lds_fft(ctx)}, {(const void *)k_fft_cols, lds_fft(ctx)},
-            // the cap sub_stage works to: the attribute is per function, shared with the
-            // projective library's launches of the same kernel
-            {(const void *)k_update_submatrix, SUB_LDS_CAP},
             {(const void *)k_vupdate_submatrix, (size_t)(SH_KMAX * (SH_KMAX + 1) + 8 * SH_KMAX) * sizeof(cplx)},
-            {(const void *)k_update_delay_reg<4>, (size_t)(1 + 2 * DSB) * ctx->nmax * sizeof(cplx) + ctx->nmax * 20 + 16 * sizeof(cplx)},
-            {(const void *)k_update_delay_reg<8>, (size_t)(1 + 2 * DSB) * ctx->nmax * sizeof(cplx) + ctx->nmax * 20 + 32 * sizeof(cplx)},
-            {(const void *)k_update_delay_reg<16>, (size_t)(1 + 2 * DSB) * ctx->nmax * sizeof(cplx) + ctx->nmax * 20 + 64 * sizeof(cplx)},
-            {(const void *)k_update_delay_reg<32>, (size_t)(1 + 2 * DSB) * ctx->nmax * sizeof(cplx) + ctx->nmax * 20 + 128 * sizeof(cplx)},
             {(const void *)k_qr_blk, blocked(ctx) ? lds_blk(ctx) : 0},
             {(const void *)k_formq_blk, blocked(ctx) ? lds_blk(ctx) : 0},
             {(const void *)k_tfactors, blocked(ctx) ? lds_blk(ctx) : 0},
@@ -876,9 +842,8 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         c.U = dalloc<cplx>(ctx, nn * (q.nst + 1)); c.V = dalloc<cplx>(ctx, nn * (q.nst + 1));
         c.D = dalloc<double>(ctx, (size_t)n * (q.nst + 1)); c.Ds = dalloc<double>(ctx, n);
         c.ldq = dalloc<cplx>(ctx, q.nst + 1);
-        // room for every depth the autotuner may pick
-        const int kb = std::max(q.nublock, SH_KMAX);
-        c.avec = dalloc<cplx>(ctx, (size_t)n * kb); c.bvec = dalloc<cplx>(ctx, (size_t)n * kb);
+        c.avec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX); c.bvec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX);
+        c.updt = dalloc<cplx>(ctx, (size_t)UB * UB); c.updp = dalloc<int32_t>(ctx, UB + 1);
         c.tau = dalloc<cplx>(ctx, n); c.jpvt = dalloc<int32_t>(ctx, n); c.piv = dalloc<int32_t>(ctx, n);
         c.lperm = dalloc<int32_t>(ctx, n);
         c.wk = dalloc<cplx>(ctx, (size_t)PB * n);
@@ -895,7 +860,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         c.stag = dupload<double>(ctx, q.stag, n);
         c.sc = dalloc<double>(ctx, SC_SIZE);
         if (!c.G || !c.Gs || !c.W1 || !c.W2 || !c.W3 || !c.W4 || !c.Us || !c.Vs || !c.U || !c.V || !c.D || !c.Ds ||
-            !c.ldq || !c.avec || !c.bvec || !c.tau || !c.jpvt || !c.piv || !c.rwork || !c.conf || !c.unif || !c.wk || !c.tblk ||
+            !c.ldq || !c.avec || !c.bvec || !c.updt || !c.updp || !c.tau || !c.jpvt || !c.piv || !c.rwork || !c.conf || !c.unif || !c.wk || !c.tblk ||
             !c.rng || !c.bonds || !c.kt || !c.ktm1 || !c.stag || !c.sc) {
             int rc = fail(ctx, SH_E_HIP, "device allocation failed");
             sh_destroy(ctx);
@@ -957,7 +922,6 @@ int sh_destroy(sh_ctx *ctx)
     for (cplx *p : ctx->trace_bufs) if (p) hipFree(p);
     for (auto e : ctx->pool) hipEventDestroy(e);
     for (auto g : ctx->gexec) if (g) hipGraphExecDestroy(g);
-    for (void *p : ctx->tune_save) hipFree(p);
     if (ctx->st) hipStreamDestroy(ctx->st);
     delete ctx;
     return 0;
@@ -1661,50 +1625,10 @@ int sh_set_graphs(sh_ctx *ctx, int enable)
 }
 
 // ---- autotuner -------------------------------------------------------------------------------
-// The update of one slice (slice ltrot, the first of a b0 pass) is timed on the chains' current
-// G at every candidate depth, with the state every trial changes (G, the slice's HS field, the
-// scalar slots) restored before each trial and at the end, and the slice's uniforms replaced
-// by a fixed low-discrepancy sequence (the next updating pass draws its own).  Then the DFT
-// kinetic kernels at every vectors-per-workgroup that fits, on the scratch matrix W1.
+// The DFT kinetic kernels are timed at every vectors-per-workgroup that fits, on the scratch matrix
+// W1.  The on-site update has no depth to pick: it flushes once per block of UB sites whatever
+// nublock is (update_kernels.hip), so nublock is returned as it is.
 }  // extern "C"
-
-__global__ void k_tune_unif(const DChain *chains)
-{
-    const DChain &c = chains[blockIdx.x];
-    for (int i = threadIdx.x; i < c.n; i += blockDim.x) {
-        const double a = 0.5 + 0.6180339887498949 * i, b = 0.25 + 0.7548776662466927 * i;
-        c.unif[2 * i] = a - floor(a);
-        c.unif[2 * i + 1] = b - floor(b);
-    }
-}
-
-static int tune_state(sh_ctx *ctx, bool save)
-{
-    const int nt = ctx->ltrot;
-    for (int ci = 0; ci < ctx->nch; ci++) {
-        const DChain &c = ctx->hc[ci];
-        const size_t gb = (size_t)c.n * c.n * sizeof(cplx), cb = (size_t)c.n * sizeof(int32_t);
-        char *p = (char *)ctx->tune_save[ci];
-        int32_t *cf = c.conf + (size_t)(nt - 1) * c.n;
-        if (save) {
-            HIPCHK(hipMemcpyAsync(p, c.G, gb, hipMemcpyDeviceToDevice, ctx->st));
-            HIPCHK(hipMemcpyAsync(p + gb, cf, cb, hipMemcpyDeviceToDevice, ctx->st));
-            HIPCHK(hipMemcpyAsync(p + gb + cb, c.sc, SC_SIZE * sizeof(double), hipMemcpyDeviceToDevice, ctx->st));
-        } else {
-            HIPCHK(hipMemcpyAsync(c.G, p, gb, hipMemcpyDeviceToDevice, ctx->st));
-            HIPCHK(hipMemcpyAsync(cf, p + gb, cb, hipMemcpyDeviceToDevice, ctx->st));
-            HIPCHK(hipMemcpyAsync(c.sc, p + gb + cb, SC_SIZE * sizeof(double), hipMemcpyDeviceToDevice, ctx->st));
-        }
-    }
-    return 0;
-}
-
-static int set_nublock(sh_ctx *ctx, int k)
-{
-    for (auto &c : ctx->hc) c.nublock = k;
-    HIPCHK(hipMemcpy(ctx->dc, ctx->hc.data(), sizeof(DChain) * ctx->nch, hipMemcpyHostToDevice));
-    return 0;
-}
 
 // best of `reps` timed runs of f (after one untimed run), in ms; before() runs outside the timing
 template <class Before, class F>
@@ -1735,44 +1659,6 @@ int sh_autotune(sh_ctx *ctx, int *tuned)
     if (ctx->timing) return fail(ctx, SH_E_STATE, "sh_autotune with the timers on");
     HIPCHK(hipStreamSynchronize(ctx->st));
     const int k0 = ctx->hc[0].nublock;
-    int best_k = k0;
-    if (ctx->hc[0].lwrapu) {
-        if (ctx->tune_save.empty()) {
-            for (auto &c : ctx->hc) {
-                void *p = nullptr;
-                const size_t bytes = (size_t)c.n * c.n * sizeof(cplx) + (size_t)c.n * sizeof(int32_t) + SC_SIZE * sizeof(double);
-                HIPCHK(hipMalloc(&p, bytes));
-                ctx->tune_save.push_back(p);
-            }
-        }
-        int rc = tune_state(ctx, true);
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_tune_unif, dim3(ctx->nch), dim3(256), 0, ctx->st, ctx->dc);
-        std::vector<int> cand;
-        if (ctx->update == SH_U_DELAY) {
-            if (k0 > 1) {
-                // register-resident depths where they fit, the memory-resident kernel above
-                for (int k : {4, 8, 16, 32}) cand.push_back(k);
-                int thr = 0;
-                for (auto &c : ctx->hc) c.nublock = 32;
-                const bool reg32 = delay_reg_depth(ctx, &thr) != 0;
-                for (auto &c : ctx->hc) c.nublock = k0;
-                if (!reg32) cand.push_back(64);
-            }
-        } else {
-            for (int k : {8, 16, 24, 32, 48, 64}) cand.push_back(k);
-        }
-        double best = 1e30;
-        for (int k : cand) {
-            if (k > ctx->nmax) continue;
-            if ((rc = set_nublock(ctx, k))) return rc;
-            const double ms = tune_time(ctx, 3, [&]() { tune_state(ctx, false); }, [&]() { update_slice(ctx, ctx->ltrot, 0); });
-            if (hipGetLastError() != hipSuccess) return fail(ctx, SH_E_HIP, "autotune launch failed");
-            if (ms < best) { best = ms; best_k = k; }
-        }
-        if ((rc = set_nublock(ctx, best_k))) return rc;
-        if ((rc = tune_state(ctx, false))) return rc;
-    }
     int best_f = 0;
     if (ctx->kmode == SH_K_FFT) {
         double best = 1e30;
@@ -1792,7 +1678,7 @@ int sh_autotune(sh_ctx *ctx, int *tuned)
     }
     HIPCHK(hipStreamSynchronize(ctx->st));
     ctx->graph_epoch++;
-    tuned[0] = best_k;
+    tuned[0] = k0;
     tuned[1] = best_f;
     return 0;
 }

@@ -80,7 +80,9 @@ struct DChain {
     cplx *U, *V;          // (nst+1) points, n*n each
     double *D, *Ds;       // (nst+1)*n, n
     cplx *ldq;            // nst+1
-    cplx *avec, *bvec;    // n*nublock
+    cplx *avec, *bvec;    // n*64 (k_upd_panel); n*nublock delayed vectors of the bond field
+    cplx *updt;           // 64 x 64: T of the on-site update's current block of sites
+    int32_t *updp;        // its accepted sites: count, then the sites
     cplx *tau;            // n
     cplx *wk;             // 16 x n work block of the blocked factorizations
     cplx *tblk;           // (n/16 + 1) triangular 16 x 16 factors of the block reflectors

@@ -296,8 +296,8 @@ class FTWalkers:
         self._check(_lib.lib().sh_set_graphs(self._ctx, int(bool(enable))), "set_graphs")
 
     def autotune(self):
-        """Pick the delay depth / submatrix block (and the DFT kernels' tile) by timing them on
-        the chains' current state, which is left unchanged; call after sweep_start_0b."""
+        """Pick the DFT kernels' vectors per workgroup by timing them; reports nublock unchanged;
+        the chains' state is left unchanged; call after sweep_start_0b."""
         out = np.zeros(2, np.int32)
         self._check(_lib.lib().sh_autotune(self._ctx, out.ctypes.data_as(_lib.ip)), "autotune")
         for t in self.tables:
