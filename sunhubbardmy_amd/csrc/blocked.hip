@@ -699,17 +699,19 @@ k_lu_blk(const DChain *chains)
 }
 
 // ------------------------------------------------------------------------------------------
-// (P L U) Y = X in place of X for N <= 256, 16 right-hand sides per workgroup (zgetrs with the
-// factors of k_lu_blk).  The workgroup's 16 columns stay in registers through the forward and
+// (P L U) Y = X in place of X for N <= 64 NW, 16 right-hand sides per workgroup of NW waves (zgetrs
+// with the factors of k_lu_blk).  The workgroup's 16 columns stay in registers through the forward and
 // the backward substitution, in the MFMA accumulator layout: wave w holds the 16-row tiles
-// t = w, w + 4, w + 8, w + 12; lane l, element r of a tile is row 16 t + 4 r + l / 16, column
+// t = w, w + NW, w + 2 NW, w + 3 NW; lane l, element r of a tile is row 16 t + 4 r + l / 16, column
 // l % 16.  Panel p (rows 16 p .. 16 p + 15) is solved by the wave that holds tile p against the
 // 16 x 16 diagonal block (staged in LDS), published to LDS, and every wave then updates its
 // tiles below (forward, L) or above (backward, U) by one rank-16 MFMA product per tile whose
 // factor block is read from global memory.  A chain's workgroups run on one XCD
 // (blockIdx.x % 8 picks it) so that they share the factor's panels in that XCD's L2.
+// Bound by the chain of 2 N/16 panel solves; with every column block on its own CU one N = 288 chain
+// takes 0.18 ms (1.87 by panels in one workgroup), sixteen N = 400 chains 0.54 (4.34).
 // ------------------------------------------------------------------------------------------
-#define SCB_T 4   // tiles per wave: N <= 256
+#define SCB_T 4   // tiles per wave
 
 // forward (unit lower, lower = 1) or backward (upper with diagonal reciprocals dinv) solve of
 // one 16 x 16 tile held in accumulator layout, against D11[a * 16 + b] in LDS
@@ -741,7 +743,7 @@ __device__ __forceinline__ void cb_tri(double4_t &xr, double4_t &xi, const cplx 
 }
 
 // tiles of this wave past (forward) or before (backward) panel p -= F(tile rows, panel cols) Xp
-template <bool FWD>
+template <int NW, bool FWD>
 __device__ __forceinline__ void cb_update(double4_t (&xr)[SCB_T], double4_t (&xi)[SCB_T], GAS cplx *A, int n, int p,
                                           int w, int lq, int l16, const cplx *Xp)
 {
@@ -751,7 +753,7 @@ __device__ __forceinline__ void cb_update(double4_t (&xr)[SCB_T], double4_t (&xi
     for (int s = 0; s < 4; s++) bv[s] = Xp[(4 * s + lq) * 16 + l16];
 #pragma unroll
     for (int tt = 0; tt < SCB_T; tt++) {
-        const int tile = w + 4 * tt;
+        const int tile = w + NW * tt;
         if (FWD ? tile > p : tile < p) {
             const int row = 16 * tile + l16;
             const size_t rowc = (size_t)min(row, n - 1);
@@ -788,7 +790,7 @@ __device__ __forceinline__ void cb_diag_load(GAS cplx *A, int n, int p, int lane
 
 // the owner of panel p stages the diagonal block (loaded ahead into d), solves its tile,
 // publishes it
-template <bool FWD>
+template <int NW, bool FWD>
 __device__ __forceinline__ void cb_panel(double4_t (&xr)[SCB_T], double4_t (&xi)[SCB_T], const cplx (&d)[4], int p,
                                          int lane, int lq, int l16, cplx *D11, cplx *dinv, cplx *Xp)
 {
@@ -797,7 +799,7 @@ __device__ __forceinline__ void cb_panel(double4_t (&xr)[SCB_T], double4_t (&xi)
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     if (!FWD && lane < 16) dinv[lane] = cinv(D11[lane * 16 + lane]);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const int tp = p >> 2;
+    const int tp = p / NW;
 #pragma unroll
     for (int tt = 0; tt < SCB_T; tt++) {
         if (tt == tp) {
@@ -808,7 +810,8 @@ __device__ __forceinline__ void cb_panel(double4_t (&xr)[SCB_T], double4_t (&xi)
     }
 }
 
-extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4 ? 3 : 2)))
 k_solve_cb(const DChain *chains, int nch, int ncb, int xsel)
 {
     const int bid = blockIdx.x, xcd = bid & 7, kb = bid >> 3;
@@ -831,7 +834,7 @@ k_solve_cb(const DChain *chains, int nch, int ncb, int xsel)
     for (int tt = 0; tt < SCB_T; tt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int row = 16 * (w + 4 * tt) + 4 * r + lq;
+            const int row = 16 * (w + NW * tt) + 4 * r + lq;
             const int pr = perm[min(row, n - 1)];
             const cplx v = gld(X + ((size_t)pr + colc));
             xr[tt][r] = row < n ? v.x : 0.0;
@@ -842,34 +845,29 @@ k_solve_cb(const DChain *chains, int nch, int ncb, int xsel)
     cplx d[4];
     if (w == 0) cb_diag_load(A, n, 0, lane, d);
     for (int p = 0; p < nt; p++) {
-        if (w == (p & 3)) cb_panel<true>(xr, xi, d, p, lane, lq, l16, D11, dinv, Xp[p & 1]);
-        if (w == ((p + 1) & 3)) cb_diag_load(A, n, p + 1 < nt ? p + 1 : nt - 1, lane, d);
+        if (w == p % NW) cb_panel<NW, true>(xr, xi, d, p, lane, lq, l16, D11, dinv, Xp[p & 1]);
+        if (w == (p + 1) % NW) cb_diag_load(A, n, p + 1 < nt ? p + 1 : nt - 1, lane, d);
         __syncthreads();
-        cb_update<true>(xr, xi, A, n, p, w, lq, l16, Xp[p & 1]);
+        cb_update<NW, true>(xr, xi, A, n, p, w, lq, l16, Xp[p & 1]);
     }
     __syncthreads();
     for (int p = nt - 1; p >= 0; p--) {
-        if (w == (p & 3)) cb_panel<false>(xr, xi, d, p, lane, lq, l16, D11, dinv, Xp[p & 1]);
-        if (w == ((p + 3) & 3)) cb_diag_load(A, n, p > 0 ? p - 1 : 0, lane, d);
+        if (w == p % NW) cb_panel<NW, false>(xr, xi, d, p, lane, lq, l16, D11, dinv, Xp[p & 1]);
+        if (w == (p + NW - 1) % NW) cb_diag_load(A, n, p > 0 ? p - 1 : 0, lane, d);
         __syncthreads();
-        cb_update<false>(xr, xi, A, n, p, w, lq, l16, Xp[p & 1]);
+        cb_update<NW, false>(xr, xi, A, n, p, w, lq, l16, Xp[p & 1]);
     }
 #pragma unroll
     for (int tt = 0; tt < SCB_T; tt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int row = 16 * (w + 4 * tt) + 4 * r + lq;
+            const int row = 16 * (w + NW * tt) + 4 * r + lq;
             if (row < n && col < n) gst(X + ((size_t)row + (size_t)col * n), make_double2(xr[tt][r], xi[tt][r]));
         }
 }
 
-extern "C" __global__ void __launch_bounds__(BLK_NT)
-k_solve_blk(const DChain *chains, int xsel)
-{
-    extern __shared__ cplx bsh[];
-    const DChain &c = chains[blockIdx.x];
-    solve_blk_body(c.W3, c.n, c.n, c.piv, chain_mat(c, xsel, 0), c.n, c.n, c.W2, bsh);
-}
+template __global__ void k_solve_cb<4>(const DChain *, int, int, int);
+template __global__ void k_solve_cb<8>(const DChain *, int, int, int);
 
 // T factors of the reflectors that the column-at-a-time (pivoted) QR left in matrix sel, panel
 // by panel, so that k_formq_blk forms Q by rank-16 MFMA products

@@ -280,13 +280,15 @@ static void lu_factor(sh_ctx *ctx)
 static void lu_solve(sh_ctx *ctx, int xsel)
 {
     Tic t(ctx, T_SOLVE);
-    if (ctx->nmax <= 16 * 4 * SCB_T) {
-        // 16 right-hand sides per workgroup, a chain's workgroups on one XCD
+    if (blocked(ctx)) {
+        // 16 right-hand sides per workgroup, a chain's workgroups on one XCD; four waves of four
+        // tiles hold 256 rows, eight hold 512
         const int ncb = (ctx->nmax + 15) / 16, nch8 = (ctx->nch + 7) / 8 * 8;
-        hipLaunchKernelGGL(k_solve_cb, dim3(nch8 * ncb), dim3(256), 0, ctx->st, ctx->dc, ctx->nch, ncb, xsel);
-    } else if (blocked(ctx))
-        hipLaunchKernelGGL(k_solve_blk, dim3(ctx->nch), dim3(BLK_NT), lds_blk(ctx), ctx->st, ctx->dc, xsel);
-    else
+        if (ctx->nmax <= 256)
+            hipLaunchKernelGGL(k_solve_cb<4>, dim3(nch8 * ncb), dim3(256), 0, ctx->st, ctx->dc, ctx->nch, ncb, xsel);
+        else
+            hipLaunchKernelGGL(k_solve_cb<8>, dim3(nch8 * ncb), dim3(512), 0, ctx->st, ctx->dc, ctx->nch, ncb, xsel);
+    } else
         hipLaunchKernelGGL(k_lu_solve, dim3(ctx->nch), dim3(512), 0, ctx->st, ctx->dc, xsel);
 }
 
@@ -768,8 +770,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
             {(const void *)k_qr_blk, blocked(ctx) ? lds_blk(ctx) : 0},
             {(const void *)k_formq_blk, blocked(ctx) ? lds_blk(ctx) : 0},
             {(const void *)k_tfactors, blocked(ctx) ? lds_blk(ctx) : 0},
-            {(const void *)k_lu_blk, blocked(ctx) ? lds_blk(ctx) : 0},
-            {(const void *)k_solve_blk, blocked(ctx) ? lds_blk(ctx) : 0}};
+            {(const void *)k_lu_blk, blocked(ctx) ? lds_blk(ctx) : 0}};
         for (auto &b : big) {
             if (b.bytes <= 64 * 1024 || b.bytes > 150 * 1024) continue;
             hipFuncAttributes fa;
