@@ -190,7 +190,7 @@ void update_u_g(shp_ctx *ctx, int nt, size_t uoff0)
     Tic t(ctx, T_UPDATE);
     hipLaunchKernelGGL(kp_u_save, dim3((n + 255) / 256, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nt);
     const int slice = (int)(uoff0 / (2 * (size_t)n));
-    site_update(ctx->st, ctx->dview, ctx->nch, n, nt, slice);
+    site_update(ctx->st, ctx->dview, ctx->nch, n, false, nt, slice);
     hipLaunchKernelGGL(kp_u_rescale, dim3((unsigned)(((size_t)n * ctx->ne + 255) / 256), 1, ctx->nch), dim3(256), 0,
                        ctx->st, ctx->dc, nt);
     inverse(ctx, P_UL, P_UR, P_ULRINV, -1);

@@ -75,6 +75,7 @@ struct sh_ctx : ctx_base {
     size_t eqt_lds = 0;           // LDS of k_eqt, 0 while no chain has correlation bins
     int lwrapv = 0;               // the batch carries the t-V bond field
     int lwrapp = 0;               // the batch carries the plaquette field
+    bool flav2 = true;            // nflr = 2 in every chain
     // push/pop_stage backups
     std::vector<void *> stage;
     std::vector<cplx *> trace_bufs;
@@ -581,20 +582,24 @@ static void set_identity(sh_ctx *ctx, int pt)
 // the on-site update of one slice (update_kernels.hip), for the chains of either sweep: one kernel
 // while every chain's G fits in the registers of a workgroup, else three launches per block of
 // UB sites (the last block's kernel is sized for the largest chain's remainder)
-static void site_update(hipStream_t st, const DChain *dc, int nch, int nmax, int nt, int slice)
+template <bool WHOLE, int NF>
+static void launch_sites(hipStream_t st, const DChain *dc, int nch, int rem, int nt, int slice, int s0)
 {
-    auto sites = [&](auto whole, int rem, int s0) {
-        constexpr bool W = decltype(whole)::value;
-        auto k = rem <= 16 ? k_upd_sites<1, W> : rem <= 32 ? k_upd_sites<2, W> : rem <= 48 ? k_upd_sites<3, W> : k_upd_sites<4, W>;
-        hipLaunchKernelGGL(k, dim3(nch), dim3(256), 0, st, dc, nt, slice, s0);
-    };
+    const int tiles = (rem + 15) / 16;
+    auto k = tiles == 1 ? k_upd_sites<1, WHOLE, NF> : tiles == 2 ? k_upd_sites<2, WHOLE, NF> :
+             tiles == 3 ? k_upd_sites<3, WHOLE, NF> : k_upd_sites<4, WHOLE, NF>;
+    hipLaunchKernelGGL(k, dim3(nch), dim3(64 * tiles), 0, st, dc, nt, slice, s0);
+}
+// flav2: every chain has two flavours (the ratio's power is then unrolled)
+static void site_update(hipStream_t st, const DChain *dc, int nch, int nmax, bool flav2, int nt, int slice)
+{
     if (nmax <= UB) {
-        sites(std::true_type(), nmax, 0);
+        (flav2 ? launch_sites<true, 2> : launch_sites<true, 0>)(st, dc, nch, nmax, nt, slice, 0);
         return;
     }
     const int ntl = (nmax + GT - 1) / GT, nch8 = (nch + 7) / 8 * 8;
     for (int s0 = 0; s0 < nmax; s0 += UB) {
-        sites(std::false_type(), std::min(UB, nmax - s0), s0);
+        (flav2 ? launch_sites<false, 2> : launch_sites<false, 0>)(st, dc, nch, std::min(UB, nmax - s0), nt, slice, s0);
         hipLaunchKernelGGL(k_upd_panel, dim3(ntl, 1, nch), dim3(256), 0, st, dc, s0);
         hipLaunchKernelGGL(k_upd_flush, dim3(nch8 * ntl * ntl), dim3(256), 0, st, dc, nch, ntl, s0);
     }
@@ -603,7 +608,7 @@ static void site_update(hipStream_t st, const DChain *dc, int nch, int nmax, int
 static void update_slice(sh_ctx *ctx, int nt, int slice_in_pass)
 {
     Tic t(ctx, T_UPDATE);
-    site_update(ctx->st, ctx->dc, ctx->nch, ctx->nmax, nt, slice_in_pass);
+    site_update(ctx->st, ctx->dc, ctx->nch, ctx->nmax, ctx->flav2, nt, slice_in_pass);
 }
 
 static void measure(sh_ctx *ctx)
@@ -750,6 +755,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         for (int i = 0; i < 2 * q.nst; i++)
             if (q.wrap_step[i] < 1 || q.wrap_step[i] > q.ltrot) { delete ctx; return SH_E_ARG; }
         ctx->nmax = std::max(ctx->nmax, q.ndim);
+        ctx->flav2 = ctx->flav2 && q.nflr == 2;
     }
     // DFT kinetic form: as many vectors per workgroup (<= 16) as fit in 96 KiB of LDS
     if (ctx->kmode == SH_K_FFT) {
