@@ -631,76 +631,8 @@ __device__ __forceinline__ void solve_blk_body(const cplx *A, int n, int lda, co
 }
 
 // ------------------------------------------------------------------------------------------
-// The finite-temperature chain's N x N factorizations (one workgroup per chain)
-// ------------------------------------------------------------------------------------------
-extern "C" __global__ void __launch_bounds__(BLK_NT)
-k_qr_blk(const DChain *chains, int sel, int out_pt)
-{
-    extern __shared__ cplx bsh[];
-    __shared__ double red[16];
-    const DChain &c = chains[blockIdx.x];
-    const int n = c.n;
-    qr_blk_body(chain_mat(c, sel, 0), n, n, n, c.tau, c.tblk, c.wk, PB, bsh);
-    // log det Q = sum_i log(1 - tau_i 2 Re(tau_i) / |tau_i|^2), summed by the whole workgroup
-    double sr = 0.0, si = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const cplx t = gld(gp(c.tau) + i);
-        if (t.x != 0.0 || t.y != 0.0) {
-            const cplx q = cdiv(cscale(t, 2.0 * t.x), cmul(t, cconj(t)));
-            const cplx l = clog_(make_double2(1.0 - q.x, -q.y));
-            sr += l.x;
-            si += l.y;
-        }
-    }
-    sr = blk_sum(sr, red);
-    si = blk_sum(si, red);
-    if (threadIdx.x == 0) c.ldq[out_pt] = make_double2(sr, si);
-}
-
-extern "C" __global__ void __launch_bounds__(BLK_NT)
-k_formq_blk(const DChain *chains, int sel, int out_pt)
-{
-    extern __shared__ cplx bsh[];
-    const DChain &c = chains[blockIdx.x];
-    const int n = c.n;
-    formq_blk_body(chain_mat(c, sel, 0), n, n, n, c.U + (size_t)n * n * out_pt, n, c.tblk, c.wk, PB, bsh);
-}
-
-extern "C" __global__ void __launch_bounds__(BLK_NT)
-k_lu_blk(const DChain *chains)
-{
-    extern __shared__ cplx bsh[];
-    const DChain &c = chains[blockIdx.x];
-    __shared__ cplx s_ld;
-    __shared__ double s_inf;
-    lu_blk_body(c.W3, c.n, c.n, c.piv, &s_ld, &s_inf, bsh);
-    // the row order of the interchanges, for k_solve_cb: the pivots into LDS, the swaps in order
-    // by one thread, the result out
-    const int n = c.n;
-    int *perm = (int *)bsh, *pv = perm + n;
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        perm[i] = i;
-        pv[i] = c.piv[i];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        c.sc[SC_ZLD] = s_ld.x;
-        c.sc[SC_ZLD + 1] = s_ld.y;
-        c.sc[SC_INFO] = s_inf;
-        for (int k = 0; k < n; k++) {
-            const int p = pv[k], t = perm[p];
-            perm[p] = perm[k];
-            perm[k] = t;
-        }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) c.lperm[i] = perm[i];
-}
-
-// ------------------------------------------------------------------------------------------
 // (P L U) Y = X in place of X for N <= 64 NW, 16 right-hand sides per workgroup of NW waves (zgetrs
-// with the factors of k_lu_blk).  The workgroup's 16 columns stay in registers through the forward and
+// with the factors of k_lu_step).  The workgroup's 16 columns stay in registers through the forward and
 // the backward substitution, in the MFMA accumulator layout: wave w holds the 16-row tiles
 // t = w, w + NW, w + 2 NW, w + 3 NW; lane l, element r of a tile is row 16 t + 4 r + l / 16, column
 // l % 16.  Panel p (rows 16 p .. 16 p + 15) is solved by the wave that holds tile p against the

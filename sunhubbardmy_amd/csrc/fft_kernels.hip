@@ -17,7 +17,7 @@
 // and once per launch from HBM.  Lines of a column are padded (one slot per n0-run, an odd
 // leading dimension per column) so that neither the lines along n0 nor the staging accesses of
 // consecutive rows fall on one LDS bank.
-#include "sunhip_kernels.h"
+#include "fft_kernels.h"
 
 #define FFT_LMAX 24
 
@@ -98,11 +98,6 @@ struct FftGeo {
     int ld;
 };
 
-__host__ __device__ __forceinline__ int fft_ld(int n, int n0)
-{
-    const int ld = n + n / n0;
-    return ld | 1;
-}
 
 __device__ __forceinline__ int fft_pad(int s, int n0) { return s + s / n0; }
 

@@ -154,61 +154,6 @@ k_sfmt_draw(const DChain *chains, int nchains, int mode)
 #define CPB 8
 #define RPB 8
 
-// Global <-> LDS staging with ST_BATCH independent 16-byte accesses in flight per thread: a
-// batch's loads are all issued before its first LDS store, so a workgroup waits for one memory
-// latency per batch instead of one per element.  ld(e) returns element e of the tile, st(e, v)
-// writes it back.
-#define ST_BATCH 8
-template <int B, class Ld, class Ix>
-__device__ __forceinline__ void stage_in_map(cplx *lds, int total, Ld ld, Ix ix)
-{
-    for (int base = threadIdx.x; base < total; base += B * blockDim.x) {
-        cplx v[B];
-#pragma unroll
-        for (int u = 0; u < B; u++) {
-            const int e = base + u * (int)blockDim.x;
-            v[u] = e < total ? ld(e) : make_double2(0.0, 0.0);
-        }
-#pragma unroll
-        for (int u = 0; u < B; u++) {
-            const int e = base + u * (int)blockDim.x;
-            if (e < total) lds[ix(e)] = v[u];
-        }
-    }
-}
-
-template <class Ld>
-__device__ __forceinline__ void stage_in(cplx *lds, int total, Ld ld)
-{
-    stage_in_map<ST_BATCH>(lds, total, ld, [](int e) { return e; });
-}
-
-template <class St>
-__device__ __forceinline__ void stage_out(const cplx *lds, int total, St st)
-{
-    for (int base = threadIdx.x; base < total; base += ST_BATCH * blockDim.x) {
-        cplx v[ST_BATCH];
-#pragma unroll
-        for (int u = 0; u < ST_BATCH; u++) {
-            const int e = base + u * (int)blockDim.x;
-            v[u] = e < total ? lds[e] : make_double2(0.0, 0.0);
-        }
-#pragma unroll
-        for (int u = 0; u < ST_BATCH; u++) {
-            const int e = base + u * (int)blockDim.x;
-            if (e < total) st(e, v[u]);
-        }
-    }
-}
-
-__device__ __forceinline__ cplx vtab(const DChain &c, int vsel, int is)
-{
-    // vsel 0: bmat, 1: bmat_inv, 2: conj(bmat)
-    cplx b = (vsel == 1) ? c.bmat_inv[is - 1] : c.bmat[is - 1];
-    if (vsel == 2) b.y = -b.y;
-    return b;
-}
-
 // one bond per thread (and a stride of columns): the bond's endpoints and 2x2 block are read
 // once per family and applied to every column the thread covers
 template <class Chain>
@@ -232,16 +177,6 @@ __device__ __forceinline__ void cb_left_fams(const Chain &c, cplx *lds, int ncol
         }
         __syncthreads();
     }
-}
-
-// the four factors of the HS components, staged in LDS once per pass (a register table indexed by
-// the component is lowered to a private-memory lookup)
-__device__ __forceinline__ const cplx *vtab_lds(const DChain &c, int vsel)
-{
-    __shared__ cplx vt[4];
-    if (threadIdx.x < 4) vt[threadIdx.x] = vtab(c, vsel, threadIdx.x + 1);
-    __syncthreads();
-    return vt;
 }
 
 __device__ static void cb_left_v(const DChain &c, cplx *lds, int ncol, int nt, int vsel)
@@ -392,13 +327,6 @@ k_vscale(const DChain *chains, int msel, int pt, int side, int vsel, int vsel2, 
 // MFMA operand layout (probed on gfx950): A(16x4): lane l holds A[l%16][l/16]; B(4x16): lane l
 // holds B[l/16][l%16]; D(16x16): lane l, element r holds D[l/16 + 4r][l%16].
 // ------------------------------------------------------------------------------------------
-#define GT 64
-#define GK 16
-
-__device__ __forceinline__ double4_t mfma(double a, double b, double4_t c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
 
 // one 64 x 64 tile (tm, tn) of C (m x n, ldc) = alpha op(A) op(B) + beta C, op(A) m x kk,
 // op(B) kk x n; op = 0: as stored, 1: conjugate transpose
@@ -963,8 +891,8 @@ k_prepivot(const DChain *chains, int dpt)
     extern __shared__ double psh[];
     const DChain &c = chains[blockIdx.x];
     const int n = c.n;
-    volatile double *vn = psh;
-    volatile int *jp = (volatile int *)(psh + n);
+    double *vn = psh;
+    int *jp = (int *)(psh + n);
     const double *Dp = c.D + (size_t)n * dpt;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     GAS cplx *B = gp(c.W1);
@@ -1000,27 +928,21 @@ k_prepivot(const DChain *chains, int dpt)
         s1 = wave_sum_dpp(s1);
         s2 = wave_sum_dpp(s2);
         if (lane == 0) {
-            vn[j] = sqrt(s1);
-            jp[j] = j + 1;
-            if (two) { vn[j2] = sqrt(s2); jp[j2] = j2 + 1; }
+            vn[j] = s1 == s1 ? sqrt(s1) : -1.0;
+            if (two) vn[j2] = s2 == s2 ? sqrt(s2) : -1.0;
         }
     }
     __syncthreads();
-    if (w == 0) {
-        for (int k = 0; k < n; k++) {
-            double bv = -1.0;
-            int bi = k;
-            for (int j = k + lane; j < n; j += 64) {
-                double a = fabs(vn[j]);
-                if (a > bv) { bv = a; bi = j; }
-            }
-            wave_argmax_dpp(bv, bi);
-            if (lane == 0 && bi != k) {
-                int it = jp[bi]; jp[bi] = jp[k]; jp[k] = it;
-                vn[bi] = vn[k];
-            }
-            __builtin_amdgcn_wave_barrier();
+    // the columns by falling norm, equal norms in their order: every thread counts how many come
+    // before its column (a NaN sorts last)
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        const double vj = vn[j];
+        int rank = 0;
+        for (int q = 0; q < n; q++) {
+            const double v = vn[q];
+            rank += v > vj || (v == vj && q < j) ? 1 : 0;
         }
+        jp[rank] = j + 1;
     }
     __syncthreads();
     for (int j = threadIdx.x; j < n; j += blockDim.x) c.jpvt[j] = jp[j];

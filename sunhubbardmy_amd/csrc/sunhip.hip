@@ -8,9 +8,10 @@
 #include "dyn_kernels.hip"
 #include "eqt_kernels.hip"
 #include "tv_kernels.hip"
-#include "update_kernels.hip"
+#include "update_kernels.h"
 #include "plq_kernels.hip"
-#include "fft_kernels.hip"
+#include "fft_kernels.h"
+#include "factor.h"
 #include "../../include/sunhip.h"
 #include "../../include/sunhip_learn.h"
 
@@ -76,6 +77,7 @@ struct sh_ctx : ctx_base {
     int lwrapv = 0;               // the batch carries the t-V bond field
     int lwrapp = 0;               // the batch carries the plaquette field
     bool flav2 = true;            // nflr = 2 in every chain
+    std::vector<int> lu_blocks;   // workgroups per chain of each launch of k_lu_step
     // push/pop_stage backups
     std::vector<void *> stage;
     std::vector<cplx *> trace_bufs;
@@ -269,12 +271,18 @@ static size_t lds_qr(sh_ctx *ctx) { return (size_t)ctx->nmax * 32; }
 static bool blocked(sh_ctx *ctx) { return ctx->nmax <= BLK_NMAX; }
 static size_t lds_blk(sh_ctx *ctx) { return ((size_t)ctx->nmax * PB + 2 * PB * PB) * sizeof(cplx) + ctx->nmax * 4; }
 
+// waves of a workgroup of the factorizations: each holds 64 of the matrix's rows
+static int fac_waves(sh_ctx *ctx) { return ctx->nmax <= 256 ? 4 : 8; }
+
 static void lu_factor(sh_ctx *ctx)
 {
     Tic t(ctx, T_LU);
-    if (blocked(ctx))
-        hipLaunchKernelGGL(k_lu_blk, dim3(ctx->nch), dim3(BLK_NT), lds_blk(ctx), ctx->st, ctx->dc);
-    else
+    if (blocked(ctx)) {
+        const int np = (ctx->nmax + FPB - 1) / FPB, nw = fac_waves(ctx);
+        for (int k = 0; k <= np; k++)
+            hipLaunchKernelGGL(nw == 4 ? k_lu_step<4> : k_lu_step<8>, dim3(ctx->nch, ctx->lu_blocks[k]), dim3(64 * nw), 0,
+                               ctx->st, ctx->dc, k);
+    } else
         hipLaunchKernelGGL(k_lu, dim3(ctx->nch), dim3(1024), (size_t)ctx->nmax * 2 * sizeof(cplx), ctx->st, ctx->dc);
 }
 
@@ -301,7 +309,18 @@ static void launch_qr(sh_ctx *ctx, int sel, int pivot, int pt)
     hipLaunchKernelGGL(k, dim3(ctx->nch), dim3(1024), lds_qr(ctx), ctx->st, ctx->dc, sel, pivot, pt);
 }
 
-// QR of W1 (first point: column pivoting) or of the prepivoted W1 diag(D[dpt]) -> point `pt`
+// Q of the reflectors in matrix sel -> U[pt]: 16 columns per workgroup, a chain's workgroups on one XCD
+static void formq(sh_ctx *ctx, int sel, int pt)
+{
+    const int ncb = (ctx->nmax + FPB - 1) / FPB, nch8 = (ctx->nch + 7) / 8 * 8, nw = fac_waves(ctx);
+    hipLaunchKernelGGL(nw == 4 ? k_formq_cb<4> : k_formq_cb<8>, dim3(nch8 * ncb), dim3(64 * nw), 0, ctx->st, ctx->dc,
+                       ctx->nch, ncb, sel, pt);
+}
+
+// QR of W1 (first: column pivoting, from U = D = V = 1) or of the prepivoted W1 diag(D[dpt]) -> point
+// `pt`.  Up to N = 512 the first point of a chain is prepivoted like the others: the product of
+// nwrap slices is the best scaled one of the chain, and column pivoting streams the trailing matrix once
+// per column (10 ms for 256 chains of N = 256 against 2.4 ms of the prepivoted form).
 static void udv_step(sh_ctx *ctx, bool first, int pt, int dpt)
 {
     if (first) {
@@ -313,7 +332,7 @@ static void udv_step(sh_ctx *ctx, bool first, int pt, int dpt)
             Tic t(ctx, T_FORMQ);
             if (blocked(ctx)) {
                 hipLaunchKernelGGL(k_tfactors, dim3(ctx->nch), dim3(BLK_NT), lds_blk(ctx), ctx->st, ctx->dc, M_W1);
-                hipLaunchKernelGGL(k_formq_blk, dim3(ctx->nch), dim3(BLK_NT), lds_blk(ctx), ctx->st, ctx->dc, M_W1, pt);
+                formq(ctx, M_W1, pt);
             } else {
                 hipLaunchKernelGGL(k_formq, dim3(ctx->nch), dim3(1024), (size_t)ctx->nmax * sizeof(cplx), ctx->st,
                                    ctx->dc, M_W1, pt);
@@ -326,15 +345,18 @@ static void udv_step(sh_ctx *ctx, bool first, int pt, int dpt)
     {
         Tic t(ctx, T_QR);
         hipLaunchKernelGGL(k_prepivot, dim3(ctx->nch), dim3(1024), (size_t)ctx->nmax * 12, ctx->st, ctx->dc, dpt);
-        if (blocked(ctx))
-            hipLaunchKernelGGL(k_qr_blk, dim3(ctx->nch), dim3(BLK_NT), lds_blk(ctx), ctx->st, ctx->dc, M_W2, pt);
-        else
+        if (blocked(ctx)) {
+            const int np = (ctx->nmax + FPB - 1) / FPB, nw = fac_waves(ctx);
+            for (int k = 0; k < np; k++)
+                hipLaunchKernelGGL(nw == 4 ? k_qr_step<4> : k_qr_step<8>, dim3(ctx->nch, np - k), dim3(64 * nw), 0, ctx->st,
+                                   ctx->dc, (int)M_W2, k, pt);
+        } else
             launch_qr(ctx, M_W2, 0, pt);
     }
     {
         Tic t(ctx, T_FORMQ);
         if (blocked(ctx))
-            hipLaunchKernelGGL(k_formq_blk, dim3(ctx->nch), dim3(BLK_NT), lds_blk(ctx), ctx->st, ctx->dc, M_W2, pt);
+            formq(ctx, M_W2, pt);
         else
             hipLaunchKernelGGL(k_formq, dim3(ctx->nch), dim3(1024), (size_t)ctx->nmax * sizeof(cplx), ctx->st,
                                ctx->dc, M_W2, pt);
@@ -429,7 +451,7 @@ static void stablize_0b(sh_ctx *ctx, int n)
         else
             left_pass(ctx, M_W1, 0, 0, 1 | 2 | 4, 0, ws1, ws2, +1);
     }
-    udv_step(ctx, n == 1, n, n - 1);
+    udv_step(ctx, n == 1 && !blocked(ctx), n, n - 1);
 }
 
 // dqmc_ft_stablize_b0_qr(n): point n-1 of the left chain from point n
@@ -445,7 +467,7 @@ static void stablize_b0(sh_ctx *ctx, int n)
         else
             left_pass(ctx, M_W1, 0, 0, 1 | 2 | 4, 2, ws2, ws1, -1);
     }
-    udv_step(ctx, n == ctx->nst, n - 1, n);
+    udv_step(ctx, n == ctx->nst && !blocked(ctx), n - 1, n);
 }
 
 // green_equaltime into Gs + scratch logweight (rsaved/lsaved select the saved chain point)
@@ -773,10 +795,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
             {(const void *)k_cb_rows, lds_rows(ctx)}, {(const void *)k_cb_cols, lds_cols(ctx)},
             {(const void *)k_fft_rows, lds_fft(ctx)}, {(const void *)k_fft_cols, lds_fft(ctx)},
             {(const void *)k_vupdate_submatrix, (size_t)(SH_KMAX * (SH_KMAX + 1) + 8 * SH_KMAX) * sizeof(cplx)},
-            {(const void *)k_qr_blk, blocked(ctx) ? lds_blk(ctx) : 0},
-            {(const void *)k_formq_blk, blocked(ctx) ? lds_blk(ctx) : 0},
-            {(const void *)k_tfactors, blocked(ctx) ? lds_blk(ctx) : 0},
-            {(const void *)k_lu_blk, blocked(ctx) ? lds_blk(ctx) : 0}};
+            {(const void *)k_tfactors, blocked(ctx) ? lds_blk(ctx) : 0}};
         for (auto &b : big) {
             if (b.bytes <= 64 * 1024 || b.bytes > 150 * 1024) continue;
             hipFuncAttributes fa;
@@ -852,7 +871,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         c.avec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX); c.bvec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX);
         c.updt = dalloc<cplx>(ctx, (size_t)UB * UB); c.updp = dalloc<int32_t>(ctx, UB + 1);
         c.tau = dalloc<cplx>(ctx, n); c.jpvt = dalloc<int32_t>(ctx, n); c.piv = dalloc<int32_t>(ctx, n);
-        c.lperm = dalloc<int32_t>(ctx, n);
+        c.lperm = dalloc<int32_t>(ctx, n); c.lup = dalloc<int32_t>(ctx, (size_t)((n + FPB - 1) / FPB) * FLMAX);
         c.wk = dalloc<cplx>(ctx, (size_t)PB * n);
         c.tblk = dalloc<cplx>(ctx, (size_t)(n / PB + 1) * PB * PB);
         c.rwork = dalloc<double>(ctx, 4 * (size_t)n);
@@ -867,7 +886,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         c.stag = dupload<double>(ctx, q.stag, n);
         c.sc = dalloc<double>(ctx, SC_SIZE);
         if (!c.G || !c.Gs || !c.W1 || !c.W2 || !c.W3 || !c.W4 || !c.Us || !c.Vs || !c.U || !c.V || !c.D || !c.Ds ||
-            !c.ldq || !c.avec || !c.bvec || !c.updt || !c.updp || !c.tau || !c.jpvt || !c.piv || !c.rwork || !c.conf || !c.unif || !c.wk || !c.tblk ||
+            !c.ldq || !c.avec || !c.bvec || !c.updt || !c.updp || !c.tau || !c.jpvt || !c.piv || !c.lperm || !c.lup || !c.rwork || !c.conf || !c.unif || !c.wk || !c.tblk ||
             !c.rng || !c.bonds || !c.kt || !c.ktm1 || !c.stag || !c.sc) {
             int rc = fail(ctx, SH_E_HIP, "device allocation failed");
             sh_destroy(ctx);
@@ -890,6 +909,12 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         sc0[SC_PHASE] = 1.0;
         hipMemcpy(c.sc, sc0, sizeof(sc0), hipMemcpyHostToDevice);
         seeds[ci] = q.seed;
+    }
+    // launch k of the LU: the column blocks from panel k on, or every block of a chain that ends there
+    ctx->lu_blocks.assign((ctx->nmax + FPB - 1) / FPB + 1, 0);
+    for (const auto &c : ctx->hc) {
+        const int np = (c.n + FPB - 1) / FPB;
+        for (int k = 0; k <= np; k++) ctx->lu_blocks[k] = std::max(ctx->lu_blocks[k], k < np ? np - k : np);
     }
     ctx->lwrapv = ctx->hc[0].lwrapv;
     ctx->lwrapp = ctx->hc[0].lwrapp;

@@ -88,6 +88,7 @@ struct DChain {
     cplx *tblk;           // (n/16 + 1) triangular 16 x 16 factors of the block reflectors
     int32_t *jpvt, *piv;  // n
     int32_t *lperm;       // n: row order of the LU's interchanges (row i of P X is row lperm[i] of X)
+    int32_t *lup;         // 512 per panel: the interchanges of the LU's panels as maps of the rows (k_lu_step)
     double *rwork;        // 4n
     int32_t *conf;        // ltrot*n
     double *unif;         // 2*n*ltrot
@@ -246,6 +247,14 @@ __device__ __forceinline__ void wave_argmax_dpp(double &v, int &idx)
     take(swap32_d(v), swap32_i(idx));
 }
 
+// tile and K chunk of the batched ZGEMMs
+#define GT 64
+#define GK 16
+__device__ __forceinline__ double4_t mfma(double a, double b, double4_t c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
 __device__ __forceinline__ cplx *chain_mat(const DChain &c, int sel, int pt)
 {
     size_t nn = (size_t)c.n * c.n;
@@ -270,3 +279,69 @@ __device__ __forceinline__ cplx *chain_mat(const DChain &c, int sel, int pt)
     }
     return nullptr;
 }
+
+// Global <-> LDS staging with ST_BATCH independent 16-byte accesses in flight per thread: a
+// batch's loads are all issued before its first LDS store, so a workgroup waits for one memory
+// latency per batch instead of one per element.  ld(e) returns element e of the tile, st(e, v)
+// writes it back.
+#define ST_BATCH 8
+template <int B, class Ld, class Ix>
+__device__ __forceinline__ void stage_in_map(cplx *lds, int total, Ld ld, Ix ix)
+{
+    for (int base = threadIdx.x; base < total; base += B * blockDim.x) {
+        cplx v[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            const int e = base + u * (int)blockDim.x;
+            v[u] = e < total ? ld(e) : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            const int e = base + u * (int)blockDim.x;
+            if (e < total) lds[ix(e)] = v[u];
+        }
+    }
+}
+
+template <class Ld>
+__device__ __forceinline__ void stage_in(cplx *lds, int total, Ld ld)
+{
+    stage_in_map<ST_BATCH>(lds, total, ld, [](int e) { return e; });
+}
+
+template <class St>
+__device__ __forceinline__ void stage_out(const cplx *lds, int total, St st)
+{
+    for (int base = threadIdx.x; base < total; base += ST_BATCH * blockDim.x) {
+        cplx v[ST_BATCH];
+#pragma unroll
+        for (int u = 0; u < ST_BATCH; u++) {
+            const int e = base + u * (int)blockDim.x;
+            v[u] = e < total ? lds[e] : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int u = 0; u < ST_BATCH; u++) {
+            const int e = base + u * (int)blockDim.x;
+            if (e < total) st(e, v[u]);
+        }
+    }
+}
+
+__device__ __forceinline__ cplx vtab(const DChain &c, int vsel, int is)
+{
+    // vsel 0: bmat, 1: bmat_inv, 2: conj(bmat)
+    cplx b = (vsel == 1) ? c.bmat_inv[is - 1] : c.bmat[is - 1];
+    if (vsel == 2) b.y = -b.y;
+    return b;
+}
+
+// the four factors of the HS components, staged in LDS once per pass (a register table indexed by
+// the component is lowered to a private-memory lookup)
+__device__ __forceinline__ const cplx *vtab_lds(const DChain &c, int vsel)
+{
+    __shared__ cplx vt[4];
+    if (threadIdx.x < 4) vt[threadIdx.x] = vtab(c, vsel, threadIdx.x + 1);
+    __syncthreads();
+    return vt;
+}
+

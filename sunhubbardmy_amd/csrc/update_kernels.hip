@@ -20,10 +20,8 @@
 // chip.  Per slice: one N = 288 chain 1.72 -> 0.27 ms, 72 chains of N = 64, 144, 256 0.90 -> 0.29 ms,
 // 256 chains of N = 256 1.20 -> 0.95 ms (per block 40 us of decisions, 55 us of panels, 140 us of
 // flush; one read and write of the 256 MiB of G takes 111 us), 16 chains of N = 64 172 -> 31 us.
-#include "sunhip_kernels.h"
+#include "update_kernels.h"
 #include <type_traits>
-
-#define UB 64
 
 // lane l's value as a wave-uniform one; l must be wave-uniform
 __device__ __forceinline__ double lane_d(double v, int l)
@@ -281,6 +279,7 @@ k_upd_sites(const DChain *chains, int nt, int slice_in_pass, int s0)
     }
 }
 
+#if !UPD_WHOLE && UPD_NF == 0
 // acc += la(i, k) lb(k, j) over k < kk on one 64 x 64 tile, the MFMA layout and LDS staging of
 // zgemm_tile; la and lb return zero outside the operands.  K chunks of 16, the next chunk's
 // operands in registers while the current one's MFMAs run.
@@ -438,3 +437,11 @@ k_upd_flush(const DChain *chains, int nch, int nt, int s0)
                     gst_nt(G + ((size_t)row + (size_t)col * n), make_double2(accr[sm][sn][r], acci[sm][sn][r]));
             }
 }
+
+#endif
+
+// one object file per (WHOLE, NF) pair, so that they compile side by side
+template __global__ void k_upd_sites<1, UPD_WHOLE, UPD_NF>(const DChain *, int, int, int);
+template __global__ void k_upd_sites<2, UPD_WHOLE, UPD_NF>(const DChain *, int, int, int);
+template __global__ void k_upd_sites<3, UPD_WHOLE, UPD_NF>(const DChain *, int, int, int);
+template __global__ void k_upd_sites<4, UPD_WHOLE, UPD_NF>(const DChain *, int, int, int);
