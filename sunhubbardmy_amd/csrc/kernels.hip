@@ -1,7 +1,7 @@
 // kernels.hip -- CDNA4 (gfx950) kernels of the DQMC sweep.  Every kernel is batched over
 // independent Markov chains: blockIdx.z (GEMM, elementwise) or blockIdx.x (one workgroup per
 // chain) selects the chain, whose matrix dimension may differ from its neighbours'.
-#include "sunhip_kernels.h"
+#include "gemm_small.h"
 
 #define FULL_DBL 1
 
@@ -407,6 +407,24 @@ __device__ __forceinline__ void zgemm_tile(const cplx *A_, int lda, const cplx *
                     gst(C + (o), make_double2(outr, outi));
                 }
             }
+}
+
+// whether a launch takes the 32 x 32 form: its 64 x 64 tiles would not give every CU one.  (At few tiles a
+// product's time is that of one tile, 56 us at K = 288 against 18; with a tile for every CU the large
+// form's reuse of operands counts: at 288 tiles of K = 64 they are level.)
+__host__ inline bool gemm_small(int m, int n, int nch) { return (size_t)((m + GT - 1) / GT) * ((n + GT - 1) / GT) * nch < 256; }
+
+template <int OPA, int OPB>
+__global__ void __launch_bounds__(256, 2)
+k_zgemm_small(const DChain *chains, int selA, int ptA, int selB, int ptB, int selC, int ptC,
+              double ar, double ai, double br, double bi)
+{
+    const DChain &c = chains[blockIdx.z];
+    const int n = c.n;
+    const int tm = blockIdx.x * GS, tn = blockIdx.y * GS;
+    if (tm >= n || tn >= n) return;
+    zgemm_small<OPA, OPB>(chain_mat(c, selA, ptA), n, chain_mat(c, selB, ptB), n, chain_mat(c, selC, ptC), n, n, n, n,
+                          tm, tn, ar, ai, br, bi);
 }
 
 template <int OPA, int OPB>

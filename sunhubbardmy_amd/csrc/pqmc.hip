@@ -33,6 +33,10 @@ void pgemm(shp_ctx *ctx, int sa, int pa, int sb, int pb_, int sc, int pc, int m,
            int ldc, double ar = 1.0, double br = 0.0)
 {
     PGemm g{sa, pa, sb, pb_, sc, pc, m, n, k, lda, ldb, ldc, ar, 0.0, br, 0.0};
+    if (gemm_small(m, n, ctx->nch)) {
+        hipLaunchKernelGGL(kp_gemm_small, dim3((m + GS - 1) / GS, (n + GS - 1) / GS, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, g);
+        return;
+    }
     dim3 grid((m + GT - 1) / GT, (n + GT - 1) / GT, ctx->nch);
     hipLaunchKernelGGL(kp_gemm, grid, dim3(256), 0, ctx->st, ctx->dc, g);
 }

@@ -94,6 +94,16 @@ kp_gemm(const PChain *chains, PGemm g)
                      g.k, tm, tn, g.ar, g.ai, g.br, g.bi);
 }
 
+extern "C" __global__ void __launch_bounds__(256, 2)
+kp_gemm_small(const PChain *chains, PGemm g)
+{
+    const PChain &c = chains[blockIdx.z];
+    const int tm = blockIdx.x * GS, tn = blockIdx.y * GS;
+    if (tm >= g.m || tn >= g.n) return;
+    zgemm_small<0, 0>(pmat(c, g.sa, g.pa), g.lda, pmat(c, g.sb, g.pb), g.ldb, pmat(c, g.sc, g.pc), g.ldc, g.m, g.n,
+                      g.k, tm, tn, g.ar, g.ai, g.br, g.bi);
+}
+
 // ---- copies -------------------------------------------------------------------------------
 // dst[e] = src[e] (or conj) for e < count
 extern "C" __global__ void __launch_bounds__(256)
