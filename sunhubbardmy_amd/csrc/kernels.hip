@@ -445,50 +445,6 @@ template __global__ void k_zgemm<1, 0>(const DChain *, int, int, int, int, int, 
 template __global__ void k_zgemm<0, 1>(const DChain *, int, int, int, int, int, int, double, double, double, double);
 
 // ------------------------------------------------------------------------------------------
-// Workgroup-level rank-k update on MFMA: G(n x n) = (G + A B^T) diag(cs) with A, B n x k
-// column-major (leading dimension n).  Used by the bond field's delay flush (cs = 1) and submatrix flush.
-// Computed as G^T tiles so that every global access is a 16-element column run.
-// ------------------------------------------------------------------------------------------
-__device__ static void wg_rank_k(cplx *G, int n, const cplx *A, const cplx *B, int k, const double *csr,
-                                 const double *csi)
-{
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    const int nt = (n + 15) >> 4;
-    const int l16 = lane & 15, kq = lane >> 4;
-    for (int tile = w; tile < nt * nt; tile += nw) {
-        const int i0 = (tile % nt) * 16, j0 = (tile / nt) * 16;
-        // accumulator = G^T tile: element (p, q) = G[i0+q][j0+p], lane holds p = l/16 + 4r, q = l%16
-        double4_t accr, acci;
-        const int row = i0 + l16;
-        for (int r = 0; r < 4; r++) {
-            int col = j0 + kq + 4 * r;
-            cplx g = (row < n && col < n) ? G[(size_t)row + (size_t)col * n] : make_double2(0.0, 0.0);
-            accr[r] = g.x; acci[r] = g.y;
-        }
-        for (int m0 = 0; m0 < k; m0 += 4) {
-            const int m = m0 + kq;
-            cplx x = make_double2(0.0, 0.0), y = make_double2(0.0, 0.0);
-            if (m < k) {
-                if (j0 + l16 < n) x = B[(size_t)(j0 + l16) + (size_t)m * n];   // X[p][m] = B[j0+p][m]
-                if (i0 + l16 < n) y = A[(size_t)(i0 + l16) + (size_t)m * n];   // Y[m][q] = A[i0+q][m]
-            }
-            accr = mfma(x.x, y.x, accr);
-            accr = mfma(-x.y, y.y, accr);
-            acci = mfma(x.x, y.y, acci);
-            acci = mfma(x.y, y.x, acci);
-        }
-        for (int r = 0; r < 4; r++) {
-            int col = j0 + kq + 4 * r;
-            if (row < n && col < n) {
-                cplx v = make_double2(accr[r], acci[r]);
-                if (csr) v = cmul(v, make_double2(csr[col], csi[col]));
-                G[(size_t)row + (size_t)col * n] = v;
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------------------------------
 // Equal-time measurement (src/dqmc_measure/equaltime_measure.f90:1-69, zkint :71-114,
 // zint_u :116-125, zspsm :283-299 -> Fourier component at the staggering vector).
 // One workgroup per chain; the G(i,j) G(j,i) sum is taken over 32x32 tile pairs staged in LDS.

@@ -137,16 +137,7 @@ void update_family_g(shp_ctx *ctx, int nt, int nf, size_t uoff0)
     hipLaunchKernelGGL(kp_v_save, dim3((nl + 255) / 256, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nt, nf);
     const int slice = (int)(uoff0 / ctx->slice_draws);
     const int p = (int)((uoff0 % ctx->slice_draws) / (2 * (size_t)nl));
-    if (ctx->update == SHP_U_DELAY) {
-        hipLaunchKernelGGL(k_vupdate_delay, dim3(ctx->nch), dim3(256), (size_t)4 * 64 * sizeof(cplx), ctx->st,
-                           ctx->dview, nt, nf, slice, p);
-    } else if (ctx->update == SHP_U_SUBMATRIX_G) {
-        const int K = std::max(2, ctx->gblock & ~1);
-        hipLaunchKernelGGL(k_vupdate_submatrix, dim3(ctx->nch), dim3(256), (size_t)(K * (K + 1) + 8 * K) * sizeof(cplx),
-                           ctx->st, ctx->dview, nt, nf, slice, p);
-    } else
-        hipLaunchKernelGGL(k_vupdate, dim3(ctx->nch), dim3(256), (size_t)4 * ctx->n * sizeof(cplx), ctx->st,
-                           ctx->dview, nt, nf, slice, p);
+    bond_update(ctx->st, ctx->dview, ctx->nch, ctx->n, nl, nt, nf, slice, p);
     hipLaunchKernelGGL(kp_v_rescale, dim3((unsigned)(((size_t)nl * ctx->ne + 255) / 256), 1, ctx->nch), dim3(256), 0,
                        ctx->st, ctx->dc, nt, nf);
     inverse(ctx, P_UL, P_UR, P_ULRINV, -1);
@@ -579,18 +570,6 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
                 shp_destroy(ctx);
                 return rc;
             }
-        }
-    }
-    if (ctx->update == SHP_U_SUBMATRIX_G) {
-        const int Kb = std::max(2, ctx->gblock & ~1);
-        const size_t ldsv = (size_t)(Kb * (Kb + 1) + 8 * Kb) * sizeof(cplx);
-        if (ldsv > 64 * 1024 &&
-            hipFuncSetAttribute((const void *)k_vupdate_submatrix, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsv) !=
-                hipSuccess) {
-            (void)hipGetLastError();
-            int rc = fail(ctx, SH_E_HIP, "dynamic LDS request above the device limit");
-            shp_destroy(ctx);
-            return rc;
         }
     }
     ctx->dc = dupload<PChain>(ctx, ctx->hc.data(), nchains);

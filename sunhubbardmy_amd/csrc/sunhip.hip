@@ -71,7 +71,6 @@ struct sh_ctx : ctx_base {
     DChain *dc = nullptr;
     int32_t *d_seeds = nullptr;
     bool started = false;
-    bool legacy_update = false;   // test hook: the fast form of the bond update whatever the build's
     int ntdm = -1;                // time-displaced measurement: bins 0 .. ntdm, -1 = off
     size_t eqt_lds = 0;           // LDS of k_eqt, 0 while no chain has correlation bins
     int lwrapv = 0;               // the batch carries the t-V bond field
@@ -382,26 +381,24 @@ static void vprop(sh_ctx *ctx, int sel, int nf, int mode, int side, int nt)
     const unsigned nb = (unsigned)(((size_t)ctx->nmax * ctx->nmax / 2 + 255) / 256);   // n nn_lf <= n^2 / 2
     hipLaunchKernelGGL(k_vprop, dim3(nb, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, sel, 0, nf, mode, side, nt);
 }
-// the bond update follows the build's algorithm as the on-site one does: the delay form
-// (dqmc_config_v/dqmc_update_delay.f90) or the submatrix form (dqmc_update_submatrix.f90) with
-// the build's depth, else the fast form (dqmc_update.f90)
+// the bond update of family nf (update_kernels.hip), for the chains of either sweep: three launches per
+// block of at most UB / 2 bonds, the blocks as even as they come.  nl: the largest chain's bonds per family
+static void bond_update(hipStream_t st, const DChain *dc, int nch, int nmax, int nl, int nt, int nf, int slice, int p)
+{
+    const int nblk = (nl + UB / 2 - 1) / (UB / 2), per = (nl + nblk - 1) / nblk, tiles = (2 * per + 15) / 16;
+    const int ntl = (nmax + GT - 1) / GT, nch8 = (nch + 7) / 8 * 8;
+    auto k = tiles == 1 ? k_upd_bonds<1> : tiles == 2 ? k_upd_bonds<2> : tiles == 3 ? k_upd_bonds<3> : k_upd_bonds<4>;
+    for (int ib0 = 0; ib0 < nl; ib0 += per) {
+        hipLaunchKernelGGL(k, dim3(nch), dim3(64 * tiles), 0, st, dc, nt, nf, slice, p, ib0, per);
+        hipLaunchKernelGGL(k_upd_panel, dim3(ntl, 1, nch), dim3(256), 0, st, dc, 0);
+        hipLaunchKernelGGL(k_upd_flush, dim3(nch8 * ntl * ntl), dim3(256), 0, st, dc, nch, ntl, 0);
+    }
+}
 static void vupdate(sh_ctx *ctx, int nt, int nf, int slice, int p)
 {
-    int kmax = 0;
-    for (auto &c : ctx->hc) kmax = std::max(kmax, c.nublock);
-    if (ctx->update == SH_U_DELAY && kmax >= 2 && !ctx->legacy_update) {
-        hipLaunchKernelGGL(k_vupdate_delay, dim3(ctx->nch), dim3(256), (size_t)4 * SH_KMAX * sizeof(cplx), ctx->st,
-                           ctx->dc, nt, nf, slice, p);
-        return;
-    }
-    if (ctx->update == SH_U_SUBMATRIX && !ctx->legacy_update) {
-        const int K = std::max(2, std::min(kmax, SH_KMAX) & ~1);
-        hipLaunchKernelGGL(k_vupdate_submatrix, dim3(ctx->nch), dim3(256), (size_t)(K * (K + 1) + 8 * K) * sizeof(cplx),
-                           ctx->st, ctx->dc, nt, nf, slice, p);
-        return;
-    }
-    hipLaunchKernelGGL(k_vupdate, dim3(ctx->nch), dim3(256), (size_t)4 * ctx->nmax * sizeof(cplx), ctx->st, ctx->dc,
-                       nt, nf, slice, p);
+    int nl = 0;
+    for (auto &c : ctx->hc) nl = std::max(nl, c.nn_lf);
+    bond_update(ctx->st, ctx->dc, ctx->nch, ctx->nmax, nl, nt, nf, slice, p);
 }
 // every plaquette of slice nt on a chain matrix: rows (side 0) or columns (side 1), the factors
 // exp(i a eta V) (inv 0) or their inverses (inv 1), plaquettes 1..lqp (rev 0) or lqp..1 (rev 1)
@@ -800,7 +797,6 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         struct { const void *f; size_t bytes; } big[] = {
             {(const void *)k_cb_rows, lds_rows(ctx)}, {(const void *)k_cb_cols, lds_cols(ctx)},
             {(const void *)k_fft_rows, lds_fft(ctx)}, {(const void *)k_fft_cols, lds_fft(ctx)},
-            {(const void *)k_vupdate_submatrix, (size_t)(SH_KMAX * (SH_KMAX + 1) + 8 * SH_KMAX) * sizeof(cplx)},
             {(const void *)k_tfactors, blocked(ctx) ? lds_blk(ctx) : 0}};
         for (auto &b : big) {
             if (b.bytes <= 64 * 1024 || b.bytes > 150 * 1024) continue;
@@ -1829,7 +1825,7 @@ extern "C" int sh_dbg_op(sh_ctx *ctx, int op, const int *a)
         break;
     case 12: measure(ctx); break;
     case 13: wrap_replace(ctx, a[0]); break;
-    case 14: ctx->legacy_update = a[0] != 0; ctx->graph_epoch++; break;
+    case 14: break;   // one form of the bond update serves every build
     default: return SH_E_ARG;
     }
     int rc = check_launch(ctx);

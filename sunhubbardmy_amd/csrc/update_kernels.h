@@ -1,9 +1,10 @@
 // update_kernels.h -- the kernels of update_kernels.hip, a translation unit of its own.
 #pragma once
-#include "sunhip_kernels.h"
+#include "exchange.h"
 
-#define UB 64   // sites of a block
 template <int NT, bool WHOLE, int NF>
 __global__ void k_upd_sites(const DChain *chains, int nt, int slice_in_pass, int s0);
+template <int NT>
+__global__ void k_upd_bonds(const DChain *chains, int nt, int nf, int slice, int p, int ib0, int per);
 extern "C" __global__ void k_upd_panel(const DChain *chains, int s0);
 extern "C" __global__ void k_upd_flush(const DChain *chains, int nch, int nt, int s0);
