@@ -24,8 +24,8 @@ def hipcc():
 
 
 # translation units, compiled side by side: source and its own definitions
-UNITS = [("sunhip.hip", []), ("fft_kernels.hip", []), ("factor.hip", [])] + [("update_kernels.hip", ["-DUPD_WHOLE=%d" % w, "-DUPD_NF=%d" % f])
-                                for w in (0, 1) for f in (0, 2)]
+UNITS = [("sunhip.hip", []), ("fft_kernels.hip", []), ("factor.hip", []), ("stock_kernels.hip", [])] + [
+    ("update_kernels.hip", ["-DUPD_WHOLE=%d" % w, "-DUPD_NF=%d" % f]) for w in (0, 1) for f in (0, 2)]
 
 
 def build(verbose=False):

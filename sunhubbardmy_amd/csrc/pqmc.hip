@@ -9,7 +9,7 @@ struct shp_ctx : ctx_base {
     int nch = 0, n = 0, ne = 0, ltrot = 0, nwrap = 0, nst = 0, kmode = 0, ns = 0, mid_len = 1;
     int nn_nf = 0, nn_lf = 0, wrap_check = 1, pb = PB;
     int update = SHP_U_LR, gblock = 0;   // update algorithm of the on-site field and its depth
-    bool lwrapu = false, lwrapv = true;
+    bool lwrapu = false, lwrapv = true, flav2 = true;   // flav2: nflr = 2 in every chain
     size_t slice_draws = 0;       // uniforms per slice of a pass
     bool tracing = false, started = false;
     std::vector<int> iwrap_nt, wrap_step;
@@ -25,7 +25,6 @@ struct shp_ctx : ctx_base {
 namespace {
 
 size_t p_lds_prop(const shp_ctx *c) { return (size_t)cb_ldr(c->n) * std::max(CPB, RPB) * sizeof(cplx); }
-size_t p_lds_bonds(const shp_ctx *c) { return (size_t)2 * c->ns * c->ns * sizeof(cplx); }
 size_t p_lds_qr(const shp_ctx *c) { return ((size_t)c->n * c->pb + 2 * PB * PB) * sizeof(cplx); }
 size_t p_lds_lu(const shp_ctx *c) { return (size_t)c->ne * PB * sizeof(cplx) + (size_t)c->ne * sizeof(int); }
 
@@ -143,8 +142,33 @@ void update_family_g(shp_ctx *ctx, int nt, int nf, size_t uoff0)
     inverse(ctx, P_UL, P_UR, P_ULRINV, -1);
 }
 
-// ---- submatrix-LR update of family nf at slice nt (the fast form: stocks of one bond), or a
-// G-based form; uoff = its first uniform in the pass ----
+// ---- one stock of the submatrix-LR update at slice nt (stock_kernels.hip): bonds ib0 .. of family nf, or
+// with nf < 0 the on-site field's sites from ib0, nup sites in all; uoff = its first uniform in the pass ----
+template <int NT>
+void stock_decide(shp_ctx *ctx, int nt, int nf, int ib0, int nup, size_t uoff)
+{
+    const dim3 grid(ctx->nch), block(64 * NT);
+    if (nf >= 0)
+        hipLaunchKernelGGL(kp_stock_bonds<NT>, grid, block, 0, ctx->st, ctx->dc, nt, nf, ib0, nup / 2, (int)uoff);
+    else if (ctx->flav2)
+        hipLaunchKernelGGL((kp_stock_sites<NT, 2>), grid, block, 0, ctx->st, ctx->dc, nt, ib0, nup, uoff);
+    else
+        hipLaunchKernelGGL((kp_stock_sites<NT, 0>), grid, block, 0, ctx->st, ctx->dc, nt, ib0, nup, uoff);
+}
+
+void stock(shp_ctx *ctx, int nt, int nf, int ib0, int nup, size_t uoff)
+{
+    const int te = (ctx->ne + GS - 1) / GS, rt = (nup + GS - 1) / GS, tiles = (nup + 15) / 16;
+    hipLaunchKernelGGL(kp_stock_pre, dim3(te, 2 * rt, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nf, ib0, nup, rt);
+    hipLaunchKernelGGL(kp_stock_f, dim3(rt, rt, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nf, ib0, nup);
+    (tiles == 1 ? stock_decide<1> : tiles == 2 ? stock_decide<2> : tiles == 3 ? stock_decide<3> : stock_decide<4>)(
+        ctx, nt, nf, ib0, nup, uoff);
+    hipLaunchKernelGGL(kp_stock_vtmp, dim3(te, rt + 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nup, rt);
+    hipLaunchKernelGGL(kp_stock_flush, dim3(te, te, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nup);
+}
+
+// ---- update of family nf at slice nt: submatrix-LR in stocks of ns / 2 bonds (the fast form: one bond), or
+// a G-based form; uoff = its first uniform in the pass ----
 void update_family(shp_ctx *ctx, int nt, int nf, size_t uoff0)
 {
     if (ctx->update == SHP_U_DELAY || ctx->update == SHP_U_SUBMATRIX_G) {
@@ -152,26 +176,8 @@ void update_family(shp_ctx *ctx, int nt, int nf, size_t uoff0)
         return;
     }
     Tic t(ctx, T_UPDATE);
-    const int ns = ctx->ns, ne = ctx->ne, nl = ctx->nn_lf;
-    const int per = ctx->update == SHP_U_FAST ? 1 : ns / 2;
-    for (int ib0 = 0; ib0 < nl; ib0 += per) {
-        const int nb = std::min(per, nl - ib0), nup = 2 * nb;
-        const int cnt = std::max(ns * ne, ns * ns);
-        hipLaunchKernelGGL(kp_stock_gather, dim3((cnt + 255) / 256, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc,
-                           nf, ib0, nup);
-        // Rrows = urP ULRINV, Felms = Rrows ulP (:121-133)
-        pgemm(ctx, P_URP, 0, P_ULRINV, 0, P_RROWS, 0, nup, ne, ne, ns, ne, ns);
-        pgemm(ctx, P_RROWS, 0, P_ULP, 0, P_FELMS, 0, nup, nup, ne, ns, ne, ns);
-        const int uoff = (int)(uoff0 + 2 * (size_t)ib0);
-        hipLaunchKernelGGL(kp_stock_bonds, dim3(ctx->nch), dim3(256), p_lds_bonds(ctx), ctx->st, ctx->dc, nt, nf, ib0,
-                           nb, uoff);
-        // Woodbury flush ULRINV -= (ULRINV Umat)(Gamma^-1 Vmat) over the whole stock width; rows
-        // and columns past the accepted count are zero (:240-266)
-        pgemm(ctx, P_GINV, 0, P_VMAT, 0, P_VTMP, 0, ns, ne, ns, ns, ns, ns);
-        pgemm(ctx, P_ULRINV, 0, P_UMAT, 0, P_UTMP, 0, ne, ns, ne, ne, ne, ne);
-        pgemm(ctx, P_UTMP, 0, P_VTMP, 0, P_ULRINV, 0, ne, ne, ns, ne, ns, ne, -1.0, 1.0);
-        hipLaunchKernelGGL(kp_stock_scale, dim3((ns * ne + 255) / 256, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc);
-    }
+    const int nl = ctx->nn_lf, per = ctx->update == SHP_U_FAST ? 1 : ctx->ns / 2;
+    for (int ib0 = 0; ib0 < nl; ib0 += per) stock(ctx, nt, nf, ib0, 2 * std::min(per, nl - ib0), uoff0 + 2 * (size_t)ib0);
 }
 
 // the G-based forms (dqmc_proj_update_delay.f90, dqmc_proj_update_submatrix_G.f90): G from the
@@ -200,23 +206,9 @@ void update_u(shp_ctx *ctx, int nt, size_t uoff0)
         return;
     }
     Tic t(ctx, T_UPDATE);
-    const int ns = ctx->ns, ne = ctx->ne, n = ctx->n;
     // the fast update is the same algebra one site at a time: stocks of one site
-    const int step = ctx->update == SHP_U_FAST ? 1 : ns;
-    for (int i0 = 0; i0 < n; i0 += step) {
-        const int nup = std::min(step, n - i0);
-        const int cnt = std::max(ns * ne, ns * ns);
-        hipLaunchKernelGGL(kp_stock_gather, dim3((cnt + 255) / 256, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc,
-                           -1, i0, nup);
-        pgemm(ctx, P_URP, 0, P_ULRINV, 0, P_RROWS, 0, nup, ne, ne, ns, ne, ns);
-        pgemm(ctx, P_RROWS, 0, P_ULP, 0, P_FELMS, 0, nup, nup, ne, ns, ne, ns);
-        hipLaunchKernelGGL(kp_stock_sites, dim3(ctx->nch), dim3(256), p_lds_bonds(ctx), ctx->st, ctx->dc, nt, i0, nup,
-                           uoff0 + 2 * (size_t)i0);
-        pgemm(ctx, P_GINV, 0, P_VMAT, 0, P_VTMP, 0, ns, ne, ns, ns, ns, ns);
-        pgemm(ctx, P_ULRINV, 0, P_UMAT, 0, P_UTMP, 0, ne, ns, ne, ne, ne, ne);
-        pgemm(ctx, P_UTMP, 0, P_VTMP, 0, P_ULRINV, 0, ne, ne, ns, ne, ns, ne, -1.0, 1.0);
-        hipLaunchKernelGGL(kp_stock_scale, dim3((ns * ne + 255) / 256, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc);
-    }
+    const int step = ctx->update == SHP_U_FAST ? 1 : ctx->ns;
+    for (int i0 = 0; i0 < ctx->n; i0 += step) stock(ctx, nt, -1, i0, std::min(step, ctx->n - i0), uoff0 + 2 * (size_t)i0);
 }
 
 // ---- scratch quantities ---------------------------------------------------------------------
@@ -398,6 +390,7 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
             delete ctx;
             return SH_E_ARG;
         }
+        ctx->flav2 = ctx->flav2 && q.nflr == 2;
         if (q.update != q0.update || q.gblock != q0.gblock || q.update < SHP_U_LR ||
             q.update > SHP_U_SUBMATRIX_G ||
             (q.update >= SHP_U_DELAY && ((q.ubmat != nullptr) == (q.vtab != nullptr) || q.gblock < 1 || q.gblock > 64))) {
@@ -440,8 +433,7 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
     if (hipStreamCreate(&ctx->st) != hipSuccess) { delete ctx; return SH_E_HIP; }
     {
         struct { const void *f; size_t bytes; } big[] = {
-            {(const void *)kp_prop, p_lds_prop(ctx)}, {(const void *)kp_stock_bonds, p_lds_bonds(ctx)},
-            {(const void *)kp_stock_sites, p_lds_bonds(ctx)},
+            {(const void *)kp_prop, p_lds_prop(ctx)},
             {(const void *)kp_qr_formq, p_lds_qr(ctx)}, {(const void *)kp_lu_inv, p_lds_lu(ctx)}};
         for (auto &b : big) {
             if (b.bytes <= 64 * 1024) continue;
@@ -470,16 +462,14 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
         c.INV2 = dalloc<cplx>(ctx, (size_t)ne * ne);
         c.G = dalloc<cplx>(ctx, nn); c.G2 = dalloc<cplx>(ctx, nn);
         c.Ust = dalloc<cplx>(ctx, nne * (q.nst + 1)); c.proj = dalloc<cplx>(ctx, nne);
-        c.urP = dalloc<cplx>(ctx, (size_t)ns * ne); c.ulP = dalloc<cplx>(ctx, (size_t)ns * ne);
         c.Rrows = dalloc<cplx>(ctx, (size_t)ns * ne); c.Felms = dalloc<cplx>(ctx, (size_t)ns * ns);
-        c.Ginv = dalloc<cplx>(ctx, (size_t)ns * ns); c.Vmat = dalloc<cplx>(ctx, (size_t)ns * ne);
-        c.Umat = dalloc<cplx>(ctx, (size_t)ns * ne); c.Vtmp = dalloc<cplx>(ctx, (size_t)ns * ne);
+        c.Ginv = dalloc<cplx>(ctx, (size_t)ns * ns); c.Vtmp = dalloc<cplx>(ctx, (size_t)ns * ne);
         c.Utmp = dalloc<cplx>(ctx, (size_t)ns * ne); c.Dvec = dalloc<cplx>(ctx, ns);
         c.tau = dalloc<cplx>(ctx, ne); c.tblk = dalloc<cplx>(ctx, (size_t)(ne / (PB / 2) + 2) * PB * PB);
         c.wk = dalloc<cplx>(ctx, (size_t)PB * std::max(n, ne));
         c.piv = dalloc<int32_t>(ctx, ne);
         c.conf = dalloc<int32_t>(ctx, (size_t)n * q.nn_nf * q.ltrot);
-        c.xvec = dalloc<int32_t>(ctx, ns); c.svec = dalloc<int32_t>(ctx, ns); c.ikd = dalloc<int32_t>(ctx, 4);
+        c.xvec = dalloc<int32_t>(ctx, ns); c.ikd = dalloc<int32_t>(ctx, 4);
         c.unif = dalloc<double>(ctx, std::max(ctx->slice_draws, (size_t)1) * q.ltrot);
         c.lwrapu = ctx->lwrapu ? 1 : 0;
         c.lwrapv = ctx->lwrapv ? 1 : 0;
@@ -508,9 +498,9 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
         c.ktm1 = dupload<cplx>(ctx, (const cplx *)q.urtm1, kl);
         c.stag = dupload<double>(ctx, q.stag, n);
         if (!c.UR || !c.UL || !c.T1 || !c.T2 || !c.ULo || !c.URo || !c.ULRINV || !c.ULR || !c.INV2 || !c.G || !c.G2 ||
-            !c.Ust || !c.proj || !c.urP || !c.ulP || !c.Rrows || !c.Felms || !c.Ginv || !c.Vmat || !c.Umat ||
+            !c.Ust || !c.proj || !c.Rrows || !c.Felms || !c.Ginv ||
             !c.Vtmp || !c.Utmp || !c.Dvec || !c.tau || !c.tblk || !c.wk || !c.piv || !c.conf || !c.xvec ||
-            !c.svec || !c.ikd || !c.unif || !c.sc || !c.logwDV || !c.rwork || !c.rng || !c.bonds || !c.kt ||
+            !c.ikd || !c.unif || !c.sc || !c.logwDV || !c.rwork || !c.rng || !c.bonds || !c.kt ||
             !c.ktm1 || !c.stag || (ctx->lwrapu && !c.uconf)) {
             int rc = fail(ctx, SH_E_HIP, "device allocation failed");
             shp_destroy(ctx);

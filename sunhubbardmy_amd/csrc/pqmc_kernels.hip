@@ -4,78 +4,7 @@
 // the QR / LU steps of the stabilization.  Every kernel is batched over chains that share N, ne
 // and the stock size; blockIdx.z (elementwise, GEMM) or blockIdx.x (one workgroup per chain)
 // selects the chain.
-#include "sunhip_kernels.h"
-
-// scalar slots of the projective chain beyond the shared layout (SC_PHASE, SC_LOGW, SC_ZLD,
-// SC_INFO, SC_OBS ... keep their meaning)
-// (the projective sweep has no saved chain point, so SC_LDQ_SAVE's first slot holds the angle
-// sum of the on-site field's phases)
-enum { PS_RLOG = 30, PS_ISGN = 31, PS_UANG = SC_LDQ_SAVE };
-
-enum {
-    P_UR = 0, P_UL, P_ULRINV, P_ULR, P_T1, P_T2, P_ULO, P_URO, P_INV2, P_G, P_G2, P_KT, P_KTM1,
-    P_URP, P_ULP, P_RROWS, P_FELMS, P_GINV, P_VMAT, P_UMAT, P_VTMP, P_UTMP, P_UST, P_PROJ
-};
-
-struct PChain {
-    int n, ne, nn_nf, nn_lf, kmode, ns, ltrot, nst, nflr, lq, pb, trace_cap;
-    cplx *UR, *UL, *ULRINV, *ULR, *T1, *T2, *ULo, *URo, *INV2, *G, *G2, *Ust, *proj;
-    cplx *urP, *ulP, *Rrows, *Felms, *Ginv, *Vmat, *Umat, *Vtmp, *Utmp, *Dvec;
-    cplx *tau, *tblk, *wk, *trace;
-    int32_t *piv, *conf, *xvec, *svec, *ikd;
-    double *unif, *sc, *logwDV, *rwork;
-    uint32_t *rng;
-    const int32_t *bonds;
-    const cplx *kt, *ktm1;
-    const double *stag;
-    cplx vt[8];   // (bp, bm, bpi, bmi) for field value 1 then 2
-    cplx vd[4];   // (dp, dm) for field value 1 then 2
-    // the on-site field (src/dqmc_config_u), when lwrapu: conf_u [ltrot][n], values 1..ulcomp
-    int lwrapu, lwrapv, ulcomp, uphase_from_conf;
-    int32_t *uconf;
-    cplx ub[4], ubi[4], ud[12], uratio[12];   // bmat, bmat_inv, delta_bmat(iflip, is), phase_ratio
-    double ug[4], upa[4];                      // gaml, arg of phase(is)
-    // the G-based updates of the on-site field: the slice's field before the update
-    int32_t *uold;
-};
-
-// uniforms of one slice in a pass: 2 per site of the on-site field, 2 per bond of every family
-__host__ __device__ __forceinline__ size_t p_slice_draws(const PChain &c)
-{
-    return (c.lwrapu ? (size_t)2 * c.n : 0) + (c.lwrapv ? (size_t)2 * c.nn_lf * c.nn_nf : 0);
-}
-
-__device__ __forceinline__ cplx *pmat(const PChain &c, int sel, int pt)
-{
-    const size_t nne = (size_t)c.n * c.ne;
-    switch (sel) {
-    case P_UR: return c.UR;
-    case P_UL: return c.UL;
-    case P_ULRINV: return c.ULRINV;
-    case P_ULR: return c.ULR;
-    case P_T1: return c.T1;
-    case P_T2: return c.T2;
-    case P_ULO: return c.ULo;
-    case P_URO: return c.URo;
-    case P_INV2: return c.INV2;
-    case P_G: return c.G;
-    case P_G2: return c.G2;
-    case P_KT: return (cplx *)c.kt;
-    case P_KTM1: return (cplx *)c.ktm1;
-    case P_URP: return c.urP;
-    case P_ULP: return c.ulP;
-    case P_RROWS: return c.Rrows;
-    case P_FELMS: return c.Felms;
-    case P_GINV: return c.Ginv;
-    case P_VMAT: return c.Vmat;
-    case P_UMAT: return c.Umat;
-    case P_VTMP: return c.Vtmp;
-    case P_UTMP: return c.Utmp;
-    case P_UST: return c.Ust + nne * pt;
-    case P_PROJ: return c.proj;
-    }
-    return nullptr;
-}
+#include "pqmc_kernels.h"
 
 // ---- batched ZGEMM with explicit shapes: C = alpha A B + beta C --------------------------
 struct PGemm {
@@ -308,462 +237,6 @@ kp_prop(const PChain *chains, POps ops)
             if (rr < nrow) M[(size_t)(r0 + rr) + (size_t)col * ne] = lds[rr * ldr + col];
         }
     }
-}
-
-// ---- submatrix-LR update (src/dqmc_config_v/dqmc_proj_update_submatrix_LR.f90) -----------
-// stock start: the stock's rows of UR (urP, nup x ne, ld ns) and columns of UL (ulP, ne x
-// nup, ld ne) in bond order (i1, i2 per bond); Gamma^-1, Vmat, Umat and the count cleared
-// nf < 0: the on-site field's stock, the consecutive sites ib0 .. ib0 + nup - 1
-extern "C" __global__ void __launch_bounds__(256)
-kp_stock_gather(const PChain *chains, int nf, int ib0, int nup)
-{
-    const PChain &c = chains[blockIdx.z];
-    const int ns = c.ns, ne = c.ne, n = c.n;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    auto site = [&](int s) {
-        if (nf < 0) return ib0 + s;
-        const int ist = nf * c.nn_lf + ib0 + s / 2;
-        return (int)c.bonds[2 * ist + (s & 1)];
-    };
-    if (e < ns * ne) {
-        const int s = e % ns, l = e / ns;       // urP(s, l)
-        cplx v = make_double2(0.0, 0.0);
-        if (s < nup) v = c.UR[(size_t)site(s) + (size_t)l * n];
-        c.urP[e] = v;
-        c.Vmat[e] = make_double2(0.0, 0.0);
-    }
-    if (e < ne * ns) {
-        const int l = e % ne, s = e / ne;       // ulP(l, s)
-        cplx v = make_double2(0.0, 0.0);
-        if (s < nup) v = c.UL[(size_t)l + (size_t)site(s) * ne];
-        c.ulP[e] = v;
-        c.Umat[e] = make_double2(0.0, 0.0);
-    }
-    if (e < ns * ns) c.Ginv[e] = make_double2(0.0, 0.0);
-    if (e == 0) c.ikd[0] = 0;
-}
-
-// the stock's bonds in order, one workgroup per chain: 2x2 ratio det(I + Vcal D) with
-// Vcal = PFP_kk - PFP_kik Gamma^-1 PFP_ikk (:146-175), Metropolis on Re(ratio phase)/Re(phase),
-// and on acceptance the bordering of Gamma^-1 by one 2x2 block (:176-222).  Felms and Gamma^-1
-// live in LDS (2 ns^2 complex).  The stock's field, acceptance uniforms and bond sites are staged
-// in LDS and the field, xvec and Dvec written back at the end, so that the bond loop itself
-// touches no global memory (a global access there would put a memory round trip on every
-// bond's critical path).
-extern "C" __global__ void __launch_bounds__(256)
-kp_stock_bonds(const PChain *chains, int nt, int nf, int ib0, int nb, int uoff)
-{
-    extern __shared__ cplx bsh[];
-    const PChain &c = chains[blockIdx.x];
-    const int ns = c.ns, ne = c.ne;
-    cplx *F = bsh;                    // Felms, ld ns
-    cplx *Gi = bsh + ns * ns;         // Gamma^-1, ld ns
-    __shared__ cplx ikk[64][2], kik[2][64], n21[2][64], vuk[4], gkk[4];
-    __shared__ int svec[64];
-    __shared__ int s_acc, s_ik;
-    __shared__ double s_accm;
-    __shared__ cplx s_phase;
-    __shared__ int cfl[32], bsite[64], xv[64];   // field and sites of the stock's nb <= 32 bonds
-    __shared__ double ua[32];                    // their acceptance uniforms
-    __shared__ cplx vdl[4], dv[64];
-    int32_t *cf = c.conf + ((size_t)(nt - 1) * c.nn_nf + nf) * c.n + ib0;
-    const double *u = c.unif + uoff;
-    for (int e = threadIdx.x; e < ns * ns; e += blockDim.x) {
-        F[e] = c.Felms[e];
-        Gi[e] = make_double2(0.0, 0.0);
-    }
-    if (threadIdx.x < nb) {
-        const int q = threadIdx.x, ist = nf * c.nn_lf + ib0 + q;
-        cfl[q] = cf[q];
-        ua[q] = u[2 * q + 1];
-        bsite[2 * q] = c.bonds[2 * ist];
-        bsite[2 * q + 1] = c.bonds[2 * ist + 1];
-    }
-    if (threadIdx.x < 4) vdl[threadIdx.x] = c.vd[threadIdx.x];
-    if (threadIdx.x == 0) {
-        s_ik = 0;
-        s_accm = 0.0;
-        s_phase = make_double2(c.sc[SC_PHASE], c.sc[SC_PHASE + 1]);
-    }
-    __syncthreads();
-    for (int q = 0; q < nb; q++) {
-        const int ik = s_ik;
-        const int s1 = 2 * q, s2 = s1 + 1;
-        if (ik > 0) {
-            // ikk = Gamma^-1 PFP_ikk (ik x 2): two threads per entry, each half of the sum
-            {
-                const int o = threadIdx.x >> 1, h = threadIdx.x & 1;
-                const int m = o % ik, col = o / ik;
-                const int sc_ = col ? s2 : s1;
-                double ar = 0.0, ai = 0.0;
-                if (o < 2 * ik) {
-                    // four terms' reads issued together, the sum in the order p = h, h + 2, ...
-                    int p = h;
-                    for (; p + 6 < ik; p += 8) {
-                        const int q0 = svec[p], q1 = svec[p + 2], q2 = svec[p + 4], q3 = svec[p + 6];
-                        const cplx g0 = Gi[m + p * ns], g1 = Gi[m + (p + 2) * ns], g2 = Gi[m + (p + 4) * ns],
-                                   g3 = Gi[m + (p + 6) * ns];
-                        const cplx f0 = F[q0 + sc_ * ns], f1 = F[q1 + sc_ * ns], f2 = F[q2 + sc_ * ns],
-                                   f3 = F[q3 + sc_ * ns];
-                        ar += g0.x * f0.x - g0.y * f0.y; ai += g0.x * f0.y + g0.y * f0.x;
-                        ar += g1.x * f1.x - g1.y * f1.y; ai += g1.x * f1.y + g1.y * f1.x;
-                        ar += g2.x * f2.x - g2.y * f2.y; ai += g2.x * f2.y + g2.y * f2.x;
-                        ar += g3.x * f3.x - g3.y * f3.y; ai += g3.x * f3.y + g3.y * f3.x;
-                    }
-                    for (; p < ik; p += 2) {
-                        const cplx g = Gi[m + p * ns], f = F[svec[p] + sc_ * ns];
-                        ar += g.x * f.x - g.y * f.y;
-                        ai += g.x * f.y + g.y * f.x;
-                    }
-                }
-                ar += dpp_d<0xB1>(ar);   // the partner lane (lane ^ 1)
-                ai += dpp_d<0xB1>(ai);
-                if (o < 2 * ik && h == 0) ikk[m][col] = make_double2(ar, ai);
-            }
-            __syncthreads();
-            // vuk = PFP_kik ikk (2 x 2): one wave per entry, one lane per term
-            {
-                const int w = threadIdx.x >> 6, m = threadIdx.x & 63;
-                if (w < 4) {
-                    const int r = w & 1, col = w >> 1;
-                    const int sr = r ? s2 : s1;
-                    double ar = 0.0, ai = 0.0;
-                    if (m < ik) {
-                        const cplx f = F[sr + svec[m] * ns], x = ikk[m][col];
-                        ar = f.x * x.x - f.y * x.y;
-                        ai = f.x * x.y + f.y * x.x;
-                    }
-                    ar = wave_sum_dpp(ar);
-                    ai = wave_sum_dpp(ai);
-                    if (m == 0) vuk[r + 2 * col] = make_double2(ar, ai);
-                }
-            }
-        } else if (threadIdx.x < 4) {
-            vuk[threadIdx.x] = make_double2(0.0, 0.0);
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const int is = cfl[q];
-            // iflip = ceiling(u * (lcomp - 1)) = 1 for the two-valued bond field
-            const cplx dp = vdl[2 * (is - 1)], dm = vdl[2 * (is - 1) + 1];
-            cplx v11 = csub(F[s1 + s1 * ns], vuk[0]), v21 = csub(F[s2 + s1 * ns], vuk[1]);
-            cplx v12 = csub(F[s1 + s2 * ns], vuk[2]), v22 = csub(F[s2 + s2 * ns], vuk[3]);
-            v11 = cadd(make_double2(1.0, 0.0), cmul(v11, dp));
-            v21 = cmul(v21, dp);
-            v12 = cmul(v12, dm);
-            v22 = cadd(make_double2(1.0, 0.0), cmul(v22, dm));
-            const cplx ratio1 = csub(cmul(v11, v22), cmul(v12, v21));
-            const cplx ph = s_phase;
-            const double ratio_re = cmul(ratio1, ph).x / ph.x;
-            const double ratio_abs = ratio_re < 0.0 ? -ratio_re : ratio_re;
-            const int acc = ratio_abs > ua[q];
-            s_acc = acc;
-            if (acc) {
-                s_accm += 1.0;
-                const double wgt = sqrt(cmul(ratio1, cconj(ratio1)).x);
-                s_phase = cscale(cmul(ph, ratio1), 1.0 / wgt);
-                gkk[0] = cdiv(cmul(v22, dp), ratio1);
-                gkk[2] = cdiv(cmul(make_double2(-v12.x, -v12.y), dp), ratio1);
-                gkk[1] = cdiv(cmul(make_double2(-v21.x, -v21.y), dm), ratio1);
-                gkk[3] = cdiv(cmul(v11, dm), ratio1);
-                cfl[q] = 3 - is;
-                xv[ik] = bsite[2 * q];
-                xv[ik + 1] = bsite[2 * q + 1];
-                dv[ik] = dp;
-                dv[ik + 1] = dm;
-            }
-        }
-        __syncthreads();
-        if (!s_acc) continue;
-        if (ik > 0) {
-            // kik = PFP_kik Gamma^-1 (2 x ik): two threads per entry
-            {
-                const int o = threadIdx.x >> 1, h = threadIdx.x & 1;
-                const int r = o % 2, p = o / 2;
-                const int sr = r ? s2 : s1;
-                double ar = 0.0, ai = 0.0;
-                if (o < 2 * ik) {
-                    int m = h;
-                    for (; m + 6 < ik; m += 8) {
-                        const int q0 = svec[m], q1 = svec[m + 2], q2 = svec[m + 4], q3 = svec[m + 6];
-                        const cplx f0 = F[sr + q0 * ns], f1 = F[sr + q1 * ns], f2 = F[sr + q2 * ns], f3 = F[sr + q3 * ns];
-                        const cplx g0 = Gi[m + p * ns], g1 = Gi[(m + 2) + p * ns], g2 = Gi[(m + 4) + p * ns],
-                                   g3 = Gi[(m + 6) + p * ns];
-                        ar += f0.x * g0.x - f0.y * g0.y; ai += f0.x * g0.y + f0.y * g0.x;
-                        ar += f1.x * g1.x - f1.y * g1.y; ai += f1.x * g1.y + f1.y * g1.x;
-                        ar += f2.x * g2.x - f2.y * g2.y; ai += f2.x * g2.y + f2.y * g2.x;
-                        ar += f3.x * g3.x - f3.y * g3.y; ai += f3.x * g3.y + f3.y * g3.x;
-                    }
-                    for (; m < ik; m += 2) {
-                        const cplx f = F[sr + svec[m] * ns], g = Gi[m + p * ns];
-                        ar += f.x * g.x - f.y * g.y;
-                        ai += f.x * g.y + f.y * g.x;
-                    }
-                }
-                ar += dpp_d<0xB1>(ar);
-                ai += dpp_d<0xB1>(ai);
-                if (o < 2 * ik && h == 0) kik[r][p] = make_double2(ar, ai);
-            }
-            __syncthreads();
-            // 21 block = -gkk kik
-            for (int e = threadIdx.x; e < 2 * ik; e += blockDim.x) {
-                const int r = e % 2, p = e / 2;
-                cplx a = cadd(cmul(gkk[r], kik[0][p]), cmul(gkk[r + 2], kik[1][p]));
-                n21[r][p] = make_double2(-a.x, -a.y);
-            }
-            __syncthreads();
-            // 11 block -= ikk n21; 12 block = -ikk gkk; 21 block stored
-            for (int e = threadIdx.x; e < ik * ik; e += blockDim.x) {
-                const int m = e % ik, p = e / ik;
-                cplx a = cadd(cmul(ikk[m][0], n21[0][p]), cmul(ikk[m][1], n21[1][p]));
-                Gi[m + p * ns] = csub(Gi[m + p * ns], a);
-            }
-            for (int e = threadIdx.x; e < 2 * ik; e += blockDim.x) {
-                const int m = e % ik, col = e / ik;
-                cplx a = cadd(cmul(ikk[m][0], gkk[2 * col]), cmul(ikk[m][1], gkk[2 * col + 1]));
-                Gi[m + (ik + col) * ns] = make_double2(-a.x, -a.y);
-                const int r = e % 2, p = e / 2;
-                Gi[(ik + r) + p * ns] = n21[r][p];
-            }
-        }
-        if (threadIdx.x < 4) Gi[(ik + (threadIdx.x & 1)) + (ik + (threadIdx.x >> 1)) * ns] = gkk[threadIdx.x];
-        if (threadIdx.x == 0) {
-            svec[ik] = s1;
-            svec[ik + 1] = s2;
-            s_ik = ik + 2;
-        }
-        __syncthreads();
-    }
-    // Gamma^-1, the accepted rows of Rrows (Vmat) and columns of ulP (Umat) for the flush; the
-    // field, the accepted sites and their deltas
-    const int ik = s_ik;
-    for (int e = threadIdx.x; e < ns * ns; e += blockDim.x) c.Ginv[e] = Gi[e];
-    for (int q = threadIdx.x; q < nb; q += blockDim.x) cf[q] = cfl[q];
-    for (int k = threadIdx.x; k < ik; k += blockDim.x) {
-        c.xvec[k] = xv[k];
-        c.Dvec[k] = dv[k];
-    }
-    for (int e = threadIdx.x; e < ik * ne; e += blockDim.x) {
-        const int m = e % ik, l = e / ik;
-        c.Vmat[m + (size_t)l * ns] = c.Rrows[svec[m] + (size_t)l * ns];
-        const int l2 = e % ne, m2 = e / ne;
-        c.Umat[l2 + (size_t)m2 * ne] = c.ulP[l2 + (size_t)svec[m2] * ne];
-    }
-    if (threadIdx.x == 0) {
-        c.ikd[0] = ik;
-        c.sc[SC_PHASE] = s_phase.x;
-        c.sc[SC_PHASE + 1] = s_phase.y;
-        c.sc[SC_ACC] += s_accm;
-        c.sc[SC_TRIED] += nb;
-    }
-}
-
-// the on-site field's stock of consecutive sites i0 .. i0 + nup - 1, one workgroup per chain
-// (src/dqmc_config_u/dqmc_proj_update_submatrix_LR.f90:83-237): per site the 1 x 1 ratio
-// 1 + (F_kk - F_kP Gamma^-1 F_Pk) Delta(iflip, is), ratiotot = ratio1^nflr gaml(isp)/gaml(is)
-// phase_ratio(iflip, is), the Metropolis test on Re(ratiotot phase)/Re(phase), and on
-// acceptance Gamma^-1 bordered by one row and column.  Felms and Gamma^-1 live in LDS, and so do
-// the stock's field, draws and HS tables (the field, xvec and Dvec are written back at the end):
-// the site loop itself touches no global memory.
-extern "C" __global__ void __launch_bounds__(256)
-kp_stock_sites(const PChain *chains, int nt, int i0, int nup, size_t uoff)
-{
-    extern __shared__ cplx bsh[];
-    const PChain &c = chains[blockIdx.x];
-    const int ns = c.ns, ne = c.ne, lc = c.ulcomp;
-    cplx *F = bsh;                    // Felms, ld ns
-    cplx *Gi = bsh + ns * ns;         // Gamma^-1, ld ns
-    __shared__ cplx ikk[64], kik[64], s_vuk, s_gkk;
-    __shared__ int svec[64];
-    __shared__ int s_acc, s_ik;
-    __shared__ double s_accm;
-    __shared__ cplx s_phase;
-    __shared__ int cfl[64], xv[64];              // field of the stock's nup <= 64 sites, accepted sites
-    __shared__ double u1l[64], u2l[64], ugl[4];  // their two uniforms; gaml
-    __shared__ cplx udl[12], url[12], dv[64];    // delta_bmat, phase_ratio; accepted deltas
-    int32_t *cf = c.uconf + (size_t)(nt - 1) * c.n + i0;
-    const double *u = c.unif + uoff;
-    const int nflr = c.nflr;
-    for (int e = threadIdx.x; e < ns * ns; e += blockDim.x) {
-        F[e] = c.Felms[e];
-        Gi[e] = make_double2(0.0, 0.0);
-    }
-    if (threadIdx.x < nup) {
-        cfl[threadIdx.x] = cf[threadIdx.x];
-        u1l[threadIdx.x] = u[2 * threadIdx.x];
-        u2l[threadIdx.x] = u[2 * threadIdx.x + 1];
-    }
-    if (threadIdx.x < 12) {
-        udl[threadIdx.x] = c.ud[threadIdx.x];
-        url[threadIdx.x] = c.uratio[threadIdx.x];
-    }
-    if (threadIdx.x < 4) ugl[threadIdx.x] = c.ug[threadIdx.x];
-    if (threadIdx.x == 0) {
-        s_ik = 0;
-        s_accm = 0.0;
-        s_phase = make_double2(c.sc[SC_PHASE], c.sc[SC_PHASE + 1]);
-    }
-    __syncthreads();
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int q = 0; q < nup; q++) {
-        const int ik = s_ik;
-        if (ik > 0) {
-            // ikk = Gamma^-1 F(P, q): four threads per entry, each a quarter of the sum
-            {
-                const int m = threadIdx.x >> 2, h = threadIdx.x & 3;
-                double ar = 0.0, ai = 0.0;
-                if (m < ik) {
-                    // four terms' reads issued together, the sum in the order p = h, h + 4, ...
-                    int p = h;
-                    for (; p + 12 < ik; p += 16) {
-                        const int q0 = svec[p], q1 = svec[p + 4], q2 = svec[p + 8], q3 = svec[p + 12];
-                        const cplx g0 = Gi[m + p * ns], g1 = Gi[m + (p + 4) * ns], g2 = Gi[m + (p + 8) * ns],
-                                   g3 = Gi[m + (p + 12) * ns];
-                        const cplx f0 = F[q0 + q * ns], f1 = F[q1 + q * ns], f2 = F[q2 + q * ns], f3 = F[q3 + q * ns];
-                        ar += g0.x * f0.x - g0.y * f0.y; ai += g0.x * f0.y + g0.y * f0.x;
-                        ar += g1.x * f1.x - g1.y * f1.y; ai += g1.x * f1.y + g1.y * f1.x;
-                        ar += g2.x * f2.x - g2.y * f2.y; ai += g2.x * f2.y + g2.y * f2.x;
-                        ar += g3.x * f3.x - g3.y * f3.y; ai += g3.x * f3.y + g3.y * f3.x;
-                    }
-                    for (; p < ik; p += 4) {
-                        const cplx g = Gi[m + p * ns], f = F[svec[p] + q * ns];
-                        ar += g.x * f.x - g.y * f.y;
-                        ai += g.x * f.y + g.y * f.x;
-                    }
-                }
-                ar += dpp_d<0xB1>(ar);   // lane ^ 1, then lane ^ 2 (in-quad DPP)
-                ai += dpp_d<0xB1>(ai);
-                ar += dpp_d<0x4E>(ar);
-                ai += dpp_d<0x4E>(ai);
-                if (m < ik && h == 0) ikk[m] = make_double2(ar, ai);
-            }
-            __syncthreads();
-            // vuk = F(q, P) ikk: wave 0, one lane per term
-            if (w == 0) {
-                double ar = 0.0, ai = 0.0;
-                if (lane < ik) {
-                    const cplx f = F[q + svec[lane] * ns], x = ikk[lane];
-                    ar = f.x * x.x - f.y * x.y;
-                    ai = f.x * x.y + f.y * x.x;
-                }
-                ar = wave_sum_dpp(ar);
-                ai = wave_sum_dpp(ai);
-                if (lane == 0) s_vuk = make_double2(ar, ai);
-            }
-        } else if (threadIdx.x == 0) {
-            s_vuk = make_double2(0.0, 0.0);
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const int is = cfl[q];
-            const int iflip = (int)ceil(u1l[q] * (lc - 1));
-            const int isp = (is + iflip - 1) % lc + 1;
-            const int k = (iflip - 1) + (lc - 1) * (is - 1);
-            const cplx d = udl[k];
-            const cplx ratio1 = cadd(make_double2(1.0, 0.0), cmul(csub(F[q + q * ns], s_vuk), d));
-            cplx rt = ratio1;
-            for (int f = 1; f < nflr; f++) rt = cmul(rt, ratio1);
-            rt = cmul(cscale(rt, ugl[isp - 1] / ugl[is - 1]), url[k]);
-            const cplx ph = s_phase;
-            const double ratio_re = cmul(rt, ph).x / ph.x;
-            const double ratio_abs = ratio_re < 0.0 ? -ratio_re : ratio_re;
-            const int acc = ratio_abs > u2l[q];
-            s_acc = acc;
-            if (acc) {
-                s_accm += 1.0;
-                const double wgt = sqrt(cmul(rt, cconj(rt)).x);
-                s_phase = cscale(cmul(ph, rt), 1.0 / wgt);
-                s_gkk = cdiv(d, ratio1);
-                cfl[q] = isp;
-                xv[ik] = i0 + q;
-                dv[ik] = d;
-            }
-        }
-        __syncthreads();
-        if (!s_acc) continue;
-        const cplx gkk = s_gkk;
-        if (ik > 0) {
-            // kik = F(q, P) Gamma^-1: four threads per entry
-            {
-                const int p = threadIdx.x >> 2, h = threadIdx.x & 3;
-                double ar = 0.0, ai = 0.0;
-                if (p < ik) {
-                    int m = h;
-                    for (; m + 12 < ik; m += 16) {
-                        const int q0 = svec[m], q1 = svec[m + 4], q2 = svec[m + 8], q3 = svec[m + 12];
-                        const cplx f0 = F[q + q0 * ns], f1 = F[q + q1 * ns], f2 = F[q + q2 * ns], f3 = F[q + q3 * ns];
-                        const cplx g0 = Gi[m + p * ns], g1 = Gi[(m + 4) + p * ns], g2 = Gi[(m + 8) + p * ns],
-                                   g3 = Gi[(m + 12) + p * ns];
-                        ar += f0.x * g0.x - f0.y * g0.y; ai += f0.x * g0.y + f0.y * g0.x;
-                        ar += f1.x * g1.x - f1.y * g1.y; ai += f1.x * g1.y + f1.y * g1.x;
-                        ar += f2.x * g2.x - f2.y * g2.y; ai += f2.x * g2.y + f2.y * g2.x;
-                        ar += f3.x * g3.x - f3.y * g3.y; ai += f3.x * g3.y + f3.y * g3.x;
-                    }
-                    for (; m < ik; m += 4) {
-                        const cplx f = F[q + svec[m] * ns], g = Gi[m + p * ns];
-                        ar += f.x * g.x - f.y * g.y;
-                        ai += f.x * g.y + f.y * g.x;
-                    }
-                }
-                ar += dpp_d<0xB1>(ar);
-                ai += dpp_d<0xB1>(ai);
-                ar += dpp_d<0x4E>(ar);
-                ai += dpp_d<0x4E>(ai);
-                if (p < ik && h == 0) kik[p] = make_double2(ar, ai);
-            }
-            __syncthreads();
-            // 11 block -= ikk (-gkk kik); 12 block = -ikk gkk; 21 block = -gkk kik
-            for (int e = threadIdx.x; e < ik * ik; e += blockDim.x) {
-                const int m = e % ik, p = e / ik;
-                const cplx n21 = cmul(gkk, kik[p]);          // minus the 21 entry
-                Gi[m + p * ns] = cadd(Gi[m + p * ns], cmul(ikk[m], n21));
-            }
-            for (int e = threadIdx.x; e < ik; e += blockDim.x) {
-                const cplx a = cmul(ikk[e], gkk), b = cmul(gkk, kik[e]);
-                Gi[e + ik * ns] = make_double2(-a.x, -a.y);
-                Gi[ik + e * ns] = make_double2(-b.x, -b.y);
-            }
-        }
-        if (threadIdx.x == 0) {
-            Gi[ik + ik * ns] = gkk;
-            svec[ik] = q;
-            s_ik = ik + 1;
-        }
-        __syncthreads();
-    }
-    const int ik = s_ik;
-    for (int e = threadIdx.x; e < ns * ns; e += blockDim.x) c.Ginv[e] = Gi[e];
-    for (int q = threadIdx.x; q < nup; q += blockDim.x) cf[q] = cfl[q];
-    for (int k = threadIdx.x; k < ik; k += blockDim.x) {
-        c.xvec[k] = xv[k];
-        c.Dvec[k] = dv[k];
-    }
-    for (int e = threadIdx.x; e < ik * ne; e += blockDim.x) {
-        const int m = e % ik, l = e / ik;
-        c.Vmat[m + (size_t)l * ns] = c.Rrows[svec[m] + (size_t)l * ns];
-        const int l2 = e % ne, m2 = e / ne;
-        c.Umat[l2 + (size_t)m2 * ne] = c.ulP[l2 + (size_t)svec[m2] * ne];
-    }
-    if (threadIdx.x == 0) {
-        c.ikd[0] = ik;
-        c.sc[SC_PHASE] = s_phase.x;
-        c.sc[SC_PHASE + 1] = s_phase.y;
-        c.sc[SC_ACC] += s_accm;
-        c.sc[SC_TRIED] += nup;
-    }
-}
-
-// UR(x_m, :) += D_m UR(x_m, :) for the stock's accepted rows (:249-254)
-extern "C" __global__ void __launch_bounds__(256)
-kp_stock_scale(const PChain *chains)
-{
-    const PChain &c = chains[blockIdx.z];
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ik = c.ikd[0];
-    if (e >= ik * c.ne) return;
-    const int m = e % ik, l = e / ik;
-    cplx *p = c.UR + (size_t)c.xvec[m] + (size_t)l * c.n;
-    *p = cadd(*p, cmul(c.Dvec[m], *p));
 }
 
 // ---- stabilization --------------------------------------------------------------------------
