@@ -58,18 +58,19 @@ __device__ __forceinline__ void cols16(F f)
     }
 }
 
+template <int FT>
 struct FBlk {
-    double4_t r[FTW], i[FTW];
+    double4_t r[FT], i[FT];
 };
 
 // rows row0 + 16 rt + 4 r + l/16 (rt = w + NW tt) of column col0 + l%16; zero past nrow and ncol
-template <int NW>
-__device__ __forceinline__ void blk_load(FBlk &x, GAS cplx *A, int lda, int nrow, int col, int ncol, int w, int lq,
+template <int NW, int FT>
+__device__ __forceinline__ void blk_load(FBlk<FT> &x, GAS cplx *A, int lda, int nrow, int col, int ncol, int w, int lq,
                                          const GAS int32_t *pm)
 {
     const size_t cc = (size_t)min(col, ncol - 1) * lda;
 #pragma unroll
-    for (int tt = 0; tt < FTW; tt++)
+    for (int tt = 0; tt < FT; tt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int row = 16 * (w + NW * tt) + 4 * r + lq, rc = min(row, nrow - 1);
@@ -90,13 +91,13 @@ __device__ __forceinline__ cplx panel_v(GAS cplx *V, int lda, int m, int b, int 
 // X <- (I - V op(T) V^H) X with the panel V (m x b, first row at tile toff of the workgroup's rows);
 // op = conjugate transpose for HERM.  red: NW x 256 complex.  One barrier; red is free for the next
 // use after the caller's next barrier (callers alternate between two).
-template <int NW, bool HERM>
-__device__ __forceinline__ void apply_panel(FBlk &x, GAS cplx *V, int lda, int m, int b, const GAS cplx *T, int toff, cplx *red,
+template <int NW, bool HERM, int FT>
+__device__ __forceinline__ void apply_panel(FBlk<FT> &x, GAS cplx *V, int lda, int m, int b, const GAS cplx *T, int toff, cplx *red,
                                             int w, int lane, int lq, int l16)
 {
     double4_t wr = {}, wi = {};
 #pragma unroll
-    for (int tt = 0; tt < FTW; tt++) {
+    for (int tt = 0; tt < FT; tt++) {
         const int rt = w + NW * tt - toff;
         if (rt >= 0 && 16 * rt < m) {
             cplx v[4];
@@ -138,7 +139,7 @@ __device__ __forceinline__ void apply_panel(FBlk &x, GAS cplx *V, int lda, int m
         yi = mfma(tv[s].y, wr[s], yi);
     }
 #pragma unroll
-    for (int tt = 0; tt < FTW; tt++) {
+    for (int tt = 0; tt < FT; tt++) {
         const int rt = w + NW * tt - toff;
         if (rt >= 0 && 16 * rt < m) {
             cplx v[4];
@@ -175,13 +176,13 @@ struct QrLds {
 // behind the only barrier).  Columns q > j give v_j^H a_q for the update, columns q < j v_j^H v_q for
 // T.  Every lane evaluates the scalars of zlarfg.  A column stays unscaled until the end (its lanes
 // keep the factor), with alpha - beta in place of its row j while it is applied, so that the loop
-// has no per-element cases outside the panel's first tile.  tau and T (zlarft) go to global memory.
-template <int NW>
-__device__ __forceinline__ void qr_panel(FBlk &x, int b, int toff, GAS cplx *tau_out, GAS cplx *T, QrLds<NW> &L,
-                                         int w, int lane, int lq, int l16)
+// has no per-element cases outside the panel's first tile.
+template <int NW, int FT>
+__device__ __forceinline__ void qr_panel(FBlk<FT> &x, int b, int toff, cplx &tau_own, QrLds<NW> &L, int w, int lane, int lq, int l16)
 {
     // of the lane's own column l16
-    cplx tau_own = make_double2(0.0, 0.0), scal_own = make_double2(1.0, 0.0);
+    tau_own = make_double2(0.0, 0.0);
+    cplx scal_own = make_double2(1.0, 0.0);
     double beta_own = 0.0;
     cols16([&](auto jc) {
         constexpr int j = decltype(jc)::value, par = j & 1;
@@ -189,9 +190,9 @@ __device__ __forceinline__ void qr_panel(FBlk &x, int b, int toff, GAS cplx *tau
         if (w == toff && lq == (j & 3)) L.rowj[par][l16] = make_double2(x.r[0][j >> 2], x.i[0][j >> 2]);
         // column j along the row groups; of tile tt = 0 only the rows below row j (the other tiles of the
         // wave always lie below)
-        cplx vb[FTW][4], s0 = make_double2(0.0, 0.0), s1 = s0;
+        cplx vb[FT > FTW ? 1 : FT][4], s0 = make_double2(0.0, 0.0), s1 = s0;
 #pragma unroll
-        for (int tt = 0; tt < FTW; tt++)
+        for (int tt = 0; tt < FT; tt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 cplx v = make_double2(row_bcast<j>(x.r[tt][r]), row_bcast<j>(x.i[tt][r]));
@@ -200,7 +201,7 @@ __device__ __forceinline__ void qr_panel(FBlk &x, int b, int toff, GAS cplx *tau
                     v.x = in ? v.x : 0.0;
                     v.y = in ? v.y : 0.0;
                 }
-                vb[tt][r] = v;
+                if (FT <= FTW || tt == 0) vb[tt][r] = v;
                 cplx &s = r & 1 ? s1 : s0;
                 s.x = fma(v.x, x.r[tt][r], fma(v.y, x.i[tt][r], s.x));
                 s.y = fma(v.x, x.i[tt][r], fma(-v.y, x.r[tt][r], s.y));
@@ -251,10 +252,17 @@ __device__ __forceinline__ void qr_panel(FBlk &x, int b, int toff, GAS cplx *tau
             vb[0][j >> 2].y = rj ? amb.y : vb[0][j >> 2].y;
         }
 #pragma unroll
-        for (int tt = 0; tt < FTW; tt++)
+        for (int tt = 0; tt < FT; tt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const cplx v = vb[tt][r];
+                cplx v;
+                if (FT <= FTW || tt == 0)
+                    v = vb[tt][r];
+                else {
+                    // broadcast again (the empty asm: not kept from above, there are no registers for it)
+                    asm volatile("" : "+v"(x.r[tt][r]), "+v"(x.i[tt][r]));
+                    v = make_double2(row_bcast<j>(x.r[tt][r]), row_bcast<j>(x.i[tt][r]));
+                }
                 x.r[tt][r] = fma(-v.x, g.x, fma(v.y, g.y, x.r[tt][r]));
                 x.i[tt][r] = fma(-v.x, g.y, fma(-v.y, g.x, x.i[tt][r]));
             }
@@ -262,7 +270,7 @@ __device__ __forceinline__ void qr_panel(FBlk &x, int b, int toff, GAS cplx *tau
     // the reflectors in units of v_j = 1, beta on the diagonal
     if (l16 < b)
 #pragma unroll
-        for (int tt = 0; tt < FTW; tt++)
+        for (int tt = 0; tt < FT; tt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int row = 4 * r + lq;
@@ -271,6 +279,12 @@ __device__ __forceinline__ void qr_panel(FBlk &x, int b, int toff, GAS cplx *tau
                 x.r[tt][r] = below ? v.x : diag ? beta_own : x.r[tt][r];
                 x.i[tt][r] = below ? v.y : diag ? 0.0 : x.i[tt][r];
             }
+}
+
+// tau and T of the panel (wave 0, after the panel is stored: T's row takes the registers that held it)
+template <int NW>
+__device__ __forceinline__ void qr_tfactor(int b, cplx tau_own, GAS cplx *tau_out, GAS cplx *T, QrLds<NW> &L, int w, int lane)
+{
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     if (w == 0 && lane < FPB) {
         // lane i builds row i of T: T(i, j) = -tau_j sum_{i <= q < j} T(i, q) S(q, j)
@@ -300,35 +314,53 @@ __device__ __forceinline__ void qr_panel(FBlk &x, int b, int toff, GAS cplx *tau
     }
 }
 
-template <int NW>
+template <int NW, int FT>
 __global__ void __launch_bounds__(64 * NW, 2)
-k_qr_step(const DChain *chains, int sel, int k, int out_pt)
+k_qr_step(const DChain *chains, int sel, int k, int out_pt, int nc)
 {
     __shared__ cplx red[NW * 256];
     __shared__ QrLds<NW> L;
     const DChain &c = chains[blockIdx.x];
-    const int n = c.n, kb = k + blockIdx.y, np = (n + FPB - 1) / FPB;
+    const int n = c.n, ncol = nc > 0 ? nc : n, kb = k + blockIdx.y, np = (ncol + FPB - 1) / FPB;
     if (kb >= np) return;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, lq = lane >> 4;
     const int k0 = FPB * max(k - 1, 0), m = n - k0, col = FPB * kb + l16, toff = k > 0 ? 1 : 0;
     GAS cplx *M = gp(chain_mat(c, sel, 0)), *A = M + k0;
-    FBlk x;
-    blk_load<NW>(x, A, n, m, col, n, w, lq, nullptr);
+    FBlk<FT> x;
+    blk_load<NW>(x, A, n, m, col, ncol, w, lq, nullptr);
     if (k > 0)
         apply_panel<NW, true>(x, A + (size_t)k0 * n, n, m, min(FPB, m), gp(c.tblk) + (size_t)(k - 1) * FPB * FPB, 0, red,
                               w, lane, lq, l16);
-    if (kb == k) {
-        const int q0 = FPB * k;
-        qr_panel<NW>(x, min(FPB, n - q0), toff, gp(c.tau) + q0, gp(c.tblk) + (size_t)k * FPB * FPB, L, w, lane, lq, l16);
-    }
+    cplx tau_own = make_double2(0.0, 0.0);
+    if (kb == k) qr_panel<NW>(x, min(FPB, ncol - FPB * k), toff, tau_own, L, w, lane, lq, l16);
 #pragma unroll
-    for (int tt = 0; tt < FTW; tt++)
+    for (int tt = 0; tt < FT; tt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int row = 16 * (w + NW * tt) + 4 * r + lq;
-            if (row < m && col < n) gst(A + ((size_t)row + (size_t)col * n), make_double2(x.r[tt][r], x.i[tt][r]));
+            if (row < m && col < ncol) gst(A + ((size_t)row + (size_t)col * n), make_double2(x.r[tt][r], x.i[tt][r]));
         }
-    if (k == np - 1) {
+    if (kb == k)
+        qr_tfactor<NW>(min(FPB, ncol - FPB * k), tau_own, gp(c.tau) + FPB * k, gp(c.tblk) + (size_t)k * FPB * FPB, L, w, lane);
+    if (k == np - 1 && nc > 0) {
+        // log|det R| and its negative diagonal entries
+        __threadfence_block();
+        __syncthreads();
+        if (w == 0) {
+            double rl = 0.0, neg = 0.0;
+            for (int i = lane; i < ncol; i += 64) {
+                const double r = gld(M + ((size_t)i + (size_t)i * n)).x;
+                neg += r < 0.0 ? 1.0 : 0.0;
+                rl += log(fabs(r));
+            }
+            rl = wave_sum_dpp(rl);
+            neg = wave_sum_dpp(neg);
+            if (lane == 0) {
+                c.sc[SC_RLOG] = rl;
+                c.sc[SC_RNEG] = neg;
+            }
+        }
+    } else if (k == np - 1) {
         // log det Q = sum_i log(1 - tau_i 2 Re(tau_i) / |tau_i|^2), after the last panel
         __threadfence_block();
         __syncthreads();
@@ -353,21 +385,21 @@ k_qr_step(const DChain *chains, int sel, int k, int out_pt)
 // The columns 16 cb .. 16 cb + 15 of Q: the identity's columns through the panels cb .. 0 (the later ones
 // leave them as they are).  The workgroups of a chain run on one XCD, which keeps the reflectors
 // in its L2; the longest chains of panels start first.
-template <int NW>
+template <int NW, int FT>
 __global__ void __launch_bounds__(64 * NW, 2)
-k_formq_cb(const DChain *chains, int nch, int ncb, int sel, int out_pt)
+k_formq_cb(const DChain *chains, int nch, int ncb, int sel, int out_pt, int nc)
 {
     __shared__ cplx red[2][NW * 256];
     const int bid = blockIdx.x, kb = bid >> 3, chain = (bid & 7) + 8 * (kb / ncb), cb = ncb - 1 - kb % ncb;
     if (chain >= nch) return;
     const DChain &c = chains[chain];
-    const int n = c.n;
-    if (FPB * cb >= n) return;
+    const int n = c.n, ncol = nc > 0 ? nc : n;
+    if (FPB * cb >= ncol) return;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, lq = lane >> 4;
     GAS cplx *A = gp(chain_mat(c, sel, 0)), *Q = gp(c.U + (size_t)n * n * out_pt);
-    FBlk x;
+    FBlk<FT> x;
 #pragma unroll
-    for (int tt = 0; tt < FTW; tt++)
+    for (int tt = 0; tt < FT; tt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             x.r[tt][r] = w + NW * tt == cb && 4 * r + lq == l16 ? 1.0 : 0.0;
@@ -375,16 +407,19 @@ k_formq_cb(const DChain *chains, int nch, int ncb, int sel, int out_pt)
         }
     for (int p = cb; p >= 0; p--) {
         const int k0 = FPB * p;
-        apply_panel<NW, false>(x, A + ((size_t)k0 + (size_t)k0 * n), n, n - k0, min(FPB, n - k0),
+        apply_panel<NW, false>(x, A + ((size_t)k0 + (size_t)k0 * n), n, n - k0, min(FPB, ncol - k0),
                                gp(c.tblk) + (size_t)p * FPB * FPB, p, red[p & 1], w, lane, lq, l16);
     }
     const int col = FPB * cb + l16;
+    // a tall matrix's first column of Q takes the sign of det R (s_zgeQR_pqmc)
+    const bool flip = nc > 0 && col == 0 && ((int)c.sc[SC_RNEG] & 1);
 #pragma unroll
-    for (int tt = 0; tt < FTW; tt++)
+    for (int tt = 0; tt < FT; tt++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int row = 16 * (w + NW * tt) + 4 * r + lq;
-            if (row < n && col < n) gst(Q + ((size_t)row + (size_t)col * n), make_double2(x.r[tt][r], x.i[tt][r]));
+            if (row < n && col < ncol)
+                gst(Q + ((size_t)row + (size_t)col * n), make_double2(flip ? -x.r[tt][r] : x.r[tt][r], flip ? -x.i[tt][r] : x.i[tt][r]));
         }
 }
 
@@ -398,7 +433,7 @@ struct LuLds {
 // the lane's entry e (0 .. 4 FTW - 1) to *dst by a binary tree of uniform branches; the empty asm keeps
 // each leaf a branch target of its own (merged, they index the registers through private memory)
 template <int LO, int HI>
-__device__ __forceinline__ void blk_pick(const FBlk &x, int e, cplx *dst)
+__device__ __forceinline__ void blk_pick(const FBlk<FTW> &x, int e, cplx *dst)
 {
     if constexpr (HI - LO == 1) {
         *dst = make_double2(x.r[LO >> 2][LO & 3], x.i[LO >> 2][LO & 3]);
@@ -420,7 +455,7 @@ __device__ __forceinline__ void blk_pick(const FBlk &x, int e, cplx *dst)
 // only the rows 0 .. 15: lane i < 16 of every row group keeps where = the place of row i and top = the row
 // at place i.
 template <int NW>
-__device__ __forceinline__ void lu_panel(FBlk &x, int &act, int b, int toff, GAS int32_t *piv, int k0, double *info, LuLds<NW> &L,
+__device__ __forceinline__ void lu_panel(FBlk<FTW> &x, int &act, int b, int toff, GAS int32_t *piv, int k0, double *info, LuLds<NW> &L,
                                          int &where, int w, int lane, int lq, int l16)
 {
     int top = l16, below = 0;
@@ -524,10 +559,10 @@ __device__ __forceinline__ void lu_panel(FBlk &x, int &act, int b, int toff, GAS
 // Launch k = 0 .. np (np panels) on W3.  Panel k leaves in lup + k FLMAX the map of its interchanges: the
 // row (relative to row 16 k) that comes to each place from row 16 k on.  Launch np brings the columns
 // left of each panel into the final row order and sums the log determinant (s_inv_logdet_lu_z: Im
-// folded into (-pi, pi]); lperm is the row order of all interchanges (row i of P X is row lperm[i] of X).
+// folded into (-pi, pi]) to the scalar slot zslot, if not negative; fresh clears the zero-pivot slot first; lperm is the row order of all interchanges (row i of P X is row lperm[i] of X).
 template <int NW>
 __global__ void __launch_bounds__(64 * NW, 2)
-k_lu_step(const DChain *chains, int k)
+k_lu_step(const DChain *chains, int k, int zslot, int fresh)
 {
     __shared__ cplx Xp[256], D11[256];
     __shared__ LuLds<NW> L;
@@ -539,7 +574,7 @@ k_lu_step(const DChain *chains, int k)
     GAS cplx *M = gp(c.W3);
     GAS int32_t *lup = gp(c.lup);
     const int col = FPB * kb + l16;
-    FBlk x;
+    FBlk<FTW> x;
     if (k == np) {
         if (kb == np - 1) {
             if (w == 0) {
@@ -553,10 +588,10 @@ k_lu_step(const DChain *chains, int k)
                 }
                 lr = wave_sum_dpp(lr);
                 li = wave_sum_dpp(li);
-                if (lane == 0) {
+                if (lane == 0 && zslot >= 0) {
                     const double k2 = round(li / 2.0 / M_PI);
-                    c.sc[SC_ZLD] = lr;
-                    c.sc[SC_ZLD + 1] = li - 2.0 * M_PI * k2;
+                    c.sc[zslot] = lr;
+                    c.sc[zslot + 1] = li - 2.0 * M_PI * k2;
                 }
             }
             return;
@@ -666,7 +701,7 @@ k_lu_step(const DChain *chains, int k)
         const int row = 16 * (w + NW * (e >> 2) - toff) + 4 * (e & 3) + lq;
         act |= row >= 0 && row < mp ? 1 << e : 0;
     }
-    if (threadIdx.x == 0 && k == 0) c.sc[SC_INFO] = 0.0;
+    if (threadIdx.x == 0 && k == 0 && fresh) c.sc[SC_INFO] = 0.0;
     // the row order before this panel, loaded before any of it is replaced
     int lp[4 * FTW];
 #pragma unroll
@@ -701,9 +736,11 @@ k_lu_step(const DChain *chains, int k)
     }
 }
 
-template __global__ void k_qr_step<4>(const DChain *, int, int, int);
-template __global__ void k_qr_step<8>(const DChain *, int, int, int);
-template __global__ void k_formq_cb<4>(const DChain *, int, int, int, int);
-template __global__ void k_formq_cb<8>(const DChain *, int, int, int, int);
-template __global__ void k_lu_step<4>(const DChain *, int);
-template __global__ void k_lu_step<8>(const DChain *, int);
+#define QR(NW, FT)                                                                          \
+    template __global__ void k_qr_step<NW, FT>(const DChain *, int, int, int, int);          \
+    template __global__ void k_formq_cb<NW, FT>(const DChain *, int, int, int, int, int);
+QR(4, FTW)
+QR(8, FTW)
+QR(8, 2 * FTW)
+template __global__ void k_lu_step<4>(const DChain *, int, int, int);
+template __global__ void k_lu_step<8>(const DChain *, int, int, int);

@@ -7,7 +7,7 @@
 
 struct shp_ctx : ctx_base {
     int nch = 0, n = 0, ne = 0, ltrot = 0, nwrap = 0, nst = 0, kmode = 0, ns = 0, mid_len = 1;
-    int nn_nf = 0, nn_lf = 0, wrap_check = 1, pb = PB;
+    int nn_nf = 0, nn_lf = 0, wrap_check = 1;
     int update = SHP_U_LR, gblock = 0;   // update algorithm of the on-site field and its depth
     bool lwrapu = false, lwrapv = true, flav2 = true;   // flav2: nflr = 2 in every chain
     size_t slice_draws = 0;       // uniforms per slice of a pass
@@ -15,6 +15,7 @@ struct shp_ctx : ctx_base {
     std::vector<int> iwrap_nt, wrap_step;
     std::vector<PChain> hc;
     PChain *dc = nullptr;
+    DChain *dlu = nullptr, *dqr = nullptr;   // each chain's ne x ne and N x ne matrices as factor.hip takes them
     DChain *dview = nullptr;      // measurement view of each chain (G, bonds, staggering, bins)
     std::vector<DChain> hview;    // host copy of the views
     size_t eqt_lds = 0;           // LDS of k_eqt, 0 while no chain has correlation bins
@@ -25,8 +26,6 @@ struct shp_ctx : ctx_base {
 namespace {
 
 size_t p_lds_prop(const shp_ctx *c) { return (size_t)cb_ldr(c->n) * std::max(CPB, RPB) * sizeof(cplx); }
-size_t p_lds_qr(const shp_ctx *c) { return ((size_t)c->n * c->pb + 2 * PB * PB) * sizeof(cplx); }
-size_t p_lds_lu(const shp_ctx *c) { return (size_t)c->ne * PB * sizeof(cplx) + (size_t)c->ne * sizeof(int); }
 
 void pgemm(shp_ctx *ctx, int sa, int pa, int sb, int pb_, int sc, int pc, int m, int n, int k, int lda, int ldb,
            int ldc, double ar = 1.0, double br = 0.0)
@@ -220,7 +219,14 @@ void inverse(shp_ctx *ctx, int ul, int ur, int inv, int slot)
         pgemm(ctx, ul, 0, ur, 0, P_ULR, 0, ctx->ne, ctx->ne, ctx->n, ctx->ne, ctx->n, ctx->ne);
     }
     Tic t(ctx, T_LU);
-    hipLaunchKernelGGL(kp_lu_inv, dim3(ctx->nch), dim3(BLK_NT), p_lds_lu(ctx), ctx->st, ctx->dc, P_ULR, inv, slot);
+    // through the chain's view of its ne x ne matrices
+    const int np = (ctx->ne + FPB - 1) / FPB, nch8 = (ctx->nch + 7) / 8 * 8;
+    const bool w4 = ctx->ne <= 256;
+    for (int k = 0; k <= np; k++)
+        hipLaunchKernelGGL(w4 ? k_lu_step<4> : k_lu_step<8>, dim3(ctx->nch, k < np ? np - k : np), dim3(w4 ? 256 : 512), 0,
+                           ctx->st, ctx->dlu, k, slot, 0);
+    hipLaunchKernelGGL(w4 ? k_solve_cb<4> : k_solve_cb<8>, dim3(nch8 * np), dim3(w4 ? 256 : 512), 0, ctx->st, ctx->dlu,
+                       ctx->nch, np, (int)(inv == P_ULRINV ? M_W1 : M_W2), 1);
 }
 
 // g = 1 - ur inv ul (src/dqmc_proj_core/green_equaltime.f90:14-21)
@@ -288,11 +294,19 @@ void save_old(shp_ctx *ctx)
     pcopy(ctx, P_URO, 0, P_UR, 0, ctx->n * ctx->ne);
 }
 
-// s_zgeQR_pqmc of asel (N x ne) with Q into T1
-void qr_to_t1(shp_ctx *ctx, int asel, int apt)
+// s_zgeQR_pqmc (lib/s_matrix.f90:1822-1996) of UR or T2 (N x ne): log|det R| and the count of negative
+// diagonal entries of R to SC_RLOG / SC_RNEG, Q into T1, its first column negated for an odd count
+void qr_to_t1(shp_ctx *ctx, int asel)
 {
     Tic t(ctx, T_QR);
-    hipLaunchKernelGGL(kp_qr_formq, dim3(ctx->nch), dim3(BLK_NT), p_lds_qr(ctx), ctx->st, ctx->dc, asel, apt, P_T1, 0);
+    // through the chain's view of its N x ne matrices; four waves hold 256 rows, eight 512 or 1024
+    const int np = (ctx->ne + FPB - 1) / FPB, nch8 = (ctx->nch + 7) / 8 * 8, nw = ctx->n <= 256 ? 4 : 8;
+    const int sel = asel == P_UR ? M_W1 : M_W2;
+    auto qr = nw == 4 ? k_qr_step<4, FTW> : ctx->n <= 512 ? k_qr_step<8, FTW> : k_qr_step<8, 2 * FTW>;
+    auto fq = nw == 4 ? k_formq_cb<4, FTW> : ctx->n <= 512 ? k_formq_cb<8, FTW> : k_formq_cb<8, 2 * FTW>;
+    for (int k = 0; k < np; k++)
+        hipLaunchKernelGGL(qr, dim3(ctx->nch, np - k), dim3(64 * nw), 0, ctx->st, ctx->dqr, sel, k, 0, ctx->ne);
+    hipLaunchKernelGGL(fq, dim3(nch8 * np), dim3(64 * nw), 0, ctx->st, ctx->dqr, ctx->nch, np, sel, 0, ctx->ne);
 }
 
 // Bmat_left_forward on UR (src/dqmc_proj_core.f90:68-116): K half, the bond fields of every
@@ -419,9 +433,7 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
         for (int i = 0; i < 2 * q.nst; i++)
             if (q.wrap_step[i] < 1 || q.wrap_step[i] > q.ltrot) { delete ctx; return SH_E_ARG; }
     }
-    // panel width of the QR: 16 columns while an N x 16 panel fits in LDS, else 8
-    ctx->pb = ((size_t)ctx->n * PB + 2 * PB * PB) * sizeof(cplx) <= 150 * 1024 ? PB : PB / 2;
-    if (p_lds_qr(ctx) > 150 * 1024 || p_lds_lu(ctx) > 150 * 1024 || p_lds_prop(ctx) > 150 * 1024) {
+    if (p_lds_prop(ctx) > 150 * 1024) {
         int rc = fail(ctx, SH_E_ARG, "matrix sizes beyond the LDS budget of the projective kernels");
         delete ctx;
         return rc;
@@ -432,30 +444,26 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
     ctx->wrap_step.assign(q0.wrap_step, q0.wrap_step + 2 * q0.nst);
     if (hipStreamCreate(&ctx->st) != hipSuccess) { delete ctx; return SH_E_HIP; }
     {
-        struct { const void *f; size_t bytes; } big[] = {
-            {(const void *)kp_prop, p_lds_prop(ctx)},
-            {(const void *)kp_qr_formq, p_lds_qr(ctx)}, {(const void *)kp_lu_inv, p_lds_lu(ctx)}};
-        for (auto &b : big) {
-            if (b.bytes <= 64 * 1024) continue;
-            if (hipFuncSetAttribute(b.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b.bytes) != hipSuccess) {
-                (void)hipGetLastError();
-                int rc = fail(ctx, SH_E_HIP, "dynamic LDS request above the device limit");
-                shp_destroy(ctx);
-                return rc;
-            }
+        const size_t bytes = p_lds_prop(ctx);
+        if (bytes > 64 * 1024 &&
+            hipFuncSetAttribute((const void *)kp_prop, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            int rc = fail(ctx, SH_E_HIP, "dynamic LDS request above the device limit");
+            shp_destroy(ctx);
+            return rc;
         }
     }
     const int n = ctx->n, ne = ctx->ne, ns = ctx->ns;
     const size_t nne = (size_t)n * ne, nn = (size_t)n * n;
     std::vector<int32_t> seeds(nchains);
-    std::vector<DChain> views(nchains);
+    std::vector<DChain> views(nchains), lus(nchains), qrs(nchains);
     ctx->hc.resize(nchains);
     for (int ci = 0; ci < nchains; ci++) {
         const shp_model &q = m[ci];
         PChain &c = ctx->hc[ci];
         memset(&c, 0, sizeof(c));
         c.n = n; c.ne = ne; c.nn_nf = q.nn_nf; c.nn_lf = q.nn_lf; c.kmode = q.kmode; c.ns = ns; c.ltrot = q.ltrot;
-        c.nst = q.nst; c.nflr = q.nflr; c.lq = q.lq; c.pb = ctx->pb;
+        c.nst = q.nst; c.nflr = q.nflr; c.lq = q.lq;
         c.UR = dalloc<cplx>(ctx, nne); c.UL = dalloc<cplx>(ctx, nne); c.T1 = dalloc<cplx>(ctx, nne);
         c.T2 = dalloc<cplx>(ctx, nne); c.ULo = dalloc<cplx>(ctx, nne); c.URo = dalloc<cplx>(ctx, nne);
         c.ULRINV = dalloc<cplx>(ctx, (size_t)ne * ne); c.ULR = dalloc<cplx>(ctx, (size_t)ne * ne);
@@ -465,8 +473,7 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
         c.Rrows = dalloc<cplx>(ctx, (size_t)ns * ne); c.Felms = dalloc<cplx>(ctx, (size_t)ns * ns);
         c.Ginv = dalloc<cplx>(ctx, (size_t)ns * ns); c.Vtmp = dalloc<cplx>(ctx, (size_t)ns * ne);
         c.Utmp = dalloc<cplx>(ctx, (size_t)ns * ne); c.Dvec = dalloc<cplx>(ctx, ns);
-        c.tau = dalloc<cplx>(ctx, ne); c.tblk = dalloc<cplx>(ctx, (size_t)(ne / (PB / 2) + 2) * PB * PB);
-        c.wk = dalloc<cplx>(ctx, (size_t)PB * std::max(n, ne));
+        c.tau = dalloc<cplx>(ctx, ne); c.tblk = dalloc<cplx>(ctx, (size_t)((ne + FPB - 1) / FPB) * FPB * FPB);
         c.piv = dalloc<int32_t>(ctx, ne);
         c.conf = dalloc<int32_t>(ctx, (size_t)n * q.nn_nf * q.ltrot);
         c.xvec = dalloc<int32_t>(ctx, ns); c.ikd = dalloc<int32_t>(ctx, 4);
@@ -499,7 +506,7 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
         c.stag = dupload<double>(ctx, q.stag, n);
         if (!c.UR || !c.UL || !c.T1 || !c.T2 || !c.ULo || !c.URo || !c.ULRINV || !c.ULR || !c.INV2 || !c.G || !c.G2 ||
             !c.Ust || !c.proj || !c.Rrows || !c.Felms || !c.Ginv ||
-            !c.Vtmp || !c.Utmp || !c.Dvec || !c.tau || !c.tblk || !c.wk || !c.piv || !c.conf || !c.xvec ||
+            !c.Vtmp || !c.Utmp || !c.Dvec || !c.tau || !c.tblk || !c.piv || !c.conf || !c.xvec ||
             !c.ikd || !c.unif || !c.sc || !c.logwDV || !c.rwork || !c.rng || !c.bonds || !c.kt ||
             !c.ktm1 || !c.stag || (ctx->lwrapu && !c.uconf)) {
             int rc = fail(ctx, SH_E_HIP, "device allocation failed");
@@ -517,6 +524,18 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
         sc0[SC_PHASE] = 1.0;
         hipMemcpy(c.sc, sc0, sizeof(sc0), hipMemcpyHostToDevice);
         seeds[ci] = q.seed;
+        DChain &lu = lus[ci], &qr = qrs[ci];
+        memset(&lu, 0, sizeof(lu));
+        lu.n = ne; lu.W3 = c.ULR; lu.W1 = c.ULRINV; lu.W2 = c.INV2; lu.piv = c.piv; lu.sc = c.sc;
+        lu.lperm = dalloc<int32_t>(ctx, ne);
+        lu.lup = dalloc<int32_t>(ctx, (size_t)((ne + FPB - 1) / FPB) * FLMAX);
+        memset(&qr, 0, sizeof(qr));
+        qr.n = n; qr.W1 = c.UR; qr.W2 = c.T2; qr.U = c.T1; qr.tau = c.tau; qr.tblk = c.tblk; qr.sc = c.sc;
+        if (!lu.lperm || !lu.lup) {
+            int rc = fail(ctx, SH_E_HIP, "device allocation failed");
+            shp_destroy(ctx);
+            return rc;
+        }
         // the measurement kernels read G, the bonds, the staggering and the bins through a view
         DChain &v = views[ci];
         memset(&v, 0, sizeof(v));
@@ -564,9 +583,11 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
     }
     ctx->dc = dupload<PChain>(ctx, ctx->hc.data(), nchains);
     ctx->dview = dupload<DChain>(ctx, views.data(), nchains);
+    ctx->dlu = dupload<DChain>(ctx, lus.data(), nchains);
+    ctx->dqr = dupload<DChain>(ctx, qrs.data(), nchains);
     ctx->hview = views;
     ctx->d_seeds = dupload<int32_t>(ctx, seeds.data(), nchains);
-    if (!ctx->dc || !ctx->dview || !ctx->d_seeds) { shp_destroy(ctx); return SH_E_HIP; }
+    if (!ctx->dc || !ctx->dview || !ctx->dlu || !ctx->dqr || !ctx->d_seeds) { shp_destroy(ctx); return SH_E_HIP; }
     hipLaunchKernelGGL(kp_seed, dim3((nchains + 63) / 64), dim3(64), 0, ctx->st, ctx->dc, nchains, ctx->d_seeds);
     if (hipStreamSynchronize(ctx->st) != hipSuccess || hipGetLastError() != hipSuccess) {
         shp_destroy(ctx);
@@ -678,7 +699,7 @@ int shp_sweep_start_0b(shp_ctx *ctx)
     weights(ctx, 3, 0, 0);
     for (int p = 1; p <= ctx->nst; p++) {
         bmat_left_forward(ctx, ctx->wrap_step[2 * (p - 1) + 1], ctx->wrap_step[2 * (p - 1)]);
-        qr_to_t1(ctx, P_UR, 0);
+        qr_to_t1(ctx, P_UR);
         pcopy(ctx, P_UR, 0, P_T1, 0, n * ne);
         pcopy(ctx, P_UST, p, P_T1, 0, n * ne);
         weights(ctx, 4, p, 0);
@@ -735,7 +756,7 @@ int shp_sweep_b0(shp_ctx *ctx, int lupdate, int lmeasure)
                 Tic t(ctx, T_QR);
                 ptranspose(ctx, P_T2, 0, P_UL, 0, ne, n);
             }
-            qr_to_t1(ctx, P_T2, 0);
+            qr_to_t1(ctx, P_T2);
             ptranspose(ctx, P_UL, 0, P_T1, 0, n, ne);
             pcopy(ctx, P_UST, pt, P_T1, 0, n * ne);
             scratch(ctx, 2, pt);
@@ -787,7 +808,7 @@ int shp_sweep_0b(shp_ctx *ctx, int lupdate, int lmeasure, int ldyn)
             const int pt = ctx->iwrap_nt[nt];
             save_old(ctx);
             ptranspose(ctx, P_UL, 0, P_UST, pt, n, ne);
-            qr_to_t1(ctx, P_UR, 0);
+            qr_to_t1(ctx, P_UR);
             pcopy(ctx, P_UR, 0, P_T1, 0, n * ne);
             scratch(ctx, 1, pt);
             pcopy(ctx, P_UST, pt, P_UR, 0, n * ne);

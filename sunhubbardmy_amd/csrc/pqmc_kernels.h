@@ -2,13 +2,14 @@
 // unit of its own.
 #pragma once
 #include "exchange.h"
+#include "factor.h"
 #include "gemm_small.h"
 
 // scalar slots of the projective chain beyond the shared layout (SC_PHASE, SC_LOGW, SC_ZLD,
 // SC_INFO, SC_OBS ... keep their meaning)
 // (the projective sweep has no saved chain point, so SC_LDQ_SAVE's first slot holds the angle
 // sum of the on-site field's phases)
-enum { PS_RLOG = 30, PS_ISGN = 31, PS_UANG = SC_LDQ_SAVE };
+enum { PS_UANG = SC_LDQ_SAVE };
 
 enum {
     P_UR = 0, P_UL, P_ULRINV, P_ULR, P_T1, P_T2, P_ULO, P_URO, P_INV2, P_G, P_G2, P_KT, P_KTM1,
@@ -16,10 +17,10 @@ enum {
 };
 
 struct PChain {
-    int n, ne, nn_nf, nn_lf, kmode, ns, ltrot, nst, nflr, lq, pb, trace_cap;
+    int n, ne, nn_nf, nn_lf, kmode, ns, ltrot, nst, nflr, lq, trace_cap;
     cplx *UR, *UL, *ULRINV, *ULR, *T1, *T2, *ULo, *URo, *INV2, *G, *G2, *Ust, *proj;
     cplx *Rrows, *Felms, *Ginv, *Vtmp, *Utmp, *Dvec;
-    cplx *tau, *tblk, *wk, *trace;
+    cplx *tau, *tblk, *trace;
     int32_t *piv, *conf, *xvec, *ikd;
     double *unif, *sc, *logwDV, *rwork;
     uint32_t *rng;

@@ -240,64 +240,6 @@ kp_prop(const PChain *chains, POps ops)
 }
 
 // ---- stabilization --------------------------------------------------------------------------
-// s_zgeQR_pqmc (lib/s_matrix.f90:1822-1996) on the tall matrix asel (N x ne): Householder QR,
-// log|det R| and the count of negative diagonal entries of R to PS_RLOG / PS_ISGN, Q formed
-// into qsel with its first column negated for an odd count
-extern "C" __global__ void __launch_bounds__(BLK_NT)
-kp_qr_formq(const PChain *chains, int asel, int apt, int qsel, int qpt)
-{
-    extern __shared__ cplx bsh[];
-    const PChain &c = chains[blockIdx.x];
-    const int n = c.n, ne = c.ne;
-    cplx *A = pmat(c, asel, apt);
-    cplx *Q = pmat(c, qsel, qpt);
-    qr_blk_body(A, n, ne, n, c.tau, c.tblk, c.wk, c.pb, bsh);
-    __shared__ int s_neg;
-    if (threadIdx.x == 0) {
-        int neg = 0;
-        double rl = 0.0;
-        for (int i = 0; i < ne; i++) {
-            double r = A[(size_t)i + (size_t)i * n].x;
-            if (r < 0.0) { neg++; rl += log(-r); } else rl += log(r);
-        }
-        s_neg = neg;
-        c.sc[PS_RLOG] = rl;
-        c.sc[PS_ISGN] = (double)neg;
-    }
-    __syncthreads();
-    formq_blk_body(A, n, ne, n, Q, n, c.tblk, c.wk, c.pb, bsh);
-    __syncthreads();
-    if (s_neg & 1)
-        for (int i = threadIdx.x; i < n; i += blockDim.x) Q[i] = make_double2(-Q[i].x, -Q[i].y);
-}
-
-// X = A^-1 for A (ne x ne) by LU with partial pivoting (s_inv_logdet_lu_z); A is overwritten
-// by its factors; with slot >= 0 the log det goes to sc[slot], sc[slot+1]; a zero pivot is
-// recorded in sc[SC_INFO] (first zero pivot + 1, kept until the host reads it)
-extern "C" __global__ void __launch_bounds__(BLK_NT)
-kp_lu_inv(const PChain *chains, int asel, int xsel, int slot)
-{
-    extern __shared__ cplx bsh[];
-    const PChain &c = chains[blockIdx.x];
-    const int ne = c.ne;
-    cplx *A = pmat(c, asel, 0);
-    cplx *X = pmat(c, xsel, 0);
-    __shared__ cplx s_ld;
-    __shared__ double s_inf;
-    lu_blk_body(A, ne, ne, c.piv, &s_ld, &s_inf, bsh);
-    for (size_t e = threadIdx.x; e < (size_t)ne * ne; e += blockDim.x)
-        X[e] = make_double2((e % ne) == (e / ne) ? 1.0 : 0.0, 0.0);
-    __syncthreads();
-    solve_blk_body(A, ne, ne, c.piv, X, ne, ne, c.T1, bsh);
-    if (threadIdx.x == 0) {
-        if (slot >= 0) {
-            c.sc[slot] = s_ld.x;
-            c.sc[slot + 1] = s_ld.y;
-        }
-        if (s_inf != 0.0 && c.sc[SC_INFO] == 0.0) c.sc[SC_INFO] = s_inf;
-    }
-}
-
 // weight bookkeeping after a scratch inverse (z = log det ULR in SC_ZLD):
 //   op 0: sweep start  logweightf = logwDV(nst) + z, phase = exp(i nflr Im z)
 //   op 1: 0b point n   logwDV(n) = logwDV(n-1) + rlog, logw = logwDV(n) [+ logwDV(n+1)] + z
@@ -314,14 +256,14 @@ extern "C" __global__ void kp_weights(const PChain *chains, int nchains, int op,
     const cplx z = make_double2(sc[SC_ZLD], sc[SC_ZLD + 1]);
     double dv = 0.0;
     if (op == 3) { lw[0] = 0.0; return; }
-    if (op == 4) { lw[n] = lw[n - 1] + sc[PS_RLOG]; return; }
+    if (op == 4) { lw[n] = lw[n - 1] + sc[SC_RLOG]; return; }
     if (op == 0) {
         dv = lw[c.nst];
     } else if (op == 1) {
-        lw[n] = lw[n - 1] + sc[PS_RLOG];
+        lw[n] = lw[n - 1] + sc[SC_RLOG];
         dv = (n == c.nst) ? lw[n] : lw[n] + lw[n + 1];
     } else {
-        lw[n + 1] = (n + 1 == c.nst) ? sc[PS_RLOG] : lw[n + 2] + sc[PS_RLOG];
+        lw[n + 1] = (n + 1 == c.nst) ? sc[SC_RLOG] : lw[n + 2] + sc[SC_RLOG];
         dv = (n == 0) ? lw[n + 1] : lw[n + 1] + lw[n];
     }
     const cplx logw = make_double2(dv + z.x, z.y);

@@ -286,7 +286,7 @@ static void lu_factor(sh_ctx *ctx)
         const int np = (ctx->nmax + FPB - 1) / FPB, nw = fac_waves(ctx);
         for (int k = 0; k <= np; k++)
             hipLaunchKernelGGL(nw == 4 ? k_lu_step<4> : k_lu_step<8>, dim3(ctx->nch, ctx->lu_blocks[k]), dim3(64 * nw), 0,
-                               ctx->st, ctx->dc, k);
+                               ctx->st, ctx->dc, k, (int)SC_ZLD, 1);
     } else
         hipLaunchKernelGGL(k_lu, dim3(ctx->nch), dim3(1024), (size_t)ctx->nmax * 2 * sizeof(cplx), ctx->st, ctx->dc);
 }
@@ -299,9 +299,9 @@ static void lu_solve(sh_ctx *ctx, int xsel)
         // tiles hold 256 rows, eight hold 512
         const int ncb = (ctx->nmax + 15) / 16, nch8 = (ctx->nch + 7) / 8 * 8;
         if (ctx->nmax <= 256)
-            hipLaunchKernelGGL(k_solve_cb<4>, dim3(nch8 * ncb), dim3(256), 0, ctx->st, ctx->dc, ctx->nch, ncb, xsel);
+            hipLaunchKernelGGL(k_solve_cb<4>, dim3(nch8 * ncb), dim3(256), 0, ctx->st, ctx->dc, ctx->nch, ncb, xsel, 0);
         else
-            hipLaunchKernelGGL(k_solve_cb<8>, dim3(nch8 * ncb), dim3(512), 0, ctx->st, ctx->dc, ctx->nch, ncb, xsel);
+            hipLaunchKernelGGL(k_solve_cb<8>, dim3(nch8 * ncb), dim3(512), 0, ctx->st, ctx->dc, ctx->nch, ncb, xsel, 0);
     } else
         hipLaunchKernelGGL(k_lu_solve, dim3(ctx->nch), dim3(512), 0, ctx->st, ctx->dc, xsel);
 }
@@ -318,8 +318,8 @@ static void launch_qr(sh_ctx *ctx, int sel, int pivot, int pt)
 static void formq(sh_ctx *ctx, int sel, int pt)
 {
     const int ncb = (ctx->nmax + FPB - 1) / FPB, nch8 = (ctx->nch + 7) / 8 * 8, nw = fac_waves(ctx);
-    hipLaunchKernelGGL(nw == 4 ? k_formq_cb<4> : k_formq_cb<8>, dim3(nch8 * ncb), dim3(64 * nw), 0, ctx->st, ctx->dc,
-                       ctx->nch, ncb, sel, pt);
+    hipLaunchKernelGGL((nw == 4 ? k_formq_cb<4, FTW> : k_formq_cb<8, FTW>), dim3(nch8 * ncb), dim3(64 * nw), 0, ctx->st, ctx->dc,
+                       ctx->nch, ncb, sel, pt, 0);
 }
 
 // QR of W1 (first: column pivoting, from U = D = V = 1) or of the prepivoted W1 diag(D[dpt]) -> point
@@ -353,8 +353,8 @@ static void udv_step(sh_ctx *ctx, bool first, int pt, int dpt)
         if (blocked(ctx)) {
             const int np = (ctx->nmax + FPB - 1) / FPB, nw = fac_waves(ctx);
             for (int k = 0; k < np; k++)
-                hipLaunchKernelGGL(nw == 4 ? k_qr_step<4> : k_qr_step<8>, dim3(ctx->nch, np - k), dim3(64 * nw), 0, ctx->st,
-                                   ctx->dc, (int)M_W2, k, pt);
+                hipLaunchKernelGGL((nw == 4 ? k_qr_step<4, FTW> : k_qr_step<8, FTW>), dim3(ctx->nch, np - k), dim3(64 * nw), 0, ctx->st,
+                                   ctx->dc, (int)M_W2, k, pt, 0);
         } else
             launch_qr(ctx, M_W2, 0, pt);
     }
@@ -874,7 +874,6 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         c.updt = dalloc<cplx>(ctx, (size_t)UB * UB); c.updp = dalloc<int32_t>(ctx, UB + 1);
         c.tau = dalloc<cplx>(ctx, n); c.jpvt = dalloc<int32_t>(ctx, n); c.piv = dalloc<int32_t>(ctx, n);
         c.lperm = dalloc<int32_t>(ctx, n); c.lup = dalloc<int32_t>(ctx, (size_t)((n + FPB - 1) / FPB) * FLMAX);
-        c.wk = dalloc<cplx>(ctx, (size_t)PB * n);
         c.tblk = dalloc<cplx>(ctx, (size_t)(n / PB + 1) * PB * PB);
         c.rwork = dalloc<double>(ctx, 4 * (size_t)n);
         c.conf = dalloc<int32_t>(ctx, (size_t)n * q.ltrot);
@@ -888,7 +887,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         c.stag = dupload<double>(ctx, q.stag, n);
         c.sc = dalloc<double>(ctx, SC_SIZE);
         if (!c.G || !c.Gs || !c.W1 || !c.W2 || !c.W3 || !c.W4 || !c.Us || !c.Vs || !c.U || !c.V || !c.D || !c.Ds ||
-            !c.ldq || !c.avec || !c.bvec || !c.updt || !c.updp || !c.tau || !c.jpvt || !c.piv || !c.lperm || !c.lup || !c.rwork || !c.conf || !c.unif || !c.wk || !c.tblk ||
+            !c.ldq || !c.avec || !c.bvec || !c.updt || !c.updp || !c.tau || !c.jpvt || !c.piv || !c.lperm || !c.lup || !c.rwork || !c.conf || !c.unif || !c.tblk ||
             !c.rng || !c.bonds || !c.kt || !c.ktm1 || !c.stag || !c.sc) {
             int rc = fail(ctx, SH_E_HIP, "device allocation failed");
             sh_destroy(ctx);

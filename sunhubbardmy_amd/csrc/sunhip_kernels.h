@@ -84,7 +84,6 @@ struct DChain {
     cplx *updt;           // 64 x 64: T of the on-site update's current block of sites
     int32_t *updp;        // its accepted sites: count, then the sites
     cplx *tau;            // n
-    cplx *wk;             // 16 x n work block of the blocked factorizations
     cplx *tblk;           // (n/16 + 1) triangular 16 x 16 factors of the block reflectors
     int32_t *jpvt, *piv;  // n
     int32_t *lperm;       // n: row order of the LU's interchanges (row i of P X is row lperm[i] of X)
