@@ -49,7 +49,6 @@ static size_t lds_block_move(int nmax, int z)
     return (size_t)SHL_MB * SHL_MB * sizeof(cplx) + 3 * SHL_MB * sizeof(cplx) + (SHL_H + 8) * sizeof(double) +
            7 * SHL_H * sizeof(float) + (4 * SHL_MB + 16 * 12) * sizeof(int) + (size_t)(3 + z) * nmax * sizeof(int);
 }
-static size_t lds_mlp_batch() { return (size_t)(SHL_H * SHL_H + 7 * SHL_H + 8) * sizeof(float) + 2 * SHL_H * sizeof(float); }
 
 static NormF normf_of(const double *nm)
 {
@@ -240,12 +239,6 @@ int shl_create(shl_net **out, int capacity, int32_t seed, int device)
         delete ctx;
         return SH_E_HIP;
     }
-    if (hipFuncSetAttribute((const void *)k_mlp_batch, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds_mlp_batch()) != hipSuccess) {
-        (void)hipGetLastError();
-        shl_destroy(ctx);
-        return SH_E_HIP;
-    }
     // the device address of this GPU's no-allocation scratch, with the device current
     if (noalloc_setup(device, &ctx->na_scratch) != 0) {
         int rc = fail(ctx, SH_E_HIP, "hipGetSymbolAddress of the no-allocation scratch failed");
@@ -258,7 +251,7 @@ int shl_create(shl_net **out, int capacity, int32_t seed, int device)
     ctx->gout = dalloc<float>(ctx, SHL_NWT);
     ctx->gpart = dalloc<float>(ctx, (size_t)SHL_TRAIN_WG * SHL_NWT);
     ctx->lpart = dalloc<double>(ctx, SHL_TRAIN_WG);
-    ctx->dloss = dalloc<double>(ctx, 1);
+    ctx->dloss = dalloc<double>(ctx, capacity);   // one per batch of an epoch
     ctx->samp = dalloc<double>(ctx, (size_t)5 * capacity);
     ctx->perm = dalloc<int32_t>(ctx, capacity);
     if (!ctx->w || !ctx->am || !ctx->av || !ctx->gout || !ctx->gpart || !ctx->lpart || !ctx->dloss || !ctx->samp ||
@@ -379,13 +372,19 @@ int shl_clear_samples(shl_net *ctx)
     return 0;
 }
 
-// one launch pair over `count` sample indices (idx may be null: samples 0..count-1)
-static int mlp_step(shl_net *ctx, const int32_t *idx, int count, float lr, float *gout)
+// samples of a training workgroup: whole groups of SHL_MS on at most SHL_TRAIN_WG workgroups
+static int mlp_per(int count)
 {
-    const int nwg = std::min(SHL_TRAIN_WG, std::max(1, (count + 3) / 4));
-    const int per = (count + nwg - 1) / nwg;
+    const int groups = (count - 1) / SHL_MS + 1;
+    return ((groups - 1) / SHL_TRAIN_WG + 1) * SHL_MS;
+}
+
+// one launch pair over `count` sample indices (idx may be null: samples 0..count-1)
+static int mlp_step(shl_net *ctx, const int32_t *idx, int count, float lr, float *gout, double *lout)
+{
+    const int per = mlp_per(count), nwg = (count + per - 1) / per;
     NormF nm = normf_of(ctx->norm);
-    hipLaunchKernelGGL(k_mlp_batch, dim3(nwg), dim3(256), lds_mlp_batch(), ctx->st, ctx->w, ctx->samp, idx, count, per,
+    hipLaunchKernelGGL(k_mlp_batch, dim3(nwg), dim3(512), 0, ctx->st, ctx->w, ctx->samp, idx, count, per,
                        nm, 1.0f / (float)count, 0, ctx->gpart, ctx->lpart, (double *)nullptr);
     float c1 = 1.0f, c2 = 1.0f;
     if (lr > 0.f) {
@@ -394,7 +393,7 @@ static int mlp_step(shl_net *ctx, const int32_t *idx, int count, float lr, float
         c2 = (float)(1.0 / (1.0 - pow(0.999, (double)ctx->adam_t)));
     }
     hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((SHL_NWT + 255) / 256), dim3(256), 0, ctx->st, ctx->gpart, nwg,
-                       ctx->lpart, ctx->w, ctx->am, ctx->av, lr, c1, c2, gout, ctx->dloss, 1.0);
+                       ctx->lpart, ctx->w, ctx->am, ctx->av, lr, c1, c2, gout, lout, 1.0);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(ctx, SH_E_HIP, std::string("training launch: ") + hipGetErrorString(e));
     return 0;
@@ -426,6 +425,7 @@ int shl_train(shl_net *ctx, int epochs, int batch, double lr, double *loss)
         if (rc) return rc;
     }
     std::vector<int32_t> perm(ctx->count);
+    std::vector<double> bl;
     for (int ep = 0; ep < epochs; ep++) {
         for (int k = 0; k < ctx->count; k++) perm[k] = k;
         for (int k = ctx->count - 1; k > 0; k--) {
@@ -433,16 +433,18 @@ int shl_train(shl_net *ctx, int epochs, int batch, double lr, double *loss)
             std::swap(perm[k], perm[std::min(q, k)]);
         }
         HIPCHK(hipMemcpyAsync(ctx->perm, perm.data(), sizeof(int32_t) * ctx->count, hipMemcpyHostToDevice, ctx->st));
-        double tot = 0.0;
-        for (int b0 = 0; b0 < ctx->count; b0 += batch) {
-            const int nb = std::min(batch, ctx->count - b0);
-            int rc = mlp_step(ctx, ctx->perm + b0, nb, (float)lr, nullptr);
+        // every batch's loss stays on the device until the epoch is queued
+        const int nbat = (ctx->count - 1) / batch + 1;
+        for (int q = 0; q < nbat; q++) {
+            const int b0 = q * batch;
+            int rc = mlp_step(ctx, ctx->perm + b0, std::min(batch, ctx->count - b0), (float)lr, nullptr, ctx->dloss + q);
             if (rc) return rc;
-            double l = 0.0;
-            HIPCHK(hipMemcpyAsync(&l, ctx->dloss, sizeof(double), hipMemcpyDeviceToHost, ctx->st));
-            HIPCHK(hipStreamSynchronize(ctx->st));
-            tot += l;
         }
+        bl.resize(nbat);
+        HIPCHK(hipMemcpyAsync(bl.data(), ctx->dloss, sizeof(double) * nbat, hipMemcpyDeviceToHost, ctx->st));
+        HIPCHK(hipStreamSynchronize(ctx->st));
+        double tot = 0.0;
+        for (double l : bl) tot += l;
         if (loss) loss[ep] = tot / ctx->count;
     }
     HIPCHK(hipStreamSynchronize(ctx->st));
@@ -460,7 +462,7 @@ int shl_loss_grad(shl_net *ctx, const double *x, int n, double *loss, float *gra
     if (!d) return fail(ctx, SH_E_HIP, "device allocation failed");
     double *keep = ctx->samp;
     ctx->samp = d;
-    int rc = mlp_step(ctx, nullptr, n, 0.0f, ctx->gout);
+    int rc = mlp_step(ctx, nullptr, n, 0.0f, ctx->gout, ctx->dloss);
     ctx->samp = keep;
     if (rc == 0) {
         double l = 0.0;
@@ -486,9 +488,8 @@ int shl_loss_grad_noalloc(shl_net *ctx, const double *x, int n, double *loss, fl
     // scratch: gradient partials first, the loss partials after them (8-byte aligned)
     float *gpart = (float *)ctx->na_scratch;
     double *lpart = (double *)ctx->na_scratch + (SHL_NA_GFLOATS + 1) / 2;
-    const int nwg = std::min(SHL_TRAIN_WG, std::max(1, (n + 3) / 4));
-    const int per = (n + nwg - 1) / nwg;
-    hipLaunchKernelGGL(k_mlp_batch, dim3(nwg), dim3(256), lds_mlp_batch(), ctx->st, ctx->w, x, (const int32_t *)nullptr,
+    const int per = mlp_per(n), nwg = (n + per - 1) / per;
+    hipLaunchKernelGGL(k_mlp_batch, dim3(nwg), dim3(512), 0, ctx->st, ctx->w, x, (const int32_t *)nullptr,
                        n, per, normf_of(ctx->norm), 1.0f / (float)n, 0, gpart, lpart, (double *)nullptr);
     hipLaunchKernelGGL(k_mlp_reduce_adam, dim3((SHL_NWT + 255) / 256), dim3(256), 0, ctx->st, gpart, nwg, lpart,
                        ctx->w, ctx->am, ctx->av, 0.0f, 1.0f, 1.0f, grad, loss, (double)n);
@@ -508,9 +509,8 @@ int shl_predict(shl_net *ctx, const double *f, int n, double *e)
     double *d = dupload<double>(ctx, x.data(), x.size());
     double *o = dalloc<double>(ctx, n);
     if (!d || !o) return fail(ctx, SH_E_HIP, "device allocation failed");
-    const int nwg = std::min(SHL_TRAIN_WG, n);
-    const int per = (n + nwg - 1) / nwg;
-    hipLaunchKernelGGL(k_mlp_batch, dim3(nwg), dim3(256), lds_mlp_batch(), ctx->st, ctx->w, d, (const int32_t *)nullptr,
+    const int per = mlp_per(n), nwg = (n + per - 1) / per;
+    hipLaunchKernelGGL(k_mlp_batch, dim3(nwg), dim3(512), 0, ctx->st, ctx->w, d, (const int32_t *)nullptr,
                        n, per, normf_of(ctx->norm), 1.0f, 1, ctx->gpart, ctx->lpart, o);
     hipError_t err = hipGetLastError();
     if (err == hipSuccess) err = hipMemcpyAsync(e, o, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->st);

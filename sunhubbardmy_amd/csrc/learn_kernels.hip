@@ -13,7 +13,8 @@
 #define SHL_H 128
 #define SHL_NWT (SHL_H * SHL_H + 7 * SHL_H + 1)
 #define SHL_MB 64
-#define SHL_TRAIN_WG 64
+#define SHL_TRAIN_WG 64   // largest number of training workgroups
+#define SHL_MS 16         // samples of a training workgroup at a time
 enum {
     WO_W1 = 0,
     WO_B1 = 4 * SHL_H,
@@ -516,113 +517,156 @@ __global__ __launch_bounds__(256) void k_block_apply(const DChain *chains, const
 
 // ------------------------------------------------------------------------------------------
 // Training: forward and backward of the network over a minibatch in FP32.  Workgroup b
-// handles samples [b*per, min((b+1)*per, count)) of the index list and writes its gradient
-// sum (weights layout) to gpart[b] and its sum of squared errors to lpart[b].  mode 1 only
+// handles samples [b*per, min((b+1)*per, count)) of the index list, sixteen at a time, and writes its
+// gradient sum (weights layout) to gpart[b] and its sum of squared errors to lpart[b].  mode 1 only
 // evaluates: pred[k] = ymu + ysd g(x_k).
+//
+// The three products with sixteen samples, A2^T = W2 H1^T, dH1^T = W2^T dA2^T and G2 += dA2^T H1, are FP32
+// MFMA (16x16x4: lane l holds A[l%16][l/16], B[l/16][l%16], element r of D[4 (l/16) + r][l%16]).
+// Wave w has the units 16 w .. 16 w + 15 of the second layer in the first and the third and of the
+// first layer in the second product, its rows of W2 and of W2^T in registers for all its samples.
+// Bound by latencies: one group of sixteen is four barriers and 96 MFMAs per wave. A batch of 512 in
+// 32 groups: 13 us, 5 with the gradients' sum and the step; one sample at a time on 64 workgroups
+// with every product on the vector units took 55 + 6 us.
 // ------------------------------------------------------------------------------------------
 struct NormF {
     double xmu[4], xsd[4], ymu, ysd;
 };
 
-__global__ __launch_bounds__(256) void k_mlp_batch(const float *wt, const double *samp, const int32_t *idx, int count,
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(512) void k_mlp_batch(const float *wt, const double *samp, const int32_t *idx, int count,
                                                    int per, NormF nm, float scale, int mode, float *gpart,
                                                    double *lpart, double *pred)
 {
-    extern __shared__ cplx lsh[];
-    float *W2s = (float *)lsh;                 // H x H
-    float *W1s = W2s + SHL_H * SHL_H;          // 4H
-    float *b1s = W1s + 4 * SHL_H, *b2s = b1s + SHL_H, *w3s = b2s + SHL_H;
-    float *h1 = w3s + SHL_H;                   // H
-    float *da2 = h1 + SHL_H;                   // H
-    float *red = da2 + SHL_H;                  // 8
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, j = t >> 1, half = t & 1;
-    for (int k = t; k < SHL_H * SHL_H; k += 256) W2s[k] = wt[WO_W2 + k];
-    for (int k = t; k < 4 * SHL_H; k += 256) W1s[k] = wt[WO_W1 + k];
-    for (int k = t; k < SHL_H; k += 256) {
-        b1s[k] = wt[WO_B1 + k];
-        b2s[k] = wt[WO_B2 + k];
-        w3s[k] = wt[WO_W3 + k];
-    }
-    const float b3 = wt[WO_B3];
-    __syncthreads();
-    float w2r[64], g2[64];
+    __shared__ float4_t H1[SHL_MS][SHL_H / 4 + 1], DA[SHL_MS][SHL_H / 4 + 1];   // [sample][unit]
+    __shared__ float xs[5][SHL_MS], red[8][SHL_MS];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, l16 = lane & 15, q = lane >> 4;
+    const float *W2 = wt + WO_W2;
+    float fw[32], bw[32];   // W2(16 w + l16, 16 b + 4 q + i) and W2(16 b + 4 q + i, 16 w + l16) at 4 b + i
 #pragma unroll
-    for (int k = 0; k < 64; k++) {
-        w2r[k] = W2s[j * SHL_H + half * 64 + k];
-        g2[k] = 0.0f;
+    for (int b = 0; b < 8; b++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            fw[4 * b + i] = W2[(16 * w + l16) * SHL_H + 16 * b + 4 * q + i];
+            bw[4 * b + i] = W2[(16 * b + 4 * q + i) * SHL_H + 16 * w + l16];
+        }
+    const int u = t & (SHL_H - 1), j0 = 16 * w + 4 * q;   // the lane's units: u before, j0 .. j0 + 3 behind the products
+    float w1[4], b2[4], w3[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        w1[k] = wt[WO_W1 + 4 * u + k];
+        b2[k] = wt[WO_B2 + j0 + k];
+        w3[k] = wt[WO_W3 + j0 + k];
     }
-    float gw1[4] = {0.f, 0.f, 0.f, 0.f}, gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f;
+    const float b1 = wt[WO_B1 + u], b3 = wt[WO_B3];
+    float4_t g2[8] = {};
+    float gw1[4][4] = {}, gb1[4] = {}, gb2[4] = {}, gw3[4] = {}, gb3 = 0.f;
     double loss = 0.0;
     const int s0 = blockIdx.x * per, s1 = min(count, s0 + per);
-    for (int sidx = s0; sidx < s1; sidx++) {
-        const int k0 = idx ? idx[sidx] : sidx;
-        const double *sp = samp + (size_t)k0 * 5;
-        float x[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) x[k] = (float)((sp[k] - nm.xmu[k]) / nm.xsd[k]);
-        const float y = (float)((sp[4] - nm.ymu) / nm.ysd);
-        if (t < SHL_H) {
-            const float a = b1s[t] + W1s[4 * t] * x[0] + W1s[4 * t + 1] * x[1] + W1s[4 * t + 2] * x[2] + W1s[4 * t + 3] * x[3];
-            h1[t] = tanhf(a);
+    for (int g = s0; g < s1; g += SHL_MS) {
+        if (t < 5 * SHL_MS) {
+            const int s = t / 5, k = t % 5, sidx = min(g + s, s1 - 1);
+            const double v = samp[(size_t)(idx ? idx[sidx] : sidx) * 5 + k];
+            xs[k][s] = (float)((v - (k < 4 ? nm.xmu[k & 3] : nm.ymu)) / (k < 4 ? nm.xsd[k & 3] : nm.ysd));
         }
         __syncthreads();
-        const float *hh = h1 + half * 64;
-        float p0 = 0.f, p1 = 0.f;
 #pragma unroll
-        for (int k = 0; k < 64; k += 2) {
-            p0 += w2r[k] * hh[k];
-            p1 += w2r[k + 1] * hh[k + 1];
+        for (int i = 0; i < 4; i++) {
+            const int s = (t >> 7) + 4 * i;
+            const float a = b1 + w1[0] * xs[0][s] + w1[1] * xs[1][s] + w1[2] * xs[2][s] + w1[3] * xs[3][s];
+            ((float *)H1[s])[u] = tanhf(a);
         }
-        float pp = p0 + p1;
-        pp += __shfl_xor(pp, 1, 64);
-        const float h2 = tanhf(pp + b2s[j]);
-        float q = half ? 0.f : w3s[j] * h2;
-        q = wave_sum_f(q);
-        if (lane == 0) red[w] = q;
         __syncthreads();
-        const float out = b3 + ((red[0] + red[1]) + (red[2] + red[3]));
+        float4_t a = {};
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const float4_t h = H1[l16][4 * b + q];
+#pragma unroll
+            for (int i = 0; i < 4; i++) a = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[4 * b + i], h[i], a, 0, 0, 0);
+        }
+        float h2[4], po = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            h2[r] = tanhf(a[r] + b2[r]);
+            po += w3[r] * h2[r];
+        }
+        po += __shfl_xor(po, 16, 64);
+        po += __shfl_xor(po, 32, 64);
+        if (q == 0) red[w][l16] = po;
+        __syncthreads();
+        const float out = b3 + (((red[0][l16] + red[1][l16]) + (red[2][l16] + red[3][l16])) +
+                                ((red[4][l16] + red[5][l16]) + (red[6][l16] + red[7][l16])));
+        const bool in = g + l16 < s1, first = w == 0 && q == 0 && in;
         if (mode == 1) {
-            if (t == 0) pred[k0] = nm.ymu + nm.ysd * (double)out;
-            __syncthreads();
+            if (first) pred[idx ? idx[g + l16] : g + l16] = nm.ymu + nm.ysd * (double)out;
             continue;
         }
-        const float e = out - y;
-        if (t == 0) loss += (double)e * e;
-        const float dout = 2.0f * e * scale;
-        const float a2 = dout * w3s[j] * (1.0f - h2 * h2);
-        if (!half) {
-            gw3 += dout * h2;
-            gb2 += a2;
-            da2[j] = a2;
+        const float e = out - xs[4][l16], dout = in ? 2.0f * e * scale : 0.f;
+        if (first) {
+            loss += (double)e * e;
+            gb3 += dout;
         }
-        if (t == 0) gb3 += dout;
+        float4_t a2;
 #pragma unroll
-        for (int k = 0; k < 64; k++) g2[k] += a2 * hh[k];
+        for (int r = 0; r < 4; r++) {
+            a2[r] = dout * w3[r] * (1.0f - h2[r] * h2[r]);
+            gw3[r] += dout * h2[r];
+            gb2[r] += a2[r];
+        }
+        DA[l16][j0 >> 2] = a2;
         __syncthreads();
-        // dh1(k) = sum_j da2(j) W2(j, k) for k = t >> 1, the two halves of j summed by lane pairs
-        float sacc = 0.f;
-        const int kk = t >> 1;
-        for (int jj = 0; jj < 64; jj++) sacc += da2[half * 64 + jj] * W2s[(half * 64 + jj) * SHL_H + kk];
-        sacc += __shfl_xor(sacc, 1, 64);
-        const float a1 = sacc * (1.0f - h1[kk] * h1[kk]);
-        if (!half) {
-            gb1 += a1;
+        float4_t d = {};
 #pragma unroll
-            for (int k = 0; k < 4; k++) gw1[k] += a1 * x[k];
+        for (int b = 0; b < 8; b++) {
+            const float4_t x = DA[l16][4 * b + q];
+#pragma unroll
+            for (int i = 0; i < 4; i++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(bw[4 * b + i], x[i], d, 0, 0, 0);
+        }
+        const float4_t h = H1[l16][j0 >> 2];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float a1 = d[r] * (1.0f - h[r] * h[r]);
+            gb1[r] += a1;
+#pragma unroll
+            for (int k = 0; k < 4; k++) gw1[r][k] += a1 * xs[k][l16];
+        }
+#pragma unroll
+        for (int st = 0; st < SHL_MS / 4; st++) {
+            const float x = ((const float *)DA[4 * st + q])[16 * w + l16];
+#pragma unroll
+            for (int kt = 0; kt < 8; kt++)
+                g2[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, ((const float *)H1[4 * st + q])[16 * kt + l16], g2[kt], 0, 0, 0);
         }
         __syncthreads();
     }
     if (mode == 1) return;
     float *gp = gpart + (size_t)blockIdx.x * SHL_NWT;
 #pragma unroll
-    for (int k = 0; k < 64; k++) gp[WO_W2 + j * SHL_H + half * 64 + k] = g2[k];
-    if (!half) {
-        gp[WO_B2 + j] = gb2;
-        gp[WO_W3 + j] = gw3;
-        gp[WO_B1 + j] = gb1;
+    for (int kt = 0; kt < 8; kt++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) gp[WO_W1 + 4 * j + k] = gw1[k];
+        for (int r = 0; r < 4; r++) gp[WO_W2 + (j0 + r) * SHL_H + 16 * kt + l16] = g2[kt][r];
+    // the sums over the samples of a group: the sixteen lanes l16
+    auto sum16 = [](auto v) {
+        for (int o = 1; o < SHL_MS; o <<= 1) v += __shfl_xor(v, o, 64);
+        return v;
+    };
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float s1b = sum16(gb1[r]), s2b = sum16(gb2[r]), s3 = sum16(gw3[r]);
+        float sw[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) sw[k] = sum16(gw1[r][k]);
+        if (l16 == 0) {
+            gp[WO_B1 + j0 + r] = s1b;
+            gp[WO_B2 + j0 + r] = s2b;
+            gp[WO_W3 + j0 + r] = s3;
+#pragma unroll
+            for (int k = 0; k < 4; k++) gp[WO_W1 + 4 * (j0 + r) + k] = sw[k];
+        }
     }
+    gb3 = sum16(gb3);
+    loss = sum16(loss);
     if (t == 0) {
         gp[WO_B3] = gb3;
         lpart[blockIdx.x] = loss;
@@ -643,6 +687,7 @@ __global__ __launch_bounds__(256) void k_mlp_reduce_adam(const float *gpart, int
     }
     if (i >= SHL_NWT) return;
     float g = 0.f;
+#pragma unroll 16
     for (int b = 0; b < nwg; b++) g += gpart[(size_t)b * SHL_NWT + i];
     if (gout) gout[i] = g;
     if (lr > 0.f) {
