@@ -409,19 +409,26 @@ __device__ __forceinline__ void zgemm_tile(const cplx *A_, int lda, const cplx *
             }
 }
 
-// whether a launch takes the 32 x 32 form: its 64 x 64 tiles would not give every CU one.  (At few tiles a
-// product's time is that of one tile, 56 us at K = 288 against 18; with a tile for every CU the large
-// form's reuse of operands counts: at 288 tiles of K = 64 they are level.)
-__host__ inline bool gemm_small(int m, int n, int nch) { return (size_t)((m + GT - 1) / GT) * ((n + GT - 1) / GT) * nch < 256; }
+// whether a launch takes the 32 x 32 form.  Per flop it is 8 % slower (256 chains of N = 256: 702 against 648 us), so
+// it is taken where the rounds of tiles over the 256 CUs give more than that: 16 chains of N = 400 178
+// against 241 us (11 rounds of a quarter tile, 4 of a tile), eight 648 x 324 x 648 products 193 against 304
+// (8 and 3), one N = 288 chain 18 against 56.
+__host__ inline bool gemm_small(int m, int n, int nch)
+{
+    auto rounds = [=](int t) { return ((long)((m - 1) / t + 1) * ((n - 1) / t + 1) * nch - 1) / 256 + 1; };
+    return 13 * rounds(GS) < 48 * rounds(GT);
+}
 
 template <int OPA, int OPB>
 __global__ void __launch_bounds__(256, 2)
-k_zgemm_small(const DChain *chains, int selA, int ptA, int selB, int ptB, int selC, int ptC,
+k_zgemm_small(const DChain *chains, int nch, int grp, int nt, int selA, int ptA, int selB, int ptB, int selC, int ptC,
               double ar, double ai, double br, double bi)
 {
-    const DChain &c = chains[blockIdx.z];
+    int ch, tile;
+    if (!tile_of(nt * nt, nch, grp, ch, tile)) return;
+    const DChain &c = chains[ch];
     const int n = c.n;
-    const int tm = blockIdx.x * GS, tn = blockIdx.y * GS;
+    const int tm = tile % nt * GS, tn = tile / nt * GS;
     if (tm >= n || tn >= n) return;
     zgemm_small<OPA, OPB>(chain_mat(c, selA, ptA), n, chain_mat(c, selB, ptB), n, chain_mat(c, selC, ptC), n, n, n, n,
                           tm, tn, ar, ai, br, bi);
@@ -429,20 +436,22 @@ k_zgemm_small(const DChain *chains, int selA, int ptA, int selB, int ptB, int se
 
 template <int OPA, int OPB>
 __global__ void __launch_bounds__(256)
-k_zgemm(const DChain *chains, int selA, int ptA, int selB, int ptB, int selC, int ptC,
+k_zgemm(const DChain *chains, int nch, int grp, int nt, int selA, int ptA, int selB, int ptB, int selC, int ptC,
         double ar, double ai, double br, double bi)
 {
-    const DChain &c = chains[blockIdx.z];
+    int ch, tile;
+    if (!tile_of(nt * nt, nch, grp, ch, tile)) return;
+    const DChain &c = chains[ch];
     const int n = c.n;
-    const int tm = blockIdx.x * GT, tn = blockIdx.y * GT;
+    const int tm = tile % nt * GT, tn = tile / nt * GT;
     if (tm >= n || tn >= n) return;
     zgemm_tile<OPA, OPB>(chain_mat(c, selA, ptA), n, chain_mat(c, selB, ptB), n, chain_mat(c, selC, ptC), n, n, n, n,
                          tm, tn, ar, ai, br, bi);
 }
 
-template __global__ void k_zgemm<0, 0>(const DChain *, int, int, int, int, int, int, double, double, double, double);
-template __global__ void k_zgemm<1, 0>(const DChain *, int, int, int, int, int, int, double, double, double, double);
-template __global__ void k_zgemm<0, 1>(const DChain *, int, int, int, int, int, int, double, double, double, double);
+template __global__ void k_zgemm<0, 0>(const DChain *, int, int, int, int, int, int, int, int, int, double, double, double, double);
+template __global__ void k_zgemm<1, 0>(const DChain *, int, int, int, int, int, int, int, int, int, double, double, double, double);
+template __global__ void k_zgemm<0, 1>(const DChain *, int, int, int, int, int, int, int, int, int, double, double, double, double);
 
 // ------------------------------------------------------------------------------------------
 // Equal-time measurement (src/dqmc_measure/equaltime_measure.f90:1-69, zkint :71-114,

@@ -31,12 +31,10 @@ void pgemm(shp_ctx *ctx, int sa, int pa, int sb, int pb_, int sc, int pc, int m,
            int ldc, double ar = 1.0, double br = 0.0)
 {
     PGemm g{sa, pa, sb, pb_, sc, pc, m, n, k, lda, ldb, ldc, ar, 0.0, br, 0.0};
-    if (gemm_small(m, n, ctx->nch)) {
-        hipLaunchKernelGGL(kp_gemm_small, dim3((m + GS - 1) / GS, (n + GS - 1) / GS, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, g);
-        return;
-    }
-    dim3 grid((m + GT - 1) / GT, (n + GT - 1) / GT, ctx->nch);
-    hipLaunchKernelGGL(kp_gemm, grid, dim3(256), 0, ctx->st, ctx->dc, g);
+    const bool small = gemm_small(m, n, ctx->nch);
+    const int ts = small ? GS : GT, tiles = ((m - 1) / ts + 1) * ((n - 1) / ts + 1);
+    hipLaunchKernelGGL((small ? kp_gemm_small : kp_gemm), dim3(tile_grid(tiles, ctx->nch)), dim3(256), 0, ctx->st, ctx->dc,
+                       ctx->nch, tile_group(ctx->nch), g);
 }
 
 void pcopy(shp_ctx *ctx, int dsel, int dpt, int ssel, int spt, int count, int conj = 0)
@@ -157,13 +155,15 @@ void stock_decide(shp_ctx *ctx, int nt, int nf, int ib0, int nup, size_t uoff)
 
 void stock(shp_ctx *ctx, int nt, int nf, int ib0, int nup, size_t uoff)
 {
-    const int te = (ctx->ne + GS - 1) / GS, rt = (nup + GS - 1) / GS, tiles = (nup + 15) / 16;
-    hipLaunchKernelGGL(kp_stock_pre, dim3(te, 2 * rt, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nf, ib0, nup, rt);
-    hipLaunchKernelGGL(kp_stock_f, dim3(rt, rt, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nf, ib0, nup);
+    const int nch = ctx->nch, grp = tile_group(nch), tiles = (nup + 15) / 16;
+    const int te = (ctx->ne - 1) / GS + 1, te16 = (ctx->ne - 1) / 16 + 1, rt = (nup - 1) / GS + 1;
+    hipLaunchKernelGGL(kp_stock_pre, dim3(tile_grid(te16 * rt + te * tiles, nch)), dim3(256), 0, ctx->st, ctx->dc, nch, grp, nf,
+                       ib0, nup);
+    hipLaunchKernelGGL(kp_stock_f, dim3(tile_grid(tiles * tiles, nch)), dim3(256), 0, ctx->st, ctx->dc, nch, grp, nf, ib0, nup);
     (tiles == 1 ? stock_decide<1> : tiles == 2 ? stock_decide<2> : tiles == 3 ? stock_decide<3> : stock_decide<4>)(
         ctx, nt, nf, ib0, nup, uoff);
-    hipLaunchKernelGGL(kp_stock_vtmp, dim3(te, rt + 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nup, rt);
-    hipLaunchKernelGGL(kp_stock_flush, dim3(te, te, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, nup);
+    hipLaunchKernelGGL(kp_stock_vtmp, dim3(tile_grid(te * (rt + 1), nch)), dim3(256), 0, ctx->st, ctx->dc, nch, grp, nup);
+    hipLaunchKernelGGL(kp_stock_flush, dim3(tile_grid(te * te, nch)), dim3(256), 0, ctx->st, ctx->dc, nch, grp, nup);
 }
 
 // ---- update of family nf at slice nt: submatrix-LR in stocks of ns / 2 bonds (the fast form: one bond), or

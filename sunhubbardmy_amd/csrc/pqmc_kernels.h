@@ -71,7 +71,7 @@ template <int NT, int NF>
 __global__ void kp_stock_sites(const PChain *chains, int nt, int i0, int nup, size_t uoff);
 template <int NT>
 __global__ void kp_stock_bonds(const PChain *chains, int nt, int nf, int ib0, int nb, int uoff);
-extern "C" __global__ void kp_stock_pre(const PChain *chains, int nf, int ib0, int nup, int rt);
-extern "C" __global__ void kp_stock_f(const PChain *chains, int nf, int ib0, int nup);
-extern "C" __global__ void kp_stock_vtmp(const PChain *chains, int nup, int rt);
-extern "C" __global__ void kp_stock_flush(const PChain *chains, int nup);
+extern "C" __global__ void kp_stock_pre(const PChain *chains, int nch, int grp, int nf, int ib0, int nup);
+extern "C" __global__ void kp_stock_f(const PChain *chains, int nch, int grp, int nf, int ib0, int nup);
+extern "C" __global__ void kp_stock_vtmp(const PChain *chains, int nch, int grp, int nup);
+extern "C" __global__ void kp_stock_flush(const PChain *chains, int nch, int grp, int nup);

@@ -14,20 +14,26 @@ struct PGemm {
 };
 
 extern "C" __global__ void __launch_bounds__(256)
-kp_gemm(const PChain *chains, PGemm g)
+kp_gemm(const PChain *chains, int nch, int grp, PGemm g)
 {
-    const PChain &c = chains[blockIdx.z];
-    const int tm = blockIdx.x * GT, tn = blockIdx.y * GT;
+    const int mt = (g.m - 1) / GT + 1, nt = (g.n - 1) / GT + 1;
+    int ch, tile;
+    if (!tile_of(mt * nt, nch, grp, ch, tile)) return;
+    const PChain &c = chains[ch];
+    const int tm = tile % mt * GT, tn = tile / mt * GT;
     if (tm >= g.m || tn >= g.n) return;
     zgemm_tile<0, 0>(pmat(c, g.sa, g.pa), g.lda, pmat(c, g.sb, g.pb), g.ldb, pmat(c, g.sc, g.pc), g.ldc, g.m, g.n,
                      g.k, tm, tn, g.ar, g.ai, g.br, g.bi);
 }
 
 extern "C" __global__ void __launch_bounds__(256, 2)
-kp_gemm_small(const PChain *chains, PGemm g)
+kp_gemm_small(const PChain *chains, int nch, int grp, PGemm g)
 {
-    const PChain &c = chains[blockIdx.z];
-    const int tm = blockIdx.x * GS, tn = blockIdx.y * GS;
+    const int mt = (g.m - 1) / GS + 1, nt = (g.n - 1) / GS + 1;
+    int ch, tile;
+    if (!tile_of(mt * nt, nch, grp, ch, tile)) return;
+    const PChain &c = chains[ch];
+    const int tm = tile % mt * GS, tn = tile / mt * GS;
     if (tm >= g.m || tn >= g.n) return;
     zgemm_small<0, 0>(pmat(c, g.sa, g.pa), g.lda, pmat(c, g.sb, g.pb), g.ldb, pmat(c, g.sc, g.pc), g.ldc, g.m, g.n,
                       g.k, tm, tn, g.ar, g.ai, g.br, g.bi);

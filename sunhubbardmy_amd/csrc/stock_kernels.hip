@@ -10,7 +10,8 @@
 //   kp_stock_vtmp   Vtmp = T R, and UR's accepted rows times 1 + delta
 //   kp_stock_flush  (UL UR)^-1 -= Utmp Vtmp
 // Bound by latencies: a product's workgroup streams its 32 x 32 tile's operands once from L2, and the decisions are
-// a serial chain.  A stock of 64 sites, eight chains of N = 648, ne = 324: 39 + 18 + 36 + 10 + 19 us.  Before:
+// a serial chain.  A stock of 64 sites, eight chains of N = 648, ne = 324: 25 + 8 + 35 + 7 + 17 us (39, 18, 10 and
+// 19 us for the products in 32 x 32 tiles dealt out without regard to the XCDs).  Before:
 // gathers, five products of 57 us each on 64 x 64 tiles and 162 us of decisions bordering Gamma^-1 one
 // bond at a time, with the whole F and Gamma^-1 in LDS.
 #include "pqmc_kernels.h"
@@ -22,45 +23,53 @@ __device__ __forceinline__ int stock_site(const PChain &c, int nf, int ib0, int 
     return gp(c.bonds)[2 * (nf * c.nn_lf + ib0) + s];
 }
 
-// grid: x tiles of ne, y < rt row tiles of R, then the same number of column tiles of Utmp
+// tiles: the 32 x 16 tiles of R, row by row of tiles, then those of Utmp
 extern "C" __global__ void __launch_bounds__(256, 2)
-kp_stock_pre(const PChain *chains, int nf, int ib0, int nup, int rt)
+kp_stock_pre(const PChain *chains, int nch, int grp, int nf, int ib0, int nup)
 {
-    const PChain &c = chains[blockIdx.z];
-    const int n = c.n, ne = c.ne, ns = c.ns, l16 = threadIdx.x & 15, t0 = blockIdx.x * GS;
-    const bool left = (int)blockIdx.y < rt;
-    const int s0 = ((int)blockIdx.y - (left ? 0 : rt)) * GS;
-    const int sa = stock_site(c, nf, ib0, min(s0 + l16, nup - 1)), sb = stock_site(c, nf, ib0, min(s0 + 16 + l16, nup - 1));
+    const int ne0 = chains[0].ne, rt = (nup - 1) / 32 + 1, te16 = (ne0 - 1) / 16 + 1, te32 = (ne0 - 1) / 32 + 1;
+    int ch, tile;
+    if (!tile_of(rt * te16 + ((nup - 1) / 16 + 1) * te32, nch, grp, ch, tile)) return;
+    const PChain &c = chains[ch];
+    const int n = c.n, ne = c.ne, ns = c.ns, l16 = threadIdx.x & 15;
     GAS cplx *UR = gp(c.UR), *UL = gp(c.UL), *I = gp(c.ULRINV);
-    if (left) {
+    if (tile < rt * te16) {
+        const int s0 = tile / te16 * 32, t0 = tile % te16 * 16;
+        const int sa = stock_site(c, nf, ib0, min(s0 + l16, nup - 1)), sb = stock_site(c, nf, ib0, min(s0 + 16 + l16, nup - 1));
         GAS cplx *R = gp(c.Rrows);
-        gemm_small_tile(
+        gemm_small_tile<2, 1>(
             ne, [=](int i, int k) { return gld(UR + ((size_t)(i < 16 ? sa : sb) + (size_t)k * n)); },
             [=](int k, int j) { return gld(I + ((size_t)k + (size_t)min(t0 + j, ne - 1) * ne)); },
             [=](int i, int j, cplx v) {
                 if (s0 + i < nup && t0 + j < ne) gst(R + ((size_t)(s0 + i) + (size_t)(t0 + j) * ns), v);
             });
     } else {
+        const int q = tile - rt * te16, t0 = q % te32 * 32, s0 = q / te32 * 16;
+        const int sa = stock_site(c, nf, ib0, min(s0 + l16, nup - 1));
         GAS cplx *U = gp(c.Utmp);
-        gemm_small_tile(
+        gemm_small_tile<2, 1>(
             ne, [=](int i, int k) { return gld(I + ((size_t)min(t0 + i, ne - 1) + (size_t)k * ne)); },
-            [=](int k, int j) { return gld(UL + ((size_t)k + (size_t)(j < 16 ? sa : sb) * ne)); },
+            [=](int k, int j) { return gld(UL + ((size_t)k + (size_t)sa * ne)); },
             [=](int i, int j, cplx v) {
                 if (t0 + i < ne && s0 + j < nup) gst(U + ((size_t)(t0 + i) + (size_t)(s0 + j) * ne), v);
             });
     }
 }
 
+// 16 x 16 tiles: at 64 x 64 x 324 four times as many as of 32 x 32, each a quarter of the chain of MFMAs
 extern "C" __global__ void __launch_bounds__(256, 2)
-kp_stock_f(const PChain *chains, int nf, int ib0, int nup)
+kp_stock_f(const PChain *chains, int nch, int grp, int nf, int ib0, int nup)
 {
-    const PChain &c = chains[blockIdx.z];
-    const int ne = c.ne, ns = c.ns, l16 = threadIdx.x & 15, tm = blockIdx.x * GS, tn = blockIdx.y * GS;
-    const int sa = stock_site(c, nf, ib0, min(tn + l16, nup - 1)), sb = stock_site(c, nf, ib0, min(tn + 16 + l16, nup - 1));
+    const int nt = (nup - 1) / 16 + 1;
+    int ch, tile;
+    if (!tile_of(nt * nt, nch, grp, ch, tile)) return;
+    const PChain &c = chains[ch];
+    const int ne = c.ne, ns = c.ns, l16 = threadIdx.x & 15, tm = tile % nt * 16, tn = tile / nt * 16;
+    const int sa = stock_site(c, nf, ib0, min(tn + l16, nup - 1));
     GAS cplx *R = gp(c.Rrows), *UL = gp(c.UL), *F = gp(c.Felms);
-    gemm_small_tile(
+    gemm_small_tile<1, 1>(
         ne, [=](int i, int k) { return gld(R + ((size_t)min(tm + i, nup - 1) + (size_t)k * ns)); },
-        [=](int k, int j) { return gld(UL + ((size_t)k + (size_t)(j < 16 ? sa : sb) * ne)); },
+        [=](int k, int j) { return gld(UL + ((size_t)k + (size_t)sa * ne)); },
         [=](int i, int j, cplx v) {
             if (tm + i < nup && tn + j < nup) gst(F + ((size_t)(tm + i) + (size_t)(tn + j) * ns), v);
         });
@@ -151,14 +160,17 @@ kp_stock_bonds(const PChain *chains, int nt, int nf, int ib0, int nb, int uoff)
     exchange_block<NT, false, true, 1>(p, 2 * nb, 1, make_double2(c.sc[SC_PHASE], c.sc[SC_PHASE + 1]));
 }
 
-// grid: x tiles of ne, y < rt row tiles of Vtmp, y = rt the rows of UR: UR(x_m, :) += D_m UR(x_m, :)
+// tiles: those of Vtmp, then 32 columns of UR each: UR(x_m, :) += D_m UR(x_m, :)
 // (dqmc_proj_update_submatrix_LR.f90:249-254)
 extern "C" __global__ void __launch_bounds__(256, 2)
-kp_stock_vtmp(const PChain *chains, int nup, int rt)
+kp_stock_vtmp(const PChain *chains, int nch, int grp, int nup)
 {
-    const PChain &c = chains[blockIdx.z];
-    const int n = c.n, ne = c.ne, ns = c.ns, t0 = blockIdx.x * GS, s0 = blockIdx.y * GS;
-    if ((int)blockIdx.y == rt) {
+    const int te = (chains[0].ne - 1) / GS + 1, rt = (nup - 1) / GS + 1;
+    int ch, tile;
+    if (!tile_of(te * (rt + 1), nch, grp, ch, tile)) return;
+    const PChain &c = chains[ch];
+    const int n = c.n, ne = c.ne, ns = c.ns, t0 = tile % te * GS, s0 = tile / te * GS;
+    if (tile >= te * rt) {
         const int ik = c.ikd[0];
         GAS cplx *UR = gp(c.UR);
         for (int e = threadIdx.x; e < ik * GS; e += 256) {
@@ -172,7 +184,7 @@ kp_stock_vtmp(const PChain *chains, int nup, int rt)
         return;
     }
     GAS cplx *T = gp(c.Ginv), *R = gp(c.Rrows), *V = gp(c.Vtmp);
-    gemm_small_tile(
+    gemm_small_tile<2, 2>(
         nup, [=](int i, int k) { return gld(T + ((size_t)min(s0 + i, nup - 1) + (size_t)k * ns)); },
         [=](int k, int j) { return gld(R + ((size_t)k + (size_t)min(t0 + j, ne - 1) * ns)); },
         [=](int i, int j, cplx v) {
@@ -181,11 +193,14 @@ kp_stock_vtmp(const PChain *chains, int nup, int rt)
 }
 
 extern "C" __global__ void __launch_bounds__(256, 2)
-kp_stock_flush(const PChain *chains, int nup)
+kp_stock_flush(const PChain *chains, int nch, int grp, int nup)
 {
-    const PChain &c = chains[blockIdx.z];
+    const int te = (chains[0].ne - 1) / GS + 1;
+    int ch, tile;
+    if (!tile_of(te * te, nch, grp, ch, tile)) return;
+    const PChain &c = chains[ch];
     const int ne = c.ne;
-    zgemm_small<0, 0>(c.Utmp, ne, c.Vtmp, c.ns, c.ULRINV, ne, ne, ne, nup, blockIdx.x * GS, blockIdx.y * GS, -1.0, 0.0, 1.0, 0.0);
+    zgemm_small<0, 0>(c.Utmp, ne, c.Vtmp, c.ns, c.ULRINV, ne, ne, ne, nup, tile % te * GS, tile / te * GS, -1.0, 0.0, 1.0, 0.0);
 }
 
 #define STOCK(NT)                                                                              \

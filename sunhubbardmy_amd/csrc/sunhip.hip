@@ -189,15 +189,10 @@ template <int OPA, int OPB>
 static void gemm(sh_ctx *ctx, int selA, int ptA, int selB, int ptB, int selC, int ptC, double ar = 1.0,
                  double br = 0.0)
 {
-    if (gemm_small(ctx->nmax, ctx->nmax, ctx->nch)) {
-        const unsigned ns = (ctx->nmax + GS - 1) / GS;
-        hipLaunchKernelGGL((k_zgemm_small<OPA, OPB>), dim3(ns, ns, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, selA, ptA,
-                           selB, ptB, selC, ptC, ar, 0.0, br, 0.0);
-        return;
-    }
-    unsigned nb = (ctx->nmax + GT - 1) / GT;
-    hipLaunchKernelGGL((k_zgemm<OPA, OPB>), dim3(nb, nb, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, selA, ptA, selB,
-                       ptB, selC, ptC, ar, 0.0, br, 0.0);
+    const bool small = gemm_small(ctx->nmax, ctx->nmax, ctx->nch);
+    const int nt = (ctx->nmax - 1) / (small ? GS : GT) + 1;
+    hipLaunchKernelGGL((small ? k_zgemm_small<OPA, OPB> : k_zgemm<OPA, OPB>), dim3(tile_grid(nt * nt, ctx->nch)), dim3(256), 0,
+                       ctx->st, ctx->dc, ctx->nch, tile_group(ctx->nch), nt, selA, ptA, selB, ptB, selC, ptC, ar, 0.0, br, 0.0);
 }
 
 static void copy_mat(sh_ctx *ctx, int dsel, int dpt, int ssel, int spt)

@@ -1,5 +1,5 @@
 """The 32 x 32 form of the chains' products (csrc/gemm_small.h) at the edges of its tiles and of its steps of
-64 along K, one chain and uneven batches, and on both sides of the launch rule (256 large tiles).
+64 along K, one chain and uneven batches, and on both sides of the launch rule.
 
 Bound: sums of N products of entries of order one, 4 N eps of N's worst sum ~ 1e-13 of the largest entry."""
 import ctypes
