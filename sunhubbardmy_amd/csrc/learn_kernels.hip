@@ -54,6 +54,12 @@ __host__ __device__ __forceinline__ uint64_t smix_next(uint64_t &s)
 __host__ __device__ __forceinline__ double smix_unif(uint64_t &s) { return (double)(smix_next(s) >> 11) * 0x1.0p-53; }
 static inline uint64_t smix_seed(int32_t seed) { return 0x9E3779B97F4A7C15ull * (uint64_t)(uint32_t)seed + 0x632BE59BD9B4E019ull; }
 
+// lane p's value (p the same in every lane)
+__device__ __forceinline__ double readlane_d(double v, int p)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), p), __builtin_amdgcn_readlane(__double2loint(v), p));
+}
+
 __device__ __forceinline__ int wave_sum_i(int v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -189,13 +195,14 @@ __global__ __launch_bounds__(64) void k_prop_features(const DChain *chains, cons
 //  1. stage the spins of slices nt-1, nt, nt+1; refresh the partial sums the local update
 //     changed; totals -> features -> g0
 //  2. nprop Metropolis attempts on E_eff at uniform sites of slice nt (spins in LDS only)
-//  3. F = flipped sites; M = 1 + Delta_F (1 - G)_FF; Gauss-Jordan inverse with partial
-//     pivoting gives det M and M^-1
+//  3. F = flipped sites; M = 1 + Delta_F (1 - G)_FF; Gauss-Jordan inverse in registers with partial
+//     pivoting gives det M and M^-1 (a launch with 64 attempts and 54 flipped sites 444 -> 243 us, of
+//     which the attempts are 108; in LDS, with three barriers and a search by shuffles a step, it took 228)
 //  4. accept with min(1, |Re(R phase)| / |Re(phase)| exp(E_eff(C') - E_eff(C))),
 //     R = det(M)^nflr prod qf
 //  5. on accept G <- G - G_:F M^-1 Delta_F (E_F - G_F:) as a rank-|F| MFMA update, flip the
 //     field, rotate the phase
-// LDS: 3n spins, the neighbour lists, M (64 x 64), pivot rows/columns, network vectors and
+// LDS: 3n spins, the neighbour lists, M^-1 (64 x 64), pivot columns, network vectors and
 // small weights.
 // ------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_block_move(const DChain *chains, const PropChain *props, PropNet pn, int nt)
@@ -206,18 +213,17 @@ __global__ __launch_bounds__(256) void k_block_move(const DChain *chains, const 
     const int n = c.n, lt = c.ltrot, z = p.z, t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int tau = nt - 1, tm = (tau + lt - 1) % lt, tp = (tau + 1) % lt;
     cplx *Mm = (cplx *)lsh;                         // 64 x 64, leading dimension 64
-    cplx *rowk = Mm + SHL_MB * SHL_MB;              // 64
-    cplx *colk = rowk + SHL_MB;                     // 64
-    cplx *dl = colk + SHL_MB;                       // 64: Delta of each flipped site
+    cplx *colk = Mm + SHL_MB * SHL_MB;              // 2 x 64
+    cplx *pvs = colk + 2 * SHL_MB;                  // 64: pivots
+    cplx *dl = pvs + SHL_MB;                        // 64: Delta of each flipped site
     double *h1 = (double *)(dl + SHL_MB);           // 128
     double *red = h1 + SHL_H;                       // 8
     float *W1s = (float *)(red + 8);                // 4H
     float *b1s = W1s + 4 * SHL_H, *b2s = b1s + SHL_H, *w3s = b2s + SHL_H;
     int *F = (int *)(w3s + SHL_H);                  // 64
     int *isF = F + SHL_MB;                          // 64: field value before the move
-    int *piv = isF + SHL_MB;                        // 64
-    int *cols = piv + SHL_MB;                       // 64
-    int *iscr = cols + SHL_MB;                      // 16 * 12
+    int *prow = isF + SHL_MB;                       // 64: pivot rows
+    int *iscr = prow + SHL_MB;                      // 16 * 12
     int *R = iscr + 16 * 12;                        // 3n spins (+-1): slices tm, tau, tp
     int *nb = R + 3 * n;                            // n * z neighbour lists
     int32_t *cf = c.conf + (size_t)tau * n;
@@ -333,77 +339,86 @@ __global__ __launch_bounds__(256) void k_block_move(const DChain *chains, const 
     const int m = min(iscr[0], SHL_MB);
     bool acc = false;
     cplx unit = make_double2(1.0, 0.0);
+    // Gauss-Jordan in place with M in registers: lane i of wave w has row i of the columns 16 w .. 16 w + 15.  Rows stay
+    // where they are: step k takes the largest entry of column k among the rows not yet used, prow[k], as its pivot
+    // (one barrier a step), and the end holds M^-1(k, prow[j]) in row prow[k], column j.
+    cplx mx[16];
+    int kstep = 0;          // the step that used this lane's row
     if (m > 0) {
         for (int a = t; a < m; a += 256) dl[a] = c.delta_bmat[isF[a] - 1];
         __syncthreads();
-        for (int e = t; e < m * m; e += 256) {
-            const int a = e % m, b = e / m;
-            const cplx g = G[(size_t)F[a] + (size_t)F[b] * n];
-            cplx val = cmul(dl[a], make_double2((a == b ? 1.0 : 0.0) - g.x, -g.y));
-            if (a == b) val.x += 1.0;
-            Mm[a + b * SHL_MB] = val;
+        {
+            const int a = min(lane, m - 1);
+            const cplx da = dl[a];
+            GAS cplx *Gg = gp(G) + F[a];
+#pragma unroll
+            for (int r = 0; r < 16; r++) mx[r] = gld(Gg + (size_t)F[min(16 * w + r, m - 1)] * n);
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int b = 16 * w + r;
+                cplx val = cmul(da, make_double2((a == b ? 1.0 : 0.0) - mx[r].x, -mx[r].y));
+                if (a == b) val.x += 1.0;
+                mx[r].x = lane < m && b < m ? val.x : 0.0;
+                mx[r].y = lane < m && b < m ? val.y : 0.0;
+            }
+        }
+        unsigned long long open = m < 64 ? (1ull << m) - 1 : ~0ull;     // rows not yet used
+        int nswap = 0;      // inversions of the pivot order
+        bool sing = false;
+        for (int kw = 0; 16 * kw < m; kw++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int k = 16 * kw + r, par = r & 1;
+                if (k < m) {
+                    if (w == kw) {
+                        double best = open >> lane & 1 ? cabs2(mx[r]) : -1.0;
+                        int bi = lane;
+                        wave_argmax_dpp(best, bi);
+                        colk[par * SHL_MB + lane] = mx[r];
+                        // (without a comparable entry: the first row not yet used)
+                        if (lane == 0) prow[k] = open >> bi & 1 ? bi : __ffsll((long long)open) - 1;
+                    }
+                    __syncthreads();
+                    const int p = __builtin_amdgcn_readfirstlane(prow[k]);
+                    const cplx pv = colk[par * SHL_MB + p], ci = colk[par * SHL_MB + lane];
+                    const bool zero = (pv.x == 0.0 && pv.y == 0.0), own = lane == p;
+                    sing = sing || zero;
+                    const cplx pinv = zero ? make_double2(0.0, 0.0) : cinv(pv);
+                    cplx g = cmul(ci, pinv);
+                    g.x = own ? -pinv.x : g.x;
+                    g.y = own ? -pinv.y : g.y;
+                    if (t == 0) pvs[k] = pv;
+                    // row i -= (its column k entry / pivot) row p, row p /= pivot, and column k of M^-1
+#pragma unroll
+                    for (int q = 0; q < 16; q++) {
+                        const cplx rp = make_double2(readlane_d(mx[q].x, p), readlane_d(mx[q].y, p));
+                        const double bx = own ? 0.0 : mx[q].x, by = own ? 0.0 : mx[q].y;
+                        mx[q].x = fma(-g.x, rp.x, fma(g.y, rp.y, bx));
+                        mx[q].y = fma(-g.x, rp.y, fma(-g.y, rp.x, by));
+                    }
+                    if (w == kw) mx[r] = make_double2(-g.x, -g.y);
+                    kstep = own ? k : kstep;
+                    nswap += __popcll(open & ((1ull << p) - 1));
+                    open &= ~(1ull << p);
+                }
+            }
         }
         __syncthreads();
-        // in-place Gauss-Jordan with row interchanges
+        // det M = (-1)^nswap prod of the pivots; prod qf in the order of the sites
         double ldr = 0.0, ldi = 0.0;
-        int nswap = 0;
-        bool sing = false;
-        for (int k = 0; k < m; k++) {
-            if (w == 0) {
-                double best = -1.0;
-                int bi = k;
-                if (k + lane < m) {
-                    best = cabs2(Mm[(k + lane) + k * SHL_MB]);
-                    bi = k + lane;
-                }
-                for (int o = 32; o > 0; o >>= 1) {
-                    const double ob = __shfl_xor(best, o, 64);
-                    const int oi = __shfl_xor(bi, o, 64);
-                    if (ob > best || (ob == best && oi < bi)) {
-                        best = ob;
-                        bi = oi;
-                    }
-                }
-                if (bi != k)
-                    for (int q = lane; q < m; q += 64) {
-                        const cplx tmp = Mm[k + q * SHL_MB];
-                        Mm[k + q * SHL_MB] = Mm[bi + q * SHL_MB];
-                        Mm[bi + q * SHL_MB] = tmp;
-                    }
-                if (lane == 0) piv[k] = bi;
+        if (lane < m) {
+            const cplx pv = pvs[lane];
+            if (pv.x != 0.0 || pv.y != 0.0) {
+                ldr = 0.5 * log(cabs2(pv));
+                ldi = atan2(pv.y, pv.x);
             }
-            __syncthreads();
-            if (piv[k] != k) nswap++;
-            const cplx pv = Mm[k + k * SHL_MB];
-            const bool zero = (pv.x == 0.0 && pv.y == 0.0);
-            sing = sing || zero;
-            if (!zero) {
-                ldr += 0.5 * log(cabs2(pv));
-                ldi += atan2(pv.y, pv.x);
-            }
-            const cplx pinv = zero ? make_double2(0.0, 0.0) : cinv(pv);
-            for (int q = t; q < m; q += 256) {
-                rowk[q] = (q == k) ? pinv : cmul(Mm[k + q * SHL_MB], pinv);
-                colk[q] = Mm[q + k * SHL_MB];
-            }
-            __syncthreads();
-            for (int e = t; e < m * m; e += 256) {
-                const int i = e % m, q = e / m;
-                if (i == k) {
-                    Mm[k + q * SHL_MB] = rowk[q];
-                } else {
-                    const cplx base = (q == k) ? make_double2(0.0, 0.0) : Mm[i + q * SHL_MB];
-                    Mm[i + q * SHL_MB] = csub(base, cmul(colk[i], rowk[q]));
-                }
-            }
-            __syncthreads();
         }
-        // ratiotot = det(M)^nflr prod qf; det(M) = (-1)^nswap exp(ldr + i ldi)
+        ldr = wave_sum(ldr);
+        ldi = wave_sum(ldi);
+        const cplx qf1 = cscale(c.phase_ratio[0], c.gaml[1] / c.gaml[0]), qf2 = cscale(c.phase_ratio[1], c.gaml[0] / c.gaml[1]);
+        const unsigned long long one = __ballot(lane < m && isF[min(lane, m - 1)] == 1);
         cplx qprod = make_double2(1.0, 0.0);
-        for (int a = 0; a < m; a++) {
-            const int is = isF[a], isp = 3 - is;
-            qprod = cmul(qprod, cscale(c.phase_ratio[is - 1], c.gaml[isp - 1] / c.gaml[is - 1]));
-        }
+        for (int a = 0; a < m; a++) qprod = cmul(qprod, one >> a & 1 ? qf1 : qf2);
         const double th = c.nflr * (ldi + ((nswap & 1) ? M_PI : 0.0)) + atan2(qprod.y, qprod.x);
         const double lmag = c.nflr * ldr + 0.5 * log(cabs2(qprod));
         unit = make_double2(cos(th), sin(th));
@@ -413,15 +428,10 @@ __global__ __launch_bounds__(256) void k_block_move(const DChain *chains, const 
         acc = !sing && pr > 0.0 && log(u3) < lacc;
     }
     if (acc) {
-        // column order of M^-1: the row interchanges undone on the columns, last first
-        if (t == 0) {
-            for (int j = 0; j < m; j++) cols[j] = j;
-            for (int l = m - 1; l >= 0; l--) {
-                const int q = piv[l], tmp = cols[l];
-                cols[l] = cols[q];
-                cols[q] = tmp;
-            }
-        }
+        if (lane < m)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (16 * w + r < m) Mm[kstep + prow[16 * w + r] * SHL_MB] = mx[r];
         __syncthreads();
         // pa = -G_:F M^-1 (n x m), 16 columns per item; the item's m entries of G are loaded
         // eight at a time ahead of their use (clamped addresses), the sums in the order b = 0, 1, ...
@@ -444,7 +454,7 @@ __global__ __launch_bounds__(256) void k_block_move(const DChain *chains, const 
 #pragma unroll
                         for (int q = 0; q < 16; q++) {
                             const int col = min(g0i + q, m - 1);
-                            const cplx mi = Mm[b + cols[col] * SHL_MB];
+                            const cplx mi = Mm[b + col * SHL_MB];
                             ar[q] += gb.x * mi.x - gb.y * mi.y;
                             ai[q] += gb.x * mi.y + gb.y * mi.x;
                         }
