@@ -376,17 +376,31 @@ static void vprop(sh_ctx *ctx, int sel, int nf, int mode, int side, int nt)
     const unsigned nb = (unsigned)(((size_t)ctx->nmax * ctx->nmax / 2 + 255) / 256);   // n nn_lf <= n^2 / 2
     hipLaunchKernelGGL(k_vprop, dim3(nb, 1, ctx->nch), dim3(256), 0, ctx->st, ctx->dc, sel, 0, nf, mode, side, nt);
 }
+// G += G(:, P) T (G(P, :) - E_P) of the block whose decisions stand in updt and updp.  The panel takes the 32 x 32 tiles
+// by rounds of the CUs like the products (16 chains of N = 400 16 -> 9.5 us).  The flush, with its loads and
+// stores of G, only where the 64 x 64 tiles leave CUs without one: one N = 288 chain (25 tiles) 11.7 -> 6.5 us,
+// but 16 chains of N = 400 (784 tiles) 33 -> 42.
+static void upd_apply(hipStream_t st, const DChain *dc, int nch, int nmax, int s0)
+{
+    const int ntl = (nmax - 1) / GT + 1, nts = (nmax - 1) / GS + 1, grp = tile_group(nch);
+    if (gemm_small(nmax, GT, nch))
+        hipLaunchKernelGGL(k_upd_panel_small, dim3(tile_grid(2 * nts, nch)), dim3(256), 0, st, dc, nch, grp, nts, s0);
+    else
+        hipLaunchKernelGGL(k_upd_panel, dim3(ntl, 1, nch), dim3(256), 0, st, dc, s0);
+    if (ntl * ntl * nch < 256)
+        hipLaunchKernelGGL(k_upd_flush_small, dim3(tile_grid(nts * nts, nch)), dim3(256), 0, st, dc, nch, grp, nts, s0);
+    else
+        hipLaunchKernelGGL(k_upd_flush, dim3((nch + 7) / 8 * 8 * ntl * ntl), dim3(256), 0, st, dc, nch, ntl, s0);
+}
 // the bond update of family nf (update_kernels.hip), for the chains of either sweep: three launches per
 // block of at most UB / 2 bonds, the blocks as even as they come.  nl: the largest chain's bonds per family
 static void bond_update(hipStream_t st, const DChain *dc, int nch, int nmax, int nl, int nt, int nf, int slice, int p)
 {
     const int nblk = (nl + UB / 2 - 1) / (UB / 2), per = (nl + nblk - 1) / nblk, tiles = (2 * per + 15) / 16;
-    const int ntl = (nmax + GT - 1) / GT, nch8 = (nch + 7) / 8 * 8;
     auto k = tiles == 1 ? k_upd_bonds<1> : tiles == 2 ? k_upd_bonds<2> : tiles == 3 ? k_upd_bonds<3> : k_upd_bonds<4>;
     for (int ib0 = 0; ib0 < nl; ib0 += per) {
         hipLaunchKernelGGL(k, dim3(nch), dim3(64 * tiles), 0, st, dc, nt, nf, slice, p, ib0, per);
-        hipLaunchKernelGGL(k_upd_panel, dim3(ntl, 1, nch), dim3(256), 0, st, dc, 0);
-        hipLaunchKernelGGL(k_upd_flush, dim3(nch8 * ntl * ntl), dim3(256), 0, st, dc, nch, ntl, 0);
+        upd_apply(st, dc, nch, nmax, 0);
     }
 }
 static void vupdate(sh_ctx *ctx, int nt, int nf, int slice, int p)
@@ -617,11 +631,9 @@ static void site_update(hipStream_t st, const DChain *dc, int nch, int nmax, boo
         (flav2 ? launch_sites<true, 2> : launch_sites<true, 0>)(st, dc, nch, nmax, nt, slice, 0);
         return;
     }
-    const int ntl = (nmax + GT - 1) / GT, nch8 = (nch + 7) / 8 * 8;
     for (int s0 = 0; s0 < nmax; s0 += UB) {
         (flav2 ? launch_sites<false, 2> : launch_sites<false, 0>)(st, dc, nch, std::min(UB, nmax - s0), nt, slice, s0);
-        hipLaunchKernelGGL(k_upd_panel, dim3(ntl, 1, nch), dim3(256), 0, st, dc, s0);
-        hipLaunchKernelGGL(k_upd_flush, dim3(nch8 * ntl * ntl), dim3(256), 0, st, dc, nch, ntl, s0);
+        upd_apply(st, dc, nch, nmax, s0);
     }
 }
 

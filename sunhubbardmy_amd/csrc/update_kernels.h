@@ -8,3 +8,5 @@ template <int NT>
 __global__ void k_upd_bonds(const DChain *chains, int nt, int nf, int slice, int p, int ib0, int per);
 extern "C" __global__ void k_upd_panel(const DChain *chains, int s0);
 extern "C" __global__ void k_upd_flush(const DChain *chains, int nch, int nt, int s0);
+extern "C" __global__ void k_upd_panel_small(const DChain *chains, int nch, int grp, int nt, int s0);
+extern "C" __global__ void k_upd_flush_small(const DChain *chains, int nch, int grp, int nt, int s0);

@@ -20,6 +20,7 @@
 // chip.  Per slice: one N = 288 chain 1.72 -> 0.27 ms, 72 chains of N = 64, 144, 256 0.90 -> 0.29 ms,
 // 256 chains of N = 256 1.20 -> 0.95 ms (per block 40 us of decisions, 55 us of panels, 140 us of
 // flush; one read and write of the 256 MiB of G takes 111 us), 16 chains of N = 64 172 -> 31 us.
+#include "gemm_small.h"
 #include "update_kernels.h"
 
 // the decisions of sites s0 .. of one chain on G; WHOLE: n <= 64 and s0 = 0
@@ -233,13 +234,64 @@ k_upd_flush(const DChain *chains, int nch, int nt, int s0)
             }
 }
 
+// The same two products on 32 x 32 tiles with K split over the waves, where those need fewer rounds of the CUs: a
+// 64 x 64 x 64 tile is 8 us of one CU's MFMAs, whatever else is idle.  One N = 288 chain: panel 13.8 -> 7.1 us,
+// flush 11.7 -> 6.5; 16 of N = 72 12.1 -> 6.3 and 9.7 -> 6.2; 16 of N = 400 the panel 16 -> 9.5.
+// A workgroup of the panel forms a tile of A, its share (half of the tile's 32 columns) of V on the way.
+extern "C" __global__ void __launch_bounds__(256, 2)
+k_upd_panel_small(const DChain *chains, int nch, int grp, int nt, int s0)
+{
+    __shared__ int P[UB];
+    int ch, tile;
+    if (!tile_of(2 * nt, nch, grp, ch, tile)) return;
+    const DChain &c = chains[ch];
+    const int n = c.n, i0 = (tile >> 1) * GS, h = tile & 1;
+    if (s0 >= n || i0 >= n) return;
+    const int ka = c.updp[0];
+    if (ka <= 0) return;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    if (t < UB) P[t] = c.updp[1 + min(t, ka - 1)];
+    __syncthreads();
+    GAS cplx *G = gp(c.G), *V = gp(c.bvec), *A = gp(c.avec), *T = gp(c.updt);
+    const int pm = P[lane], j0 = i0 + 16 * h + w;
+    cplx v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = gld(G + ((size_t)pm + (size_t)min(j0 + 4 * q, n - 1) * n));
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int j = j0 + 4 * q;
+        if (pm == j) v[q].x -= 1.0;
+        if (lane < ka && j < n) gst(V + ((size_t)j * UB + lane), v[q]);
+    }
+    if (GS * h >= ka) return;
+    gemm_small_tile<2, 2>(
+        ka, [=](int i, int k) { return gld(G + ((size_t)min(i0 + i, n - 1) + (size_t)P[k] * n)); },
+        [=](int k, int j) { return gld(T + (k + UB * min(GS * h + j, ka - 1))); },
+        [=](int i, int j, cplx a) {
+            if (i0 + i < n && GS * h + j < ka) gst(A + ((size_t)(i0 + i) + (size_t)(GS * h + j) * n), a);
+        });
+}
+
+extern "C" __global__ void __launch_bounds__(256, 2)
+k_upd_flush_small(const DChain *chains, int nch, int grp, int nt, int s0)
+{
+    int ch, tile;
+    if (!tile_of(nt * nt, nch, grp, ch, tile)) return;
+    const DChain &c = chains[ch];
+    const int n = c.n, i0 = tile % nt * GS, j0 = tile / nt * GS;
+    if (s0 >= n || i0 >= n || j0 >= n) return;
+    const int ka = c.updp[0];
+    if (ka <= 0) return;
+    zgemm_small<0, 0>(c.avec, n, c.bvec, UB, c.G, n, n, n, ka, i0, j0, 1.0, 0.0, 1.0, 0.0);
+}
+
 // The t-V bond field's decisions of one family (src/dqmc_config_v/dqmc_update.f90, dqmc_update_delay.f90:
 // 28-128, dqmc_update_submatrix.f90:63-250: the same decisions), 32 bonds at a time on the block of G at
 // their 64 sites, gathered; T and the sites go to k_upd_panel and k_upd_flush as the on-site field's do.
 // (The reference's v3(2,1) at dqmc_update_submatrix.f90:153 is -v5(2,1) v5(2,2) / (v5(1,1) det v5), not
 // the inverse's -v5(2,1) / det v5; the inverse is used here, with which its three forms agree.)
 // 16 chains of N = 72 and 36 bonds a family: 240 us in one workgroup with delayed vectors, 85 us
-// here with the panels and the flush.
+// here with the panels and the flush (64 x 64 tiles; 67 with the small ones).
 struct GBonds {
     const DChain &c;
     GAS cplx *G;
