@@ -46,8 +46,8 @@ static int noalloc_setup(int device, void **out)
 
 static size_t lds_block_move(int nmax, int z)
 {
-    return (size_t)SHL_MB * SHL_MB * sizeof(cplx) + 4 * SHL_MB * sizeof(cplx) + (SHL_H + 8) * sizeof(double) +
-           7 * SHL_H * sizeof(float) + (3 * SHL_MB + 16 * 12) * sizeof(int) + (size_t)(3 + z) * nmax * sizeof(int);
+    return (size_t)SHL_MB * SHL_MB * sizeof(cplx) + 3 * SHL_MB * sizeof(cplx) + (SHL_H + 8) * sizeof(double) +
+           7 * SHL_H * sizeof(float) + (4 * SHL_MB + 16 * 12) * sizeof(int) + (size_t)(3 + z) * nmax * sizeof(int);
 }
 
 static NormF normf_of(const double *nm)

@@ -214,9 +214,9 @@ __global__ __launch_bounds__(256) void k_block_move(const DChain *chains, const 
     const int tau = nt - 1, tm = (tau + lt - 1) % lt, tp = (tau + 1) % lt;
     cplx *Mm = (cplx *)lsh;                         // 64 x 64, leading dimension 64
     cplx *colk = Mm + SHL_MB * SHL_MB;              // 2 x 64
-    cplx *pvs = colk + 2 * SHL_MB;                  // 64: pivots
-    cplx *dl = pvs + SHL_MB;                        // 64: Delta of each flipped site
+    cplx *dl = colk + 2 * SHL_MB;                   // 64: Delta of each flipped site
     double *h1 = (double *)(dl + SHL_MB);           // 128
+    cplx *pvs = (cplx *)h1;                         // 64: pivots, after the network's last evaluation
     double *red = h1 + SHL_H;                       // 8
     float *W1s = (float *)(red + 8);                // 4H
     float *b1s = W1s + 4 * SHL_H, *b2s = b1s + SHL_H, *w3s = b2s + SHL_H;
