@@ -47,7 +47,7 @@ HBM_PEAK = 8.0e12          # MI355X HBM3E, B/s
 
 
 def model_kw(args):
-    # nublock 0: start from the reference's heuristic depth, then the autotuner picks it
+    # nublock 0: start from the reference's heuristic depth, then the autotuner (DFT tiles)
     return dict(lattice="square", la=16, lb=16, beta=8.0, dtau=0.1, rt=1.0, mu=0.0, rhub=6.0, nu=0.0, nflr=2,
                 exact_hs=True, kmode="checkerboard", update="delay", nwrap=10, nublock=args.nublock)
 
@@ -78,6 +78,9 @@ def graph_demo(sweeps=40):
     return out
 
 
+UPDATE_BLOCK = 64   # sites between two updates of G, whatever the build's nublock
+
+
 def algorithmic_work(group, n, nchains, ltrot, nwrap, acc, k):
     """(kind, amount per launch) of the kernel group, all chains of the launch."""
     nn = float(n) * n
@@ -88,7 +91,7 @@ def algorithmic_work(group, n, nchains, ltrot, nwrap, acc, k):
     if group == "bprod":
         return "bytes", nchains * 2 * 16 * nn                       # one pass over the propagated U
     if group == "update":
-        return "flops", nchains * 8.0 * acc * n * nn * (1.0 + k / n)  # rank-k flushes + column builds
+        return "flops", nchains * 8.0 * acc * n * nn * (1.0 + k / n)  # rank-64 flushes + panels of 64-site blocks
     if group in ("qr", "formq"):
         return "flops", nchains * 16.0 / 3.0 * n * nn
     if group == "gemm":
@@ -253,7 +256,7 @@ def bench_c3(args):
         best = max(tm, key=lambda g: tm[g][0])
         ms, cnt = tm[best]
         a = float(np.mean(acc))
-        k = w.tables[0]["nublock"]
+        k = UPDATE_BLOCK
         if best == "update":
             amount = sum(8.0 * a * n * n * (n + k) for n in sizes)
             kind = "flops"
@@ -318,11 +321,11 @@ def timed_phase(w, steps, tau_sweeps, timers, label):
             "acc": float(acc), "means": means, "series": series, "series_len": int(series.shape[0])}
 
 
-def read_traffic(chains, n, nublock):
-    """HBM bytes per launch of the update kernel, replayed from the committed counter summary
+def read_traffic(chains, n):
+    """HBM bytes per slice of the update kernels, replayed from the committed counter summary
     (two rocprofv3 --pmc runs of this workload), when the run is the workload it was measured on."""
     path = os.path.join(ROOT, "profiles", "hbm_traffic_ft_hubbard16x16_256chains.txt")
-    if not (chains == 256 and n == 256 and nublock == 32) or not os.path.exists(path):
+    if not (chains == 256 and n == 256) or not os.path.exists(path):
         return None
     kv = dict(l.strip().split("=", 1) for l in open(path) if "=" in l and not l.startswith("#"))
     return float(kv["fetch_bytes"]) + float(kv["write_bytes"])
@@ -335,7 +338,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=60)
     ap.add_argument("--chains", type=int, default=256)
     ap.add_argument("--nublock", type=int, default=0,
-                    help="delay depth; 0: the autotuner picks it on the warmed-up chains")
+                    help="delay depth of the build (no effect on the work); 0: the reference's heuristic, and the DFT tiles tuned")
     ap.add_argument("--nprop", type=int, default=16, help="inner Metropolis attempts per block proposal (<= 64)")
     ap.add_argument("--tau-sweeps", type=int, default=100,
                     help="length of each phase's per-sweep series for tau_int (the first --steps are timed)")
@@ -469,10 +472,10 @@ def main():
         a = head["acc"]
         best = max(tm, key=lambda g: tm[g][0])
         ms, cnt = tm[best]
-        kind, amount = algorithmic_work(best, n, args.chains, ltrot, 10, a, t["nublock"])
+        kind, amount = algorithmic_work(best, n, args.chains, ltrot, 10, a, UPDATE_BLOCK)
         avg_s = ms / 1000.0 / max(cnt, 1)
         achieved = amount / avg_s
-        traffic = read_traffic(args.chains, n, t["nublock"]) if best == "update" else None
+        traffic = read_traffic(args.chains, n) if best == "update" else None
         traffic_src = "profiles/hbm_traffic_ft_hubbard16x16_256chains.txt (replayed, not measured in this run)" \
             if traffic is not None else None
         if kind == "flops":

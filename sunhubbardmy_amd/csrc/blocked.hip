@@ -240,7 +240,7 @@ template __global__ void k_solve_cb<4>(const DChain *, int, int, int, int);
 template __global__ void k_solve_cb<8>(const DChain *, int, int, int, int);
 
 // T factors of the reflectors that the column-at-a-time (pivoted) QR left in matrix sel, panel
-// by panel, so that k_formq_blk forms Q by rank-16 MFMA products
+// by panel, so that k_formq_cb forms Q by rank-16 MFMA products
 extern "C" __global__ void __launch_bounds__(BLK_NT)
 k_tfactors(const DChain *chains, int sel)
 {
