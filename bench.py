@@ -321,16 +321,6 @@ def timed_phase(w, steps, tau_sweeps, timers, label):
             "acc": float(acc), "means": means, "series": series, "series_len": int(series.shape[0])}
 
 
-def read_traffic(chains, n):
-    """HBM bytes per slice of the update kernels, replayed from the committed counter summary
-    (two rocprofv3 --pmc runs of this workload), when the run is the workload it was measured on."""
-    path = os.path.join(ROOT, "profiles", "hbm_traffic_ft_hubbard16x16_256chains.txt")
-    if not (chains == 256 and n == 256) or not os.path.exists(path):
-        return None
-    kv = dict(l.strip().split("=", 1) for l in open(path) if "=" in l and not l.startswith("#"))
-    return float(kv["fetch_bytes"]) + float(kv["write_bytes"])
-
-
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -475,16 +465,12 @@ def main():
         kind, amount = algorithmic_work(best, n, args.chains, ltrot, 10, a, UPDATE_BLOCK)
         avg_s = ms / 1000.0 / max(cnt, 1)
         achieved = amount / avg_s
-        traffic = read_traffic(args.chains, n) if best == "update" else None
-        traffic_src = "profiles/hbm_traffic_ft_hubbard16x16_256chains.txt (replayed, not measured in this run)" \
-            if traffic is not None else None
         if kind == "flops":
             roof = {"bound": "mfma", "achieved": achieved / 1e12, "peak": FP64_MFMA_PEAK / 1e12, "unit": "TFLOP/s",
-                    "frac": achieved / FP64_MFMA_PEAK, "traffic": traffic}
+                    "frac": achieved / FP64_MFMA_PEAK, "traffic": None}
         else:
             roof = {"bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
-                    "frac": achieved / HBM_PEAK, "traffic": traffic}
-        roof["traffic_source"] = traffic_src
+                    "frac": achieved / HBM_PEAK, "traffic": None}
         roof["kernel_group"] = best
         roof["avg_launch_ms"] = ms / max(cnt, 1)
         line["roofline"] = roof

@@ -26,6 +26,9 @@
 // 2360 -> 659 / 1460 -> 960, 16 of N = 400 4500 -> 1010 / 2750 -> 1400, 256 of N = 256 2080 -> 1300 /
 // 1550 -> 1340; Q: 256 of N = 256 1240 -> 680, one of N = 288 1220 -> 104. Broadcasting a column through LDS
 // instead of the row lanes costs 1300 cycles a column more.
+// Tall matrices (N x nc, the projective sweep's propagators, N <= 1024): the same kernels with nc columns; above 512 rows
+// a wave holds eight tiles and broadcasts a column twice instead of keeping it.  Eight of 648 x 324: QR 1.6 ms and
+// Q 0.25 (14.8 together in one workgroup per chain), the inverse of 324 x 324 1.3 ms (4.5).
 #include "factor.h"
 #include <type_traits>
 

@@ -17,7 +17,7 @@
 // Why this split: keeping the delayed vectors of all N rows next to the decisions costs a pass over
 // N k entries per site in one workgroup (2 us per site at N = 256, k = 32) and a rank-k update of G
 // on one CU; here a decision touches 64 x 64 entries and every flop of O(N^2) runs on the whole
-// chip.  Per slice: one N = 288 chain 1.72 -> 0.27 ms, 72 chains of N = 64, 144, 256 0.90 -> 0.29 ms,
+// chip.  Per slice: one N = 288 chain 1.72 -> 0.23 ms, 72 chains of N = 64, 144, 256 0.90 -> 0.27 ms,
 // 256 chains of N = 256 1.20 -> 0.95 ms (per block 40 us of decisions, 55 us of panels, 140 us of
 // flush; one read and write of the 256 MiB of G takes 111 us), 16 chains of N = 64 172 -> 31 us.
 #include "gemm_small.h"
