@@ -13,6 +13,13 @@ __device__ __forceinline__ cplx cfma(cplx a, cplx b, cplx c)
     return make_double2(fma(-b.y, c.y, fma(b.x, c.x, a.x)), fma(b.y, c.x, fma(b.x, c.y, a.y)));
 }
 
+// z times a power of two: the larger part in [1/2, 1)
+__device__ __forceinline__ cplx pow2_unit(cplx z)
+{
+    const int k = -__builtin_amdgcn_frexp_exp(fmax(fabs(z.x), fabs(z.y)));
+    return make_double2(ldexp(z.x, k), ldexp(z.y, k));
+}
+
 // The decisions of the block's sites 0 .. nb - 1, nb <= 16 NT, by a workgroup of NT waves.  Wave w holds the
 // columns 16 w .. 16 w + 15 of the block H as NT accumulator tiles of the FP64 MFMA (element r of lane l:
 // column l/16 + 4r, row l%16 of the tile).  Four sites g at a time, one barrier each: every wave
@@ -37,8 +44,10 @@ __device__ __forceinline__ cplx cfma(cplx a, cplx b, cplx c)
 // time with the block spread over 16 x 16 threads takes 1360 cycles a site, 41 us a block against 30
 // here: a barrier and eleven LDS reads per thread and site for one rank-1 update.
 // Acceptance is |Re(ratiotot phase)| > u2 |Re(phase)| with ratiotot = ratio1^nflr qf: the
-// reference's |Re(ratiotot phase) / Re(phase)| > u2 without the division, which lets phase grow
-// unnormalised over the block.
+// reference's |Re(ratiotot phase) / Re(phase)| > u2 without the division.  Only the direction of phase
+// counts; so that the accepted ratios of a block (1e200 for twelve flavours far from the weights' maximum) do not leave the
+// exponent range, it takes an exact power of two after every group, and with nflr not known here (NF = 0)
+// after every site: neither decisions nor direction depend on it.
 //
 // P: load(i, j) the entry of the block; factors(site, db, qf, u2) of a site < nb, its delta, field-only
 // factor and acceptance uniform (PAIR: qf and u2 of the bond's first site); store(i, j, v, ri, rj) for
@@ -180,6 +189,7 @@ __device__ __forceinline__ void exchange_block(P &pol, int nb, int nflr, cplx ph
                 const bool acc = fabs(rt.x) > u2[k] * fabs(phase.x);
                 phase.x = acc ? rt.x : phase.x;
                 phase.y = acc ? rt.y : phase.y;
+                if (NF == 0) phase = pow2_unit(phase);
                 sg[k].x = acc ? sk.x : 0.0;
                 sg[k].y = acc ? sk.y : 0.0;
                 mg |= (__ballot(acc) != 0 ? 1u : 0u) << k;
@@ -191,6 +201,7 @@ __device__ __forceinline__ void exchange_block(P &pol, int nb, int nflr, cplx ph
                 }
             }
         }
+        if (PAIR || NF > 0) phase = pow2_unit(phase);
         factors(min(s + 4, UB - 4));   // the next group's, on their way while this one is applied
         if (mg != 0) {
             mask |= (unsigned long long)mg << s;

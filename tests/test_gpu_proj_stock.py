@@ -20,3 +20,8 @@ def test_bond_stocks(la, nustock):
 @pytest.mark.parametrize("nflr", [2, 4])
 def test_site_stocks(la, nustock, nflr):
     run_parity(dict(KW, la=la, nustock=nustock, rv=0.0, rhub=4.0, nflr=nflr), nsweeps=1)
+
+
+def test_site_stock_ratios_beyond_the_exponent_range():
+    """The first stock of 24 flavours at U = -8 from a random field: its accepted ratios multiply to more than 1e154."""
+    run_parity(dict(KW, la=66, nustock=64, rv=0.0, rhub=-8.0, nflr=24, exact_hs=False), nsweeps=1)

@@ -90,3 +90,11 @@ def test_one_chain(n):
 def test_uneven_batch(kw):
     check([64, 14, 130, 48, 66, 200, 2], **kw)
     check([62, 16, 30], **kw)
+
+
+# A field far from the weights' maximum: the accepted ratios of a block multiply to 1e200 (12 flavours, U = -8; two
+# flavours, U = -120) and 1e312 (U = -16; -240), where the decisions and the phase need only their direction.
+@pytest.mark.parametrize("sizes", [[64], [130], [64, 130, 34]])
+@pytest.mark.parametrize("nflr,u", [(12, -8.0), (12, -16.0), (2, -120.0), (2, -240.0)])
+def test_ratios_beyond_the_exponent_range(nflr, u, sizes):
+    check(sizes, rhub=u, nflr=nflr, exact_hs=False, update="delay", nublock=16)
