@@ -228,14 +228,10 @@ __device__ __forceinline__ void qr_panel(FBlk<FT> &x, int b, int toff, cplx &tau
             double nrm = n2 * rs;
             nrm = fma(0.5 * rs, fma(-nrm, nrm, n2), nrm);
             beta = alpha.x >= 0 ? -nrm : nrm;
-            const double ib = alpha.x >= 0 ? -rs : rs, sum = nrm + fabs(alpha.x);
+            const double ib = alpha.x >= 0 ? -rs : rs;
             amb = make_double2(alpha.x - beta, alpha.y);
             tau = make_double2(-amb.x * ib, -amb.y * ib);
-            const double d = fma(sum, sum, alpha.y * alpha.y);     // |alpha - beta|^2
-            double rc = __builtin_amdgcn_rcp(d);
-            rc = fma(rc, fma(-d, rc, 1.0), rc);
-            rc = fma(rc, fma(-d, rc, 1.0), rc);
-            scal = cscale(cconj(amb), rc);
+            scal = cinv_s(amb);     // scaled: |alpha - beta|^2 leaves the exponent range before n2 does
         }
         // v_j^H (column l16): the sum over the rows below j in units of the unscaled column j
         const cplx wq = cadd(cmul(cconj(scal), s), ajq);

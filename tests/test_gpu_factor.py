@@ -79,6 +79,27 @@ def test_qr_and_q(sizes):
     b.w.close()
 
 
+# Columns whose squared norm is still a number but |alpha - beta|^2 of their reflector, up to four times that, is beyond
+# either end of the exponent range: its reciprocal is not representable below 2^-1024, its square not above
+# 2^1024.  Squares near 2^-1074 are rounded to that absolute step: relative to nu^2 / n, the least a reflector meets,
+# n 2^-1075 / nu^2 < 1e-13 at nu = 3e-155 and n = 34, so 1e-11 for the sums of them.
+@pytest.mark.parametrize("n", [2, 18, 34])
+@pytest.mark.parametrize("scale", [3e-155, 1.1e154])
+def test_qr_at_the_ends_of_the_exponent_range(n, scale):
+    b = Batch([n])
+    rng = np.random.default_rng(n)
+    A = np.eye(n) + 0.1 * rnd(n, rng) / np.sqrt(n)      # the diagonal carries most of a column's norm
+    A /= np.linalg.norm(A, axis=0)
+    b.put("W1", 0, A)
+    b.vec(100, 0, n, 0, np.full(n, scale))
+    b.put("V", 0, np.eye(n), 0)
+    b.op(4, 1, 0)
+    U, V, D = b.get("U", 0, 1), b.get("V", 0, 1), b.vec(100, 0, n, 1)
+    assert np.abs(U.conj().T @ U - np.eye(n)).max() < 1e-11
+    assert np.abs(U @ np.diag(D / scale) @ V - A).max() < 1e-11
+    b.w.close()
+
+
 @pytest.mark.parametrize("sizes", CASES)
 def test_lu_and_solve(sizes):
     b = Batch(sizes)
