@@ -1,9 +1,7 @@
 // blocked.hip -- substitution with the LU factors of factor.hip, sixteen right-hand sides per
-// workgroup, and the T factors of the column-at-a-time QR's reflectors.
+// workgroup.
 #include "sunhip_kernels.h"
 
-#define PB 16          // panel width (T factors are stored PB x PB)
-#define BLK_NT 512     // threads per workgroup (8 waves)
 #define BLK_NMAX 512   // largest N of the kernels here and in factor.hip
 
 // MFMA operand layout (gfx950): A(16x4): lane l holds A[l%16][l/16]; B(4x16): lane l holds
@@ -11,61 +9,6 @@
 __device__ __forceinline__ double4_t mfma64(double a, double b, double4_t c)
 {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-// V[r][p] of a Householder panel stored LAPACK-style (unit diagonal implicit, zeros above)
-__device__ __forceinline__ cplx vpanel(const cplx *P, int ldp, int r, int p)
-{
-    if (r > p) return P[p * ldp + r];
-    return make_double2(r == p ? 1.0 : 0.0, 0.0);
-}
-
-// T factor of one panel (zlarft, forward, columnwise): S = V^H V over the panel's m rows,
-// T(:,j) = -tau_j T(:,0:j) S(0:j, j); V is the m x b panel in LDS (ld M, unit diagonal implicit).
-// Row i of T only needs row i itself and S (T(i, j) = -tau_j sum_{i <= q < j} T(i, q) S(q, j)),
-// so lane i builds its row in registers, all rows at once.
-__device__ static void panel_tfactor(const cplx *P, int M, int m, int b, const cplx *tau, cplx *T, cplx *S)
-{
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    for (int pr = w; pr < b * b; pr += nw) {
-        int i = pr % b, j = pr / b;
-        if (i >= j) continue;
-        double sr = 0.0, si = 0.0;
-        for (int r = j + lane; r < m; r += 64) {
-            cplx vi = vpanel(P, M, r, i), vj = vpanel(P, M, r, j);
-            sr += vi.x * vj.x + vi.y * vj.y;
-            si += vi.x * vj.y - vi.y * vj.x;
-        }
-        sr = wave_sum(sr);
-        si = wave_sum(si);
-        if (lane == 0) S[j * PB + i] = make_double2(sr, si);
-    }
-    __syncthreads();
-    if (threadIdx.x < PB) {
-        const int i = threadIdx.x;
-        GAS cplx *tg = gp(tau);
-        cplx tv[PB], trow[PB];
-#pragma unroll
-        for (int j = 0; j < PB; j++) {
-            tv[j] = gld(tg + min(j, b - 1));
-            trow[j] = make_double2(0.0, 0.0);
-        }
-#pragma unroll
-        for (int j = 0; j < PB; j++) {
-            if (j < b && j > i) {
-                cplx acc = make_double2(0.0, 0.0);
-#pragma unroll
-                for (int q = 0; q < PB; q++)
-                    if (q >= i && q < j) acc = cadd(acc, cmul(trow[q], S[j * PB + q]));
-                trow[j] = cmul(make_double2(-tv[j].x, -tv[j].y), acc);
-            } else if (j < b && j == i) {
-                trow[j] = tv[j];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < PB; j++) T[j * PB + i] = trow[j];
-    }
-    __syncthreads();
 }
 
 // ------------------------------------------------------------------------------------------
@@ -238,28 +181,3 @@ k_solve_cb(const DChain *chains, int nch, int ncb, int xsel, int ident)
 
 template __global__ void k_solve_cb<4>(const DChain *, int, int, int, int);
 template __global__ void k_solve_cb<8>(const DChain *, int, int, int, int);
-
-// T factors of the reflectors that the column-at-a-time (pivoted) QR left in matrix sel, panel
-// by panel, so that k_formq_cb forms Q by rank-16 MFMA products
-extern "C" __global__ void __launch_bounds__(BLK_NT)
-k_tfactors(const DChain *chains, int sel)
-{
-    extern __shared__ cplx bsh[];
-    const DChain &c = chains[blockIdx.x];
-    const int n = c.n;
-    cplx *P = bsh;
-    cplx *T = bsh + (size_t)n * PB;
-    cplx *S = T + PB * PB;
-    const cplx *A = chain_mat(c, sel, 0);
-    for (int k0 = 0; k0 < n; k0 += PB) {
-        const int m = n - k0, b = min(PB, m);
-        for (int e = threadIdx.x; e < m * b; e += blockDim.x) {
-            int r = e % m, p = e / m;
-            P[p * n + r] = A[(size_t)(k0 + r) + (size_t)(k0 + p) * n];
-        }
-        __syncthreads();
-        panel_tfactor(P, n, m, b, c.tau + k0, T, S);
-        for (int e = threadIdx.x; e < PB * PB; e += blockDim.x) c.tblk[(size_t)(k0 / PB) * PB * PB + e] = T[e];
-        __syncthreads();
-    }
-}

@@ -673,14 +673,13 @@ __device__ __forceinline__ void qr_apply_col(GAS cplx *a, const cplx (&x)[NQ], i
 
 // Householder QR, column-at-a-time, with column pivoting (pivot = 1, zgeqp3's choice by the
 // downdated partial norms) or in the given order (pivot = 0); R above the diagonal, the
-// reflectors below, tau to c.tau, log det Q to ldq[out_pt].  Every column a wave works on is
-// read once into registers (NQ = rows / 64), and the wave's next trailing column is loaded while
-// the current one is reduced.
-template <int NQ>
-__global__ void __launch_bounds__(1024)
+// reflectors below, tau to c.tau, log det Q to ldq[out_pt].  The sweeps' form above N = 512.  Every column a
+// wave works on is read once into registers (NQ slots of 64 rows).
+extern "C" __global__ void __launch_bounds__(1024)
 k_qr(const DChain *chains, int sel, int pivot, int out_pt)
 {
     extern __shared__ double qrsh[];
+    constexpr int NQ = 16;
     const DChain &c = chains[blockIdx.x];
     const int n = c.n;
     double *vn1 = qrsh, *vn2 = qrsh + n;
@@ -773,28 +772,12 @@ k_qr(const DChain *chains, int sel, int pivot, int out_pt)
         }
         __syncthreads();
         const cplx tc = cconj(s_tau);
-        // apply H^H to the trailing columns, one wave per column; the wave's next column is
-        // in flight while the current one is reduced
-        int j = i + 1 + w;
-        if (NQ > 4) {
-            // (two register sets of more than four slots would spill at 1024 threads)
-            for (; j < n; j += nw) {
-                cplx xa[NQ];
-                qr_col_load<NQ>(A + (size_t)j * n, i, n, lane, xa);
-                qr_apply_col<NQ>(A + (size_t)j * n, xa, i, j, n, lane, tc, v, pivot, vn1, vn2, tol3z);
-            }
-        } else if (j < n) {
-            cplx xa[NQ], xb[NQ];
+        // apply H^H to the trailing columns, one wave per column (a second register set for the next column would
+        // spill at 1024 threads)
+        for (int j = i + 1 + w; j < n; j += nw) {
+            cplx xa[NQ];
             qr_col_load<NQ>(A + (size_t)j * n, i, n, lane, xa);
-            for (; j < n; j += 2 * nw) {
-                const int j2 = j + nw;
-                if (j2 < n) qr_col_load<NQ>(A + (size_t)j2 * n, i, n, lane, xb);
-                qr_apply_col<NQ>(A + (size_t)j * n, xa, i, j, n, lane, tc, v, pivot, vn1, vn2, tol3z);
-                if (j2 < n) {
-                    if (j2 + nw < n) qr_col_load<NQ>(A + (size_t)(j2 + nw) * n, i, n, lane, xa);
-                    qr_apply_col<NQ>(A + (size_t)j2 * n, xb, i, j2, n, lane, tc, v, pivot, vn1, vn2, tol3z);
-                }
-            }
+            qr_apply_col<NQ>(A + (size_t)j * n, xa, i, j, n, lane, tc, v, pivot, vn1, vn2, tol3z);
         }
         __syncthreads();
     }
@@ -814,10 +797,6 @@ k_qr(const DChain *chains, int sel, int pivot, int out_pt)
     si = block_sum(si, red);
     if (threadIdx.x == 0) c.ldq[out_pt] = make_double2(sr, si);
 }
-
-template __global__ void k_qr<4>(const DChain *, int, int, int);
-template __global__ void k_qr<8>(const DChain *, int, int, int);
-template __global__ void k_qr<16>(const DChain *, int, int, int);
 
 // Q = H_1 ... H_n from the reflectors in matrix `sel` (zung2r), written to chain point U[pt]
 // (dest 0) or Us (dest 1)

@@ -8,7 +8,7 @@
 struct shp_ctx : ctx_base {
     int nch = 0, n = 0, ne = 0, ltrot = 0, nwrap = 0, nst = 0, kmode = 0, ns = 0, mid_len = 1;
     int nn_nf = 0, nn_lf = 0, wrap_check = 1;
-    int update = SHP_U_LR, gblock = 0;   // update algorithm of the on-site field and its depth
+    int update = SHP_U_LR;        // update algorithm
     bool lwrapu = false, lwrapv = true, flav2 = true;   // flav2: nflr = 2 in every chain
     size_t slice_draws = 0;       // uniforms per slice of a pass
     bool tracing = false, started = false;
@@ -388,7 +388,6 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
     ctx->lwrapv = q0.vtab != nullptr;
     ctx->lwrapu = q0.ubmat != nullptr;
     ctx->update = q0.update;
-    ctx->gblock = q0.gblock;
     ctx->slice_draws = (ctx->lwrapu ? (size_t)2 * q0.ndim : 0) + (ctx->lwrapv ? (size_t)2 * q0.nn_lf * q0.nn_nf : 0);
     for (int c = 0; c < nchains; c++) {
         const shp_model &q = m[c];
@@ -543,12 +542,9 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
         v.G = c.G; v.bonds = c.bonds; v.stag = c.stag; v.sc = c.sc; v.rwork = c.rwork;
         v.kin_weight = q.kin_weight != 0.0 ? q.kin_weight : 1.0;
         if (ctx->update >= SHP_U_DELAY) {
-            // ... and the G-based updates of the on-site field the HS field, its draws and tables,
-            // the delayed vectors and the submatrix scratch
-            const int K = ctx->gblock;
+            // ... and the G-based updates the field, its draws and tables and the block update's scratch
             c.uold = dalloc<int32_t>(ctx, n);
-            v.ltrot = q.ltrot; v.nublock = K;
-            v.update = ctx->update == SHP_U_DELAY ? SH_U_DELAY : SH_U_SUBMATRIX;
+            v.ltrot = q.ltrot;
             if (ctx->lwrapu) {
                 v.conf = c.uconf; v.unif = c.unif;
                 v.lcomp = q.ulcomp;
@@ -566,15 +562,11 @@ int shp_create(shp_ctx **out, int nchains, const shp_model *m, int device)
                 for (int k = 0; k < 4; k++) v.vdl[k] = c.vd[k];
                 v.vacc = c.sc + SC_ACC;
             }
-            // (the bond field's submatrix form borders by 2 x 2 blocks: at least two columns)
-            const int Ka = std::max(K, 2);
             v.avec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX);
             v.bvec = dalloc<cplx>(ctx, (size_t)n * SH_KMAX);
             v.updt = dalloc<cplx>(ctx, (size_t)UB * UB);
             v.updp = dalloc<int32_t>(ctx, UB + 1);
-            v.W1 = dalloc<cplx>(ctx, (size_t)n * Ka);
-            v.W2 = dalloc<cplx>(ctx, (size_t)Ka * Ka);
-            if (!c.uold || !v.avec || !v.bvec || !v.updt || !v.updp || !v.W1 || !v.W2) {
+            if (!c.uold || !v.avec || !v.bvec || !v.updt || !v.updp) {
                 int rc = fail(ctx, SH_E_HIP, "device allocation failed");
                 shp_destroy(ctx);
                 return rc;

@@ -311,7 +311,6 @@ static void wrap_pass(sh_ctx *ctx, bool add, int prog, int nt)
 // ---- stabilization -------------------------------------------------------------------------
 static size_t lds_qr(sh_ctx *ctx) { return (size_t)ctx->nmax * 32; }
 static bool blocked(sh_ctx *ctx) { return ctx->nmax <= BLK_NMAX; }
-static size_t lds_blk(sh_ctx *ctx) { return ((size_t)ctx->nmax * PB + 2 * PB * PB) * sizeof(cplx) + ctx->nmax * 4; }
 
 // waves of a workgroup of the factorizations: each holds 64 of the matrix's rows
 static int fac_waves(sh_ctx *ctx) { return ctx->nmax <= 256 ? 4 : 8; }
@@ -343,12 +342,10 @@ static void lu_solve(sh_ctx *ctx, int xsel)
         hipLaunchKernelGGL(k_lu_solve, dim3(ctx->nch), dim3(512), 0, ctx->st, ctx->dc, xsel);
 }
 
-// column-at-a-time QR of matrix sel (pivot: zgeqp3's column pivoting), rows held in registers
-// in NQ = ceil(N / 64) slots
+// column-at-a-time QR of matrix sel (pivot: zgeqp3's column pivoting)
 static void launch_qr(sh_ctx *ctx, int sel, int pivot, int pt)
 {
-    auto k = ctx->nmax <= 256 ? k_qr<4> : ctx->nmax <= 512 ? k_qr<8> : k_qr<16>;
-    hipLaunchKernelGGL(k, dim3(ctx->nch), dim3(1024), lds_qr(ctx), ctx->st, ctx->dc, sel, pivot, pt);
+    hipLaunchKernelGGL(k_qr, dim3(ctx->nch), dim3(1024), lds_qr(ctx), ctx->st, ctx->dc, sel, pivot, pt);
 }
 
 // Q of the reflectors in matrix sel -> U[pt]: 16 columns per workgroup, a chain's workgroups on one XCD
@@ -360,8 +357,8 @@ static void formq(sh_ctx *ctx, int sel, int pt)
 }
 
 // QR of W1 (first: column pivoting, from U = D = V = 1) or of the prepivoted W1 diag(D[dpt]) -> point
-// `pt`.  Up to N = 512 the first point of a chain is prepivoted like the others: the product of
-// nwrap slices is the best scaled one of the chain, and column pivoting streams the trailing matrix once
+// `pt`.  Up to N = 512 no sweep asks for first: the first point of a chain is prepivoted like the others, since the
+// product of nwrap slices is the best scaled one of the chain, and column pivoting streams the trailing matrix once
 // per column (10 ms for 256 chains of N = 256 against 2.4 ms of the prepivoted form).
 static void udv_step(sh_ctx *ctx, bool first, int pt, int dpt)
 {
@@ -372,13 +369,8 @@ static void udv_step(sh_ctx *ctx, bool first, int pt, int dpt)
         }
         {
             Tic t(ctx, T_FORMQ);
-            if (blocked(ctx)) {
-                hipLaunchKernelGGL(k_tfactors, dim3(ctx->nch), dim3(BLK_NT), lds_blk(ctx), ctx->st, ctx->dc, M_W1);
-                formq(ctx, M_W1, pt);
-            } else {
-                hipLaunchKernelGGL(k_formq, dim3(ctx->nch), dim3(1024), (size_t)ctx->nmax * sizeof(cplx), ctx->st,
-                                   ctx->dc, M_W1, pt);
-            }
+            hipLaunchKernelGGL(k_formq, dim3(ctx->nch), dim3(1024), (size_t)ctx->nmax * sizeof(cplx), ctx->st, ctx->dc,
+                               M_W1, pt);
         }
         Tic t(ctx, T_OTHER);
         hipLaunchKernelGGL(k_v_from_qrcp, grid_elem(ctx), dim3(256), 0, ctx->st, ctx->dc, M_W1, pt);
@@ -845,8 +837,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
     {
         struct { const void *f; size_t bytes; } big[] = {
             {(const void *)k_cb_rows, lds_rows(ctx)}, {(const void *)k_cb_cols, lds_cols(ctx)},
-            {(const void *)k_fft_rows, lds_fft(ctx)}, {(const void *)k_fft_cols, lds_fft(ctx)},
-            {(const void *)k_tfactors, blocked(ctx) ? lds_blk(ctx) : 0}};
+            {(const void *)k_fft_rows, lds_fft(ctx)}, {(const void *)k_fft_cols, lds_fft(ctx)}};
         for (auto &b : big) {
             if (b.bytes <= 64 * 1024 || b.bytes > 150 * 1024) continue;
             hipFuncAttributes fa;
@@ -873,7 +864,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         const int n = q.ndim;
         const size_t nn = (size_t)n * n;
         c.n = n; c.lq = q.lq; c.nn_nf = q.nn_nf; c.nn_lf = q.nn_lf; c.lcomp = q.lcomp; c.nflr = q.nflr;
-        c.kmode = q.kmode; c.nublock = q.nublock; c.update = q.update; c.lwrapT = q.lwrapT; c.lwrapu = q.lwrapu;
+        c.kmode = q.kmode; c.nublock = q.nublock; c.lwrapT = q.lwrapT; c.lwrapu = q.lwrapu;
         c.phase_from_conf = q.phase_from_conf; c.ltrot = q.ltrot; c.nst = q.nst;
         c.kin_weight = q.kin_weight != 0.0 ? q.kin_weight : 1.0;
         if (q.vtab) {
@@ -923,7 +914,7 @@ int sh_create(sh_ctx **out, int nchains, const sh_model *m, int device)
         c.updt = dalloc<cplx>(ctx, (size_t)UB * UB); c.updp = dalloc<int32_t>(ctx, UB + 1);
         c.tau = dalloc<cplx>(ctx, n); c.jpvt = dalloc<int32_t>(ctx, n); c.piv = dalloc<int32_t>(ctx, n);
         c.lperm = dalloc<int32_t>(ctx, n); c.lup = dalloc<int32_t>(ctx, (size_t)((n + FPB - 1) / FPB) * FLMAX);
-        c.tblk = dalloc<cplx>(ctx, (size_t)(n / PB + 1) * PB * PB);
+        c.tblk = dalloc<cplx>(ctx, (size_t)(n / FPB + 1) * FPB * FPB);
         c.rwork = dalloc<double>(ctx, 4 * (size_t)n);
         c.conf = dalloc<int32_t>(ctx, (size_t)n * q.ltrot);
         c.unif = dalloc<double>(ctx, (size_t)2 * n * q.ltrot);

@@ -74,7 +74,7 @@ enum {
 enum { M_G = 0, M_GS, M_W1, M_W2, M_W3, M_W4, M_US, M_VS, M_U, M_V, M_KT, M_KTM1, M_GT0, M_G0T, M_G00, M_GT0S, M_G0TS };
 
 struct DChain {
-    int n, lq, nn_nf, nn_lf, lcomp, nflr, kmode, nublock, update, lwrapT, lwrapu, phase_from_conf;
+    int n, lq, nn_nf, nn_lf, lcomp, nflr, kmode, nublock, lwrapT, lwrapu, phase_from_conf;
     int ltrot, nst, pad0, pad1;
     cplx *G, *Gs, *W1, *W2, *W3, *W4, *Us, *Vs;
     cplx *U, *V;          // (nst+1) points, n*n each
