@@ -32,7 +32,7 @@ int sh_dbg_get(sh_ctx *ctx, int chain, int sel, int pt, double *dst);
  * 11: draw the pass uniforms (2 N ltrot) from each chain's generator
  * 12: measurement of G into the observable sums
  * 13: wrap check/replace (compare = a0)
- * 14: no effect (the builds share one form of the bond-field update) */
+ * 14: DFT kinetic form: a0 = 2, 4, 8 or 16 vectors per workgroup (within 96 KiB of LDS) */
 int sh_dbg_op(sh_ctx *ctx, int op, const int *a);
 
 #ifdef __cplusplus

@@ -1852,7 +1852,13 @@ extern "C" int sh_dbg_op(sh_ctx *ctx, int op, const int *a)
         break;
     case 12: measure(ctx); break;
     case 13: wrap_replace(ctx, a[0]); break;
-    case 14: break;   // one form of the bond update serves every build
+    case 14:
+        if (ctx->kmode != SH_K_FFT || (a[0] != 2 && a[0] != 4 && a[0] != 8 && a[0] != 16) ||
+            (size_t)a[0] * ctx->fft_ld * sizeof(cplx) > 96 * 1024)
+            return SH_E_ARG;
+        ctx->fft_fcb = a[0];
+        ctx->graph_epoch++;
+        break;
     default: return SH_E_ARG;
     }
     int rc = check_launch(ctx);
