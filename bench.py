@@ -441,7 +441,7 @@ def main():
         "warmup": args.warmup, "ms_per_step": 1000.0 * head["dt"] / args.steps, "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f64", "data": "synthetic",
         "config": {"workload": wl, "chains": args.chains, "nublock": t["nublock"],
-                   "nublock_from": "autotuner (sh_autotune)" if tuned is not None else "--nublock",
+                   "nublock_from": "heuristic (no result or launch depends on it)" if args.nublock == 0 else "--nublock",
                    "proposal": "learned (block moves of %d attempts after each slice's local update)" % args.nprop
                    if learned is not None else "plain local delay update"},
     }

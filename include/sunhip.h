@@ -63,7 +63,7 @@ typedef struct sh_model {
     int phase_from_conf;    /* 1 when set_phase multiplies u0conf%phase (rhub > 0) */
     const double *stag;     /* [ndim] +-1 staggering used for S_stag (S(pi,pi) on the square lattice) */
     int update;             /* SH_U_* */
-    int nublock;            /* delay depth / submatrix block */
+    int nublock;            /* delay depth / submatrix block of the build, 1 .. 64; no result or launch depends on it */
     int32_t seed;           /* SFMT19937 seed of this chain (spring_sfmt_init) */
     double kin_weight;      /* factor of the zkint bin: 1 (0 is read as 1) in 2D and 3D, nflr * rt for
                                the chain (src/dqmc_measure/equaltime_measure1d.f90:76) */
@@ -212,10 +212,10 @@ int sh_synchronize(sh_ctx *ctx);
 int sh_set_graphs(sh_ctx *ctx, int enable);
 
 /* Autotuner, after sh_sweep_start_0b: with the FFT kinetic form the DFT kernels are timed at 2 .. 16
- * vectors per workgroup on scratch matrices and the fastest is kept for every chain.  The on-site
- * update needs no depth (it flushes once per block of sites), so the batch's nublock, which the
- * bond field's delay and submatrix forms use, is returned as it is.  tuned[0] = nublock, tuned[1] =
- * vectors per workgroup (0: not FFT).  The chains' state is left bit for bit as it was. */
+ * vectors per workgroup on scratch matrices and the fastest is kept for every chain.  The updates
+ * need no depth (G takes the product of a whole block of sites or bonds), so the batch's nublock is
+ * returned as it is.  tuned[0] = nublock, tuned[1] = vectors per workgroup (0: not FFT).  The chains'
+ * state is left bit for bit as it was. */
 int sh_autotune(sh_ctx *ctx, int *tuned);
 
 #ifdef __cplusplus

@@ -58,9 +58,9 @@ typedef struct shp_model {
      * src/dqmc_config_v/dqmc_proj_update*.f90; the reference selects it for both by its build):
      * SHP_U_LR submatrix-LR in stocks of nustock rows (default 0);
      * SHP_U_FAST one site (bond) at a time: rank-1 (rank-2) updates of UR and (UL UR)^-1;
-     * SHP_U_DELAY / SHP_U_SUBMATRIX_G updates of G = 1 - UR (UL UR)^-1 UL (the delay form with
-     * depth gblock 1..64, or G updated at every accepted site or bond), then UR's flipped rows
-     * and a fresh (UL UR)^-1.  The four take the same decisions from the same draws.  The
+     * SHP_U_DELAY / SHP_U_SUBMATRIX_G updates of G = 1 - UR (UL UR)^-1 UL, one block form for both
+     * (gblock, 1..64, is checked and changes nothing), then UR's flipped rows and a fresh
+     * (UL UR)^-1.  The four take the same decisions from the same draws.  The
      * G-based forms need one field alone (on-site or bond).  All chains of a batch share update
      * and gblock. */
     int update, gblock;

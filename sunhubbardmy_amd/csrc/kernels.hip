@@ -857,8 +857,8 @@ k_v_from_qrcp(const DChain *chains, int sel, int pt)
 }
 
 // prepivot: Btmp = Bd diag(Dprev); columns sorted by decreasing norm (s_zmcpt); the sorted
-// matrix goes to W2, the order to jpvt.  One workgroup per chain; the selection sort (first
-// maximum wins, the displaced entry takes the maximum's slot) runs in wave 0 without barriers.
+// matrix goes to W2, the order to jpvt.  One workgroup per chain; a column's place is the count of
+// the columns that come before it (equal norms keep their order; s_zmcpt's selection sort exchanges them).
 // A wave scales two columns at a time and the copy moves eight entries per thread at a time,
 // every batch's loads issued before its first store (clamped addresses).
 extern "C" __global__ void __launch_bounds__(1024)

@@ -413,7 +413,8 @@ static void vprop(sh_ctx *ctx, int sel, int nf, int mode, int side, int nt)
 // G += G(:, P) T (G(P, :) - E_P) of the block whose decisions stand in updt and updp.  The panel takes the 32 x 32 tiles
 // by rounds of the CUs like the products (16 chains of N = 400 16 -> 9.5 us).  The flush, with its loads and
 // stores of G, only where the 64 x 64 tiles leave CUs without one: one N = 288 chain (25 tiles) 11.7 -> 6.5 us,
-// but 16 chains of N = 400 (784 tiles) 33 -> 42.
+// but 16 chains of N = 400 (784 tiles) 33 -> 42 and 72 chains of N = 64, 144, 256 18.5 -> 27.  Both rules count every
+// chain as the largest one: of those 72 chains' 1152 large tiles 504 have work.
 static void upd_apply(hipStream_t st, const DChain *dc, int nch, int nmax, int s0)
 {
     const int ntl = (nmax - 1) / GT + 1, nts = (nmax - 1) / GS + 1, grp = tile_group(nch);
@@ -697,8 +698,7 @@ static int check_launch(sh_ctx *ctx)
 // executable hipGraph per pass kind and flags and replayed, so that a pass costs one host launch.
 // Kernel arguments are captured by value; the chain descriptors are read from device memory at
 // run time.  Every setter that changes which kernels a pass launches, their shapes or by-value
-// arguments (proposals, correlation bins, the time-displaced pass, the autotuned depth and tiles,
-// the delay-kernel switch) advances graph_epoch, which retires the captured graphs.
+// arguments (proposals, correlation bins, the time-displaced pass, the autotuned DFT tiles) advances graph_epoch, which retires the captured graphs.
 template <class Body>
 static int run_pass(sh_ctx *ctx, int key, Body body)
 {

@@ -80,8 +80,8 @@ struct DChain {
     cplx *U, *V;          // (nst+1) points, n*n each
     double *D, *Ds;       // (nst+1)*n, n
     cplx *ldq;            // nst+1
-    cplx *avec, *bvec;    // n*64 (k_upd_panel); n*nublock delayed vectors of the bond field
-    cplx *updt;           // 64 x 64: T of the on-site update's current block of sites
+    cplx *avec, *bvec;    // n*64: A and V of the block update (k_upd_panel)
+    cplx *updt;           // 64 x 64: T of the current block of sites or bonds
     int32_t *updp;        // its accepted sites: count, then the sites
     cplx *tau;            // n
     cplx *tblk;           // (n/16 + 1) triangular 16 x 16 factors of the block reflectors

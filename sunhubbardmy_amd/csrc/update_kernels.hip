@@ -6,13 +6,13 @@
 // The sites are visited in blocks of UB = 64 consecutive sites.  The decisions of a block read
 // only the 64 x 64 diagonal block of G, so three kernels take turns per block:
 //   k_upd_sites   one workgroup per chain: the block's sequential decisions, with the block of G in
-//                 registers and brought up to date after every accepted site;
+//                 registers and brought up to date after every four sites;
 //   k_upd_panel   64-row strips of every chain: A = G(:, P) T and V = (G(P, :) - E_P) of the ka
 //                 accepted sites P;
 //   k_upd_flush   64 x 64 tiles of every chain: G += A V, rank ka, on FP64 MFMA.
 // With W = diag(1/delta_p) + 1 - G(P, P) and T = W^-1 the product of the accepted single-site
 // updates is G + G(:, P) T (G(P, :) - E_P).  T needs no factorization of its own: the sites kernel
-// runs Gauss-Jordan exchange steps (below) that leave it in the rows and columns of P.
+// runs Gauss-Jordan exchange steps (exchange.h) that leave it in the rows and columns of P.
 //
 // Why this split: keeping the delayed vectors of all N rows next to the decisions costs a pass over
 // N k entries per site in one workgroup (2 us per site at N = 256, k = 32) and a rank-k update of G
@@ -184,8 +184,8 @@ k_upd_panel(const DChain *chains, int s0)
 
 // G += A V over 64 x 64 tiles, the accumulators loaded with the tile of G while the first chunk of
 // A and V is on its way.  The tiles of a chain are dealt to one XCD (workgroups go round the eight
-// XCDs in launch order), whose L2 then holds the chain's A and V: nch8 = the chain count rounded
-// up to 8, nt = tiles per side of the largest chain.
+// XCDs in launch order, the chains are taken eight at a time), whose L2 then holds the chain's A and V.
+// nt = tiles per side of the largest chain.
 extern "C" __global__ void __launch_bounds__(256)
 k_upd_flush(const DChain *chains, int nch, int nt, int s0)
 {
